@@ -379,10 +379,10 @@ extern "C" int dm_batched_posv(int dtype, int num_items, void* A_base, void* B_b
 // launch over all systems still active at it (systems sorted largest first,
 // so those are a prefix of the system table):
 //   for each 64-column block jj:
-//     1. the 64 x 64 diagonal block of every system is factored by one wave
-//        (potrf_diag_block, the tile POTRF's diagonal step);
+//     1. the 64 x 64 diagonal block of every system is factored by one
+//        workgroup (pb_factor, the tile POTRF's diagonal step);
 //     2. its panel row U[jj, jj+64:n] := U_jj^-T A[jj, jj+64:n] over the
-//        system's full width, one wave per 64 columns (potrf_row_solve);
+//        system's full width, one workgroup per 64 columns (pb_solve);
 //     3. the rows left in the current outer tile of nb columns get the
 //        block's update (a batched SYRK-shaped GEMM with K = 64);
 //   after an outer tile's last block, the trailing matrix below it gets the
@@ -441,29 +441,59 @@ __global__ void zero_info_kernel(const TiledSys* __restrict__ d, int count,
   if (i < count) info[d[i].sys] = 0;
 }
 
-// Diagonal block (jj, jj) of every active system, one wave each; a system
-// whose info is set (an earlier pivot failed) is skipped, so info keeps the
-// first failure: jj + local column.  A full block with columns to its right
-// also gets W = U_jj^-T (64 x 64) in slot blockIdx.x of Wall, for the panel
-// row U[jj, jj+64:n] := W A[jj, jj+64:n] that follows as a batched GEMM.
+// Diagonal block (jj, jj) of every active system, one workgroup each; a
+// system whose info is set (an earlier pivot failed) is skipped, so info keeps
+// the first failure: jj + local column.
 template <typename T>
-__global__ __launch_bounds__(64) void bpotrf_diag_kernel(T* __restrict__ A,
-                                                         const TiledSys* __restrict__ d, int jj,
-                                                         int* __restrict__ info,
-                                                         T* __restrict__ Wall) {
-  __shared__ T rowb[2 * 64];
-  __shared__ T pv;
-  __shared__ T Us[64 * 64 + 64];
-  __shared__ T invd[64];
+__global__ __launch_bounds__(256) void bpotrf_diag_kernel(T* __restrict__ A,
+                                                          const TiledSys* __restrict__ d, int jj,
+                                                          int* __restrict__ info) {
+  __shared__ T M[PBE];
+  __shared__ int fail;
   const TiledSys s = d[blockIdx.x];
   if (info[s.sys]) return;
   T* As = A + s.a_off;
-  potrf_diag_block<T, true, 64>(As, s.n, s.ld, jj, info + s.sys, nullptr, 0, rowb, &pv);
-  if (s.n - jj <= 64) return;  // no panel row (uniform)
-  __syncthreads();             // the factored block is visible to the whole workgroup
-  if (info[s.sys]) return;     // uniform
-  potrf_row_stage<T, true, 64>(As, s.ld, jj, Us, invd);
-  potrf_row_inverse<T, 64>(Wall + (size_t)blockIdx.x * 64 * 64, 64, Us, invd);
+  const int kb = min(PB, s.n - jj);
+  T v[16];
+  pb_load_diag<T, true>(As, s.ld, jj, kb, v);
+  pb_put<T, true>(M, v);
+  __syncthreads();
+  const int bad = pb_factor<T>(M, kb, &fail);
+  pb_store_diag<T, true>(As, s.ld, jj, kb, bad ? bad - 1 : kb, M);
+  if (bad && threadIdx.x == 0) info[s.sys] = jj + bad;
+}
+
+// Panel row U[jj, jj+64:n] := U_jj^-T A[jj, jj+64:n] of every active system,
+// in place: one workgroup per 64 columns (begin[i]: the first workgroup of
+// system i), which reads its block, solves it in LDS and writes it back.
+template <typename T>
+__global__ __launch_bounds__(256) void bpotrf_row_kernel(T* __restrict__ A,
+                                                         const TiledSys* __restrict__ d,
+                                                         const int* __restrict__ begin, int count,
+                                                         int jj, const int* __restrict__ info) {
+  __shared__ T M[PBE];
+  __shared__ T X[PBE];
+  __shared__ T Wi[PIE];
+  int lo = 0, hi = count - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (begin[mid] <= (int)blockIdx.x) lo = mid; else hi = mid - 1;
+  }
+  const TiledSys s = d[lo];
+  if (info[s.sys]) return;
+  T* As = A + s.a_off;
+  const int c0 = jj + PB + PB * ((int)blockIdx.x - begin[lo]);
+  T v[16], x[16];
+  pb_load_diag<T, true>(As, s.ld, jj, PB, v);
+  pb_load<T, true>(As, s.ld, jj, c0, s.n - c0, x);
+  pb_put<T, true>(M, v);
+  pb_put<T, true>(X, x);
+  __syncthreads();
+  pb_inv16<T>(M, Wi);
+  __syncthreads();
+  pb_solve<T>(M, Wi, X, (threadIdx.x >> 6) * 16);
+  __syncthreads();
+  pb_store<T, true>(As, s.ld, jj, c0, s.n - c0, X);
 }
 
 // Z := U_k^-T Z (FWD) or U_k^-1 Z for the kb x kb diagonal tile at
@@ -561,7 +591,9 @@ struct BatchTiled : BatchTiledBase {
   };
   struct Step {            // 64-column block jj = 64 b
     int count = 0;         // systems with n > jj (a prefix of the system table)
-    Launch row;            // panel rows U[jj, jj+64:n] := W A[jj, jj+64:n], in place
+    int rows = 0, row_wgs = 0;          // systems with a panel row, its workgroups
+    std::vector<int> row_begin;         // first workgroup of each of them
+    const int* row_begin_dev = nullptr;
     Launch inner, trail;   // rows left in the outer tile; after its last block, A22
   };
   struct Tile {            // outer tile c0 = nb k of the sweeps
@@ -570,12 +602,11 @@ struct BatchTiled : BatchTiledBase {
   };
   T* A = nullptr;
   int nb = 256, nsys = 0, nrhs_sys = 0;
-  void* data = nullptr;    // working slab of right-hand sides, then the W slots
+  void* data = nullptr;    // working slab of right-hand sides
   void* tables = nullptr;  // system tables, copy jobs, GEMM jobs
   const TiledSys* sys_dev = nullptr;
   const TiledSys* rhs_dev = nullptr;
   T* Z = nullptr;
-  T* W = nullptr;          // one 64 x 64 block inverse per system
   std::vector<Step> steps;
   std::vector<Tile> tiles;
   Copies z_copy, x_copy;
@@ -614,10 +645,15 @@ struct BatchTiled : BatchTiledBase {
     for (size_t b = 0; b < steps.size(); ++b) {
       const Step& S = steps[b];
       const int jj = (int)b * 64, cnt = S.count;
-      T* w = W;
-      hipLaunchKernelGGL((bpotrf_diag_kernel<T>), dim3(cnt), dim3(64), 0, s, a, sd, jj, info, w);
+      hipLaunchKernelGGL((bpotrf_diag_kernel<T>), dim3(cnt), dim3(256), 0, s, a, sd, jj, info);
       DM_LAUNCH_CHECK("bpotrf_diag_kernel");
-      if ((rc = gemm(S.row, s))) return rc;
+      if (S.row_wgs) {
+        const int* rb = S.row_begin_dev;
+        const int nrow = S.rows;
+        hipLaunchKernelGGL((bpotrf_row_kernel<T>), dim3(S.row_wgs), dim3(256), 0, s, a, sd, rb,
+                           nrow, jj, info);
+        DM_LAUNCH_CHECK("bpotrf_row_kernel");
+      }
       if ((rc = gemm(S.inner, s))) return rc;
       if ((rc = gemm(S.trail, s))) return rc;
     }
@@ -673,9 +709,8 @@ struct BatchTiled : BatchTiledBase {
     }
     nrhs_sys = (int)rd.size();
     const size_t z_bytes = (sizeof(T) * (size_t)z_elems + 255) / 256 * 256;
-    DM_HIP(hipMalloc(&data, z_bytes + sizeof(T) * 64 * 64 * (size_t)nsys));
+    DM_HIP(hipMalloc(&data, std::max<size_t>(z_bytes, 256)));
     Z = (T*)data;
-    W = (T*)((char*)data + z_bytes);
     const int nblk = (td[0].n + 63) / 64;
     steps.assign(nblk, Step());
     auto a_at = [&](const TiledSys& t, int64_t r, int64_t c) {
@@ -693,16 +728,10 @@ struct BatchTiled : BatchTiledBase {
         const int tnb = t.tnb;
         const int64_t c0 = (int64_t)(jj / tnb) * tnb;  // the outer tile holding this block
         const bool last_in_tile = jj + 64 == c0 + tnb;
-        {  // in place: one workgroup holds all 64 rows of its columns and
-           // reads them (K = 64) before it stores (beta = 0: C is not read)
-          GemmJob<T> g{};
-          g.A = W + (size_t)i * 64 * 64; g.lda = 64;
-          g.B = a_at(t, jj, jj + 64); g.ldb = t.ld;
-          g.C = a_at(t, jj, jj + 64); g.ldc = t.ld;
-          g.M = 64; g.N = nrem; g.K = 64;
-          g.alpha = T(1); g.beta = T(0);
-          S.row.jobs.push_back(g);
-        }
+        // the panel row (systems are sorted by size, so these are a prefix)
+        S.row_begin.push_back(S.row_wgs);
+        S.row_wgs += (nrem + PB - 1) / PB;
+        S.rows = i + 1;
         const int c_end = (int)std::min<int64_t>(c0 + tnb, t.n);
         const int rows = c_end - jj - 64;
         if (rows > 0) {  // rows of this outer tile below the block, K = 64:
@@ -786,13 +815,9 @@ struct BatchTiled : BatchTiledBase {
     std::vector<Launch*> gl;
     for (Step& S : steps)
       for (Launch* L : {&S.inner, &S.trail}) gl.push_back(L);
-    std::vector<Launch*> rows;  // the in-place panel rows: 64-row tiles only
-    for (Step& S : steps) rows.push_back(&S.row);
     const size_t n_factor = gl.size();
     for (Tile& K : tiles)
       for (Launch* L : {&K.fwd, &K.bwd}) gl.push_back(L);
-    const size_t n_pick = gl.size();
-    for (Launch* L : rows) gl.push_back(L);
     size_t off = 0;
     auto take = [&](size_t bytes) {
       const size_t o = off;
@@ -803,6 +828,8 @@ struct BatchTiled : BatchTiledBase {
     const size_t o_rhs = take(sizeof(TiledSys) * std::max<size_t>(rd.size(), 1));
     const size_t o_zc = take(sizeof(BlockCopy) * z_copy.jobs.size());
     const size_t o_xc = take(sizeof(BlockCopy) * x_copy.jobs.size());
+    std::vector<size_t> o_row(steps.size(), 0);
+    for (size_t b = 0; b < steps.size(); ++b) o_row[b] = take(sizeof(int) * steps[b].row_begin.size());
     std::vector<size_t> o_gl(gl.size(), 0);
     for (size_t q = 0; q < gl.size(); ++q) {
       Launch& L = *gl[q];
@@ -817,8 +844,7 @@ struct BatchTiled : BatchTiledBase {
       // stay on 128 x 128 tiles: measured 30 ms against 45 ms on 256 x 128
       // tiles for the 4096-system mix (the picker takes the wider tile only
       // for vector-load launches)
-      L.cfg = q >= n_pick ? GemmCfgId{1, 64, 64}
-                          : gemm_pick_cfg<T>(mM, mN, mK, (int)L.jobs.size(), L.vec && q >= n_factor);
+      L.cfg = gemm_pick_cfg<T>(mM, mN, mK, (int)L.jobs.size(), L.vec && q >= n_factor);
       L.total = gemm_prepare_jobs<T>(L.jobs.data(), (int)L.jobs.size(), L.cfg);
       o_gl[q] = take(sizeof(GemmJob<T>) * L.jobs.size());
     }
@@ -836,6 +862,11 @@ struct BatchTiled : BatchTiledBase {
     rhs_dev = (const TiledSys*)(tb + o_rhs);
     z_copy.dev = (const BlockCopy*)(tb + o_zc);
     x_copy.dev = (const BlockCopy*)(tb + o_xc);
+    for (size_t b = 0; b < steps.size(); ++b) {
+      Step& S = steps[b];
+      put(o_row[b], S.row_begin.data(), sizeof(int) * S.row_begin.size());
+      S.row_begin_dev = (const int*)(tb + o_row[b]);
+    }
     for (size_t q = 0; q < gl.size(); ++q) {
       Launch& L = *gl[q];
       if (L.jobs.empty()) continue;

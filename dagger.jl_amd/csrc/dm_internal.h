@@ -242,11 +242,6 @@ int trsm_full(char side, char uplo, char transa, char diag, int m, int n,
 // ------------------------------------------------------------ POTRF
 // info: LAPACK info of this call (local order); abort (may be null): set to
 // global_offset + local order on failure and checked by every launch.
-// Trailing SYRK of the 64-wide POTRF panel at j0 fused with the
-// factorization of the next diagonal block (gemm.hip).
-template <typename T>
-int potrf_update_launch(bool upper, int n, T* A, int lda, int j0, int* info, int* abort,
-                        int global_base, hipStream_t s);
 // C = beta C + alpha A X on tiled FP64 operands where X and C are one block
 // column of at most 64 columns (mixed.hip): one launch, A read once.
 bool tiled_skinny_gemm_ok(char ta, char tb, const dm_tiled& A, const dm_tiled& X,

@@ -4,90 +4,181 @@
 // 2-18, spawned at :39/:84).  info follows LAPACK: 0, or k > 0 when the
 // leading minor of order k is not positive definite (pivot <= 0 or NaN).
 //
-// Structure: blocked right-looking factorization with 64-wide panels, two
-// launches per panel:
-//  1. potrf_row_kernel (one wave per 64 columns): the panel row
-//     U12 := U11^-T A12 (U) / A21 := A21 L11^-T (L), one column (row) per
-//     lane against the factored block held in LDS;
-//  2. the trailing update A22 -= U12^T U12 (A21 A21^T for L) on MFMA, fused
-//     with the factorization of the next 64 x 64 diagonal block
-//     (potrf_update_kernel, gemm.hip).
-// The first diagonal block is factored by potrf_diag_kernel (one wave, the
-// block in registers: lane c owns column c of U, or row c of L = column c
-// of L^T, broadcasting the current row through LDS -- no barriers).
+// Structure: blocked right-looking factorization with 64-wide panels, one
+// launch per panel (potrf_step_kernel) after the first diagonal block
+// (potrf_diag_kernel).  A launch takes the factored diagonal block U_kk, and
+// each of its workgroups owns one 64 x 64 tile (i, j) of the trailing
+// triangle: it solves the two panel-row blocks it needs, U_ki = U_kk^-T A_ki
+// and U_kj, in LDS for itself and updates its tile.  Solving them in every
+// workgroup costs 2 x 64^3 flops on a chip that is mostly idle and saves the
+// launch (and the trip through memory) that a separate panel-row step needs.
+// Workgroup 0 owns the next diagonal block, keeps it in LDS and factors it.
+// The panel row in memory stays unsolved meanwhile (other workgroups still
+// read it); the next launch's extra workgroups finish it, beside that
+// launch's tiles, which only touch later rows.  The last launch has a single
+// tile and finishes its own row.
+//
+// Bound by the chain of launches and pivots, not by flops.  Measured per 64
+// columns of a 512 tile (FP64): one launch of 20 us, 8 of them the diagonal
+// block; the panel row and the update as two launches, with the block factored
+// by one lane per column from LDS rows, took 23 + 40 us.
 // Every launch first checks the abort flag (and info), so after a failed
 // pivot the remaining launches are no-ops.
 #include <type_traits>
 #include "dm_internal.h"
+#include "gemm_tiles.h"
 #include "potrf_diag.h"
 
 namespace dm {
 
+// Factor the block in M (columns from kb on the identity's), store it at j0,
+// report a failed pivot.
+template <typename T, bool UPPER>
+__device__ __forceinline__ void potrf_block(T* M, int* fail, T* __restrict__ A, int lda, int j0,
+                                            int kb, int* __restrict__ info,
+                                            int* __restrict__ abort, int global_base) {
+  const int bad = pb_factor<T>(M, kb, fail);
+  pb_store_diag<T, UPPER>(A, lda, j0, kb, bad ? bad - 1 : kb, M);
+  if (bad && threadIdx.x == 0) {
+    if (info) *info = j0 + bad;
+    if (abort) *abort = global_base + j0 + bad;
+  }
+}
 
-// The diagonal block of panel j0 (see potrf_diag.h), one wave.
-template <typename T, bool UPPER, int PW>
-__global__ __launch_bounds__(64) void potrf_diag_kernel(T* __restrict__ A, int n, int lda, int j0,
-                                                        int* __restrict__ info,
-                                                        int* __restrict__ abort,
-                                                        int global_base) {
-  __shared__ T rowb[2 * 64];
-  __shared__ T pv;
+template <typename T, bool UPPER>
+__global__ __launch_bounds__(256) void potrf_diag_kernel(T* __restrict__ A, int n, int lda,
+                                                         int* __restrict__ info,
+                                                         int* __restrict__ abort,
+                                                         int global_base) {
+  __shared__ T M[PBE];
+  __shared__ int fail;
   if (abort && *abort) return;
   if (info && *info) return;
   raise_wave_priority();  // always on the critical path of a factorization
-  potrf_diag_block<T, UPPER, PW>(A, n, lda, j0, info, abort, global_base, rowb, &pv);
+  const int kb = min(PB, n);
+  T v[16];
+  pb_load_diag<T, UPPER>(A, lda, 0, kb, v);
+  pb_put<T, UPPER>(M, v);
+  __syncthreads();
+  potrf_block<T, UPPER>(M, &fail, A, lda, 0, kb, info, abort, global_base);
 }
 
-// Panel row beside a factored full PW x PW block: U12 := U11^-T A12 (U) or
-// A21 := A21 L11^-T (L).  One wave per 64 columns of A12 (rows of A21), one
-// column (row) per lane (potrf_row_stage / potrf_row_solve, potrf_diag.h).
-template <typename T, bool UPPER, int PW>
-__global__ __launch_bounds__(64) void potrf_row_kernel(T* __restrict__ A, int n, int lda, int j0,
-                                                       const int* __restrict__ info,
-                                                       const int* __restrict__ abort) {
-  __shared__ T Us[PW * PW + PW];
-  __shared__ T invd[PW];
+// The launch of panel j0 (see above): workgroups [0, ntile) own the tiles of
+// the trailing triangle, the others finish the row of panel j0 - 64.
+template <typename T, bool UPPER>
+__global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int n, int lda, int j0,
+                                                         int ntile, int* __restrict__ info,
+                                                         int* __restrict__ abort,
+                                                         int global_base) {
+  typedef typename PMfma<T>::v4 v4;
+  __shared__ T M[PBE];
+  __shared__ T Xi_[PBE];
+  __shared__ T Xj[PBE];
+  __shared__ T Wi[PIE];
+  __shared__ int fail;
   if (abort && *abort) return;
   if (info && *info) return;
   raise_wave_priority();
-  potrf_row_stage<T, UPPER, PW>(A, lda, j0, Us, invd);
-  potrf_row_solve<T, UPPER, PW>(A, n, lda, j0, blockIdx.x * 64, Us, invd);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int t = blockIdx.x;
+  const bool finish = t >= ntile;
+  const int jp = finish ? j0 - PB : j0;
+  int ti, tj;
+  if (finish) ti = tj = t - ntile;
+  else upper_tri_decode(t, ti, tj);
+  const int ci = jp + PB + PB * ti, cj = jp + PB + PB * tj;
+  const bool two = ti != tj;
+  // every load of the launch is issued before the first wait
+  T v[16], xi[16], xj[16];
+  pb_load_diag<T, UPPER>(A, lda, jp, PB, v);
+  pb_load<T, UPPER>(A, lda, jp, cj, n - cj, xj);
+  if (two) pb_load<T, UPPER>(A, lda, jp, ci, n - ci, xi);
+  // this wave's 32 x 32 quadrant of the tile: element (m, n) of block (p, q)
+  // in item r, the matrix's contiguous axis along the lanes
+  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
+  const bool work = !finish && (two || wm <= wn);
+  auto row_of = [&](int p, int r) { return wm + 16 * p + (UPPER ? lr : PMfma<T>::row(lk, r)); };
+  auto col_of = [&](int q, int r) { return wn + 16 * q + (UPPER ? PMfma<T>::row(lk, r) : lr); };
+  auto inside = [&](int m, int c) { return ci + m < n && cj + c < n && (two || m <= c); };
+  T old[2][2][4];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int m = row_of(p, r), c = col_of(q, r);
+        old[p][q][r] =
+            work && inside(m, c) ? *gptr(pb_at<T, UPPER>(A, lda, ci + m, cj + c)) : T(0);
+      }
+  pb_put<T, UPPER>(M, v);
+  __syncthreads();
+  pb_inv16<T>(M, Wi);
+  pb_put<T, UPPER>(Xj, xj);
+  if (two) pb_put<T, UPPER>(Xi_, xi);
+  __syncthreads();
+  pb_solve<T>(M, Wi, Xj, wave * 16);
+  if (two) pb_solve<T>(M, Wi, Xi_, wave * 16);
+  __syncthreads();
+  if (finish) {
+    pb_store<T, UPPER>(A, lda, jp, cj, n - cj, Xj);
+    return;
+  }
+  if (ntile == 1) pb_store<T, UPPER>(A, lda, j0, cj, n - cj, Xj);  // the only reader of this row
+  if (work) {
+    const T* Xi = two ? Xi_ : Xj;
+    // the 64 products are summed by themselves and subtracted once: rounding
+    // at the tile's own magnitude happens once, not at every k-step
+    v4 acc[2][2];
+    acc[0][0] = acc[0][1] = acc[1][0] = acc[1][1] = v4{0, 0, 0, 0};
+#pragma unroll 4
+    for (int s = 0; s < PB / 4; ++s) {
+      const int k = (4 * s + lk) * PBS;
+      T a[2], b[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) a[p] = Xi[k + wm + 16 * p + lr];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) b[q] = Xj[k + wn + 16 * q + lr];
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          acc[p][q] = UPPER ? PMfma<T>::mac(b[q], a[p], acc[p][q])
+                            : PMfma<T>::mac(a[p], b[q], acc[p][q]);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = row_of(p, r), c = col_of(q, r);
+          const T v = old[p][q][r] - acc[p][q][r];
+          if (t == 0) M[m * PBS + c] = inside(m, c) ? v : (m == c ? T(1) : T(0));
+          else if (inside(m, c)) *gptr(pb_at<T, UPPER>(A, lda, ci + m, cj + c)) = v;
+        }
+  }
+  if (t != 0) return;
+  __syncthreads();
+  potrf_block<T, UPPER>(M, &fail, A, lda, j0 + PB, min(PB, n - j0 - PB), info, abort, global_base);
 }
 
 namespace {
-template <typename T, int PW>
-int potrf_panels(bool upper, int n, T* A, int lda, int* info, int* abort, int global_offset,
-                 hipStream_t s) {
+template <typename T, bool UPPER>
+int potrf_panels(int n, T* A, int lda, int* info, int* abort, int global_offset, hipStream_t s) {
   // Launches after a failed pivot are no-ops: they watch the plan-level
   // abort flag when there is one, else info.
-  static_assert(PW == 64, "the fused update kernel factors 64-wide diagonal blocks");
-  bool diag_done = false;  // the previous panel's fused update factored this block
-  for (int j0 = 0; j0 < n; j0 += PW) {
-    if (!diag_done) {
-      if (upper)
-        hipLaunchKernelGGL((potrf_diag_kernel<T, true, PW>), dim3(1), dim3(64), 0, s, A, n, lda,
-                           j0, info, abort, global_offset);
-      else
-        hipLaunchKernelGGL((potrf_diag_kernel<T, false, PW>), dim3(1), dim3(64), 0, s, A, n, lda,
-                           j0, info, abort, global_offset);
-      DM_LAUNCH_CHECK("potrf_diag_kernel");
-    }
-    diag_done = false;
-    const int kb = n - j0 < PW ? n - j0 : PW;
-    const int rest = n - j0 - kb;
-    if (rest <= 0) break;  // a block narrower than PW is the last one
-    const unsigned nwg = (unsigned)((rest + 63) / 64);
-    if (upper)
-      hipLaunchKernelGGL((potrf_row_kernel<T, true, PW>), dim3(nwg), dim3(64), 0, s, A, n, lda, j0,
-                         info, abort);
-    else
-      hipLaunchKernelGGL((potrf_row_kernel<T, false, PW>), dim3(nwg), dim3(64), 0, s, A, n, lda,
-                         j0, info, abort);
-    DM_LAUNCH_CHECK("potrf_row_kernel");
-    // trailing update + next diagonal block in one launch
-    const int rc = potrf_update_launch<T>(upper, n, A, lda, j0, info, abort, global_offset, s);
-    if (rc) return rc;
-    diag_done = true;
+  if (n <= 0) return 0;
+  hipLaunchKernelGGL((potrf_diag_kernel<T, UPPER>), dim3(1), dim3(256), 0, s, A, n, lda, info, abort,
+                     global_offset);
+  DM_LAUNCH_CHECK("potrf_diag_kernel");
+  for (int j0 = 0; n - j0 > PB; j0 += PB) {
+    const int nt = (n - j0 - 1) / PB;  // 64-column blocks right of the panel
+    const int ntile = nt * (nt + 1) / 2;
+    const int nfin = j0 > 0 ? nt + 1 : 0;
+    hipLaunchKernelGGL((potrf_step_kernel<T, UPPER>), dim3((unsigned)(ntile + nfin)), dim3(256), 0, s,
+                       A, n, lda, j0, ntile, info, abort, global_offset);
+    DM_LAUNCH_CHECK("potrf_step_kernel");
   }
   return 0;
 }
@@ -97,7 +188,8 @@ template <typename T>
 int potrf_full(bool upper, int n, T* A, int lda, int* info, int* abort, int global_offset, T* ws,
                hipStream_t s) {
   (void)ws;
-  return potrf_panels<T, 64>(upper, n, A, lda, info, abort, global_offset, s);
+  return upper ? potrf_panels<T, true>(n, A, lda, info, abort, global_offset, s)
+               : potrf_panels<T, false>(n, A, lda, info, abort, global_offset, s);
 }
 
 template int potrf_full<double>(bool, int, double*, int, int*, int*, int, double*, hipStream_t);

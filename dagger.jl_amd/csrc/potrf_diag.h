@@ -1,237 +1,368 @@
-// The diagonal-block and panel-row steps of the tile POTRF (one wave each),
-// shared by potrf_diag_kernel / potrf_row_kernel (potrf.hip), the fused
-// trailing-update kernel that factors the next diagonal block (gemm.hip) and
-// the batched level-synchronous factorization (batched.hip).
+// The 64-wide panel of the tile POTRF as steps of a 256-thread workgroup on
+// LDS-resident blocks, shared by the tile kernels (potrf.hip) and the batched
+// level-synchronous factorization (batched.hip):
+//   pb_load / pb_store   a 64 x 64 block of the matrix <-> LDS
+//   pb_factor            Cholesky of a block in LDS
+//   pb_inv16             inverses of its four 16 x 16 diagonal blocks
+//   pb_solve             U^-T X for 16 columns of X per wave
+//
+// Blocks are kept as the matrix's upper view: element (r, c) is A[r, c] for
+// 'U' and A[c, r] for 'L' (so the factor is always U with U^T U = view).
+// An LDS block is row-major with an odd stride of 65 elements: reads along a
+// row and along a column of 8-byte elements both touch distinct banks.
 #pragma once
-#include <type_traits>
 #include "dm_internal.h"
 
 namespace dm {
 
-// Both panel kernels keep their code small enough for the instruction
-// cache: a single wave runs them, so every instruction fetched from L2
-// costs the whole kernel.  Instead of unrolling the 64 steps (a triangle
-// of static register indices, tens of KB of code), each lane keeps a
-// window of its column that slides by one row per step (the update of
-// row i+1 lands in register i, so the row being eliminated is always in
-// register 0), and the step loop stays rolled.  The window shrinks in
-// phases of 16 steps, so the update length follows the triangle in
-// steps of 16 rows.
+constexpr int PB = 64;        // panel width
+constexpr int PBS = PB + 1;   // LDS row stride of a block
+constexpr int PBE = PB * PBS; // LDS elements of a block
+constexpr int PIS = 17;       // LDS row stride of an inverted 16 x 16 block
+constexpr int PIE = 4 * 16 * PIS + 64;  // LDS elements of pb_inv16's result
 
-// sd = sqrt(d) and inv = 1/sqrt(d) for a pivot d > 0.  In the normal range
-// the reciprocal square root comes from the hardware estimate refined by
-// Newton steps (y += y/2 (1 - d y^2)), and sd = d y is corrected once by
-// the residual d - sd^2: about a quarter of the dependent latency of a
-// correctly rounded sqrt followed by a division, which sits on the serial
-// chain of every column step.  Both results are within an ulp or two.
-__device__ __forceinline__ void sqrt_inv(double d, double& sd, double& inv) {
-  if (d > 1e-290 && d < 1e290) {
-    double y = __builtin_amdgcn_rsq(d);
-    double e = __builtin_fma(-d * y, y, 1.0);
-    y = __builtin_fma(0.5 * y, e, y);
-    e = __builtin_fma(-d * y, y, 1.0);
-    y = __builtin_fma(0.5 * y, e, y);
-    double s = d * y;
-    const double r = __builtin_fma(-s, s, d);
-    sd = __builtin_fma(0.5 * y, r, s);
-    inv = y;
-  } else {  // tiny, huge, zero, negative or NaN: the exact forms
-    sd = sqrt(d);
-    inv = 1.0 / sd;
+template <typename T> struct PMfma;
+// Output layouts (lane l, accumulator item r; 16x16 block D[i][j], j = l%16):
+//   f64 16x16x4: i = 4*r + l/16        f32 16x16x4: i = 4*(l/16) + r
+template <> struct PMfma<double> {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ int row(int lk, int r) { return 4 * r + lk; }
+  static __device__ __forceinline__ v4 mac(double a, double b, v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
-}
-__device__ __forceinline__ void sqrt_inv(float d, float& sd, float& inv) {
-  if (d > 1e-30f && d < 1e30f) {
-    float y = __builtin_amdgcn_rsqf(d);
-    const float e = __builtin_fmaf(-d * y, y, 1.0f);
-    y = __builtin_fmaf(0.5f * y, e, y);
-    const float s = d * y;
-    const float r = __builtin_fmaf(-s, s, d);
-    sd = __builtin_fmaf(0.5f * y, r, s);
-    inv = y;
-  } else {
-    sd = sqrtf(d);
-    inv = 1.0f / sd;
-  }
-}
-
-// Factor the kb x kb diagonal block at (j0, j0), kb = min(PW, n - j0), in one
-// wave.  Element (r, c), r <= c, of the block's upper view is A[j0+r, j0+c]
-// (U) or A[j0+c, j0+r] (L, i.e. L^T); lane c holds rows j.. of column c of
-// that view at step j.  On a failed pivot at local column j: info =
-// j0 + j + 1 and *abort = global_base + j0 + j + 1.
-template <typename T, bool UPPER, int PW>
-struct PotrfDiag {
-  T c[PW];     // c[i] = element (j + i, t) of the upper view at step j
-  T d, sd, inv;  // pivot of the current step, its square root and reciprocal
-  T* rowb;     // LDS: row j of the factor (PW entries) then PW zeros
-  T* pv;       // LDS: next pivot
-  T* A;
-  int lda, j0, kb, t;
-
-  __device__ __forceinline__ void put(int r, T v) {
-    if (UPPER) A[(size_t)(j0 + t) * lda + j0 + r] = v;
-    else A[(size_t)(j0 + r) * lda + j0 + t] = v;
-  }
-
-  // Steps j0s .. j0s+15 (those below kb) with a window of L live rows.
-  // Returns the failed local column + 1, or 0.
-  template <int L>
-  __device__ __forceinline__ int phase(int js) {
-    const int je = min(js + 16, kb);
-#pragma unroll 1
-    for (int j = js; j < je; ++j) {
-      if (!(d > T(0))) return j + 1;
-      T u = T(0), fin = c[0];
-      if (t == j) fin = sd;
-      else if (t > j) {
-        u = c[0] * inv;
-        fin = u;
-      }
-      if (t >= j && t < kb) put(j, fin);
-      if (t == j + 1) *pv = c[1] - u * u;
-      rowb[t] = u;  // zero for lanes <= j: their columns are left unchanged
-      __builtin_amdgcn_wave_barrier();
-      d = *pv;
-      sqrt_inv(d, sd, inv);
-      const T* rb = rowb + j + 1;  // reads past PW land in the zero half
-#pragma unroll
-      for (int i = 0; i < L - 1; ++i) c[i] = c[i + 1] - rb[i] * u;
-      c[L - 1] = T(0);
-      __builtin_amdgcn_wave_barrier();  // rowb/pv are rewritten by the next step
-    }
-    return 0;
+};
+template <> struct PMfma<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
+  static __device__ __forceinline__ v4 mac(float a, float b, v4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
 };
 
-// Factor the kb x kb block at (j0, j0) of A, kb = min(PW, n - j0), with the
-// first wave of the calling workgroup (threadIdx.x < 64 run it; others
-// return at once).  rowb: 128 LDS elements, pv: one.  On a failed pivot at
-// local column j: info = j0 + j + 1 and *abort = global_base + j0 + j + 1.
-template <typename T, bool UPPER, int PW>
-__device__ __forceinline__ void potrf_diag_block(T* __restrict__ A, int n, int lda, int j0,
-                                                 int* __restrict__ info, int* __restrict__ abort,
-                                                 int global_base, T* rowb, T* pv_) {
-  static_assert(PW == 32 || PW == 64, "panel width");
-  if (threadIdx.x >= 64) return;
-  PotrfDiag<T, UPPER, PW> f;
-  f.t = threadIdx.x;
-  f.kb = min(PW, n - j0);
-  f.A = A;
-  f.lda = lda;
-  f.j0 = j0;
-  f.rowb = rowb;
-  f.pv = pv_;
-  const int t = f.t;
+// Lane l's value in every lane (l uniform): a scalar register, no LDS trip.
+__device__ __forceinline__ float lane_bcast(float v, int l) {
+  int i;
+  __builtin_memcpy(&i, &v, 4);
+  i = __builtin_amdgcn_readlane(i, l);
+  __builtin_memcpy(&v, &i, 4);
+  return v;
+}
+__device__ __forceinline__ double lane_bcast(double v, int l) {
+  int i[2];
+  __builtin_memcpy(i, &v, 8);
+  i[0] = __builtin_amdgcn_readlane(i[0], l);
+  i[1] = __builtin_amdgcn_readlane(i[1], l);
+  __builtin_memcpy(&v, i, 8);
+  return v;
+}
+
+// 1/sqrt(d) for a pivot d in the normal range (PivotBits): the hardware
+// estimate y (relative error at most 2^-22) gets one third-order step,
+// y + y e (1/2 + 3/8 e) with e = 1 - d y^2, whose error of order e^3 is below
+// the rounding (FP32: one Newton step).  Straight-line and four dependent
+// operations long, against a correctly rounded sqrt and a division of several
+// tens each: it sits on the serial chain of every column.
+__device__ __forceinline__ double inv_sqrt(double d) {
+  const double y = __builtin_amdgcn_rsq(d);
+  const double e = __builtin_fma(-d * y, y, 1.0);
+  return __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+}
+__device__ __forceinline__ float inv_sqrt(float d) {
+  const float y = __builtin_amdgcn_rsqf(d);
+  const float e = __builtin_fmaf(-d * y, y, 1.0f);
+  return __builtin_fmaf(0.5f * y, e, y);
+}
+// sqrt(d): d / sqrt(d) corrected once by its residual.
+template <typename T>
+__device__ __forceinline__ T sqrt_of(T d) {
+  const T y = inv_sqrt(d), s = d * y;
+  return s + T(0.5) * y * (d - s * s);
+}
+// The normal range of a pivot by its exponent bits as an unsigned number
+// counted from lo: at most span exactly for 2^-960 <= d < 2^960 (FP32: 2^-96
+// and 2^96); zero, negative, infinite and NaN pivots lie outside too.
+template <typename T> struct PivotBits;
+template <> struct PivotBits<double> {
+  static constexpr unsigned lo = (1023u - 960u) << 20, span = (1920u << 20) - 1;
+  static __device__ __forceinline__ unsigned of(double d) {
+    unsigned long long b;
+    __builtin_memcpy(&b, &d, 8);
+    return (unsigned)(b >> 32) - lo;
+  }
+};
+template <> struct PivotBits<float> {
+  static constexpr unsigned lo = (127u - 96u) << 23, span = (192u << 23) - 1;
+  static __device__ __forceinline__ unsigned of(float d) {
+    unsigned b;
+    __builtin_memcpy(&b, &d, 4);
+    return b - lo;
+  }
+};
+
+// This thread's wave, as a scalar the compiler knows to be uniform (branches
+// on it are scalar branches instead of execution masks).
+__device__ __forceinline__ int wave_id() {
+  return __builtin_amdgcn_readlane((int)threadIdx.x >> 6, 0);
+}
+
+// Address of element (r, c) of the upper view.
+template <typename T, bool UPPER>
+__device__ __forceinline__ T* pb_at(T* A, int lda, int r, int c) {
+  return UPPER ? A + (size_t)c * lda + r : A + (size_t)r * lda + c;
+}
+
+// This thread's 16 elements of a 64 x 64 block: element q is (r, c) with the
+// contiguous axis of the matrix along the lanes.
+template <bool UPPER>
+__device__ __forceinline__ void pb_coord(int q, int& r, int& c) {
+  const int a = threadIdx.x & 63, b = (threadIdx.x >> 6) + 4 * q;
+  r = UPPER ? a : b;
+  c = UPPER ? b : a;
+}
+
+// v = rows r0.. and columns c0.. of the view, zero from column ncol on
+// (16 loads in flight per thread).
+template <typename T, bool UPPER>
+__device__ __forceinline__ void pb_load(const T* A, int lda, int r0, int c0, int ncol, T (&v)[16]) {
 #pragma unroll
-  for (int r = 0; r < PW; ++r) {
-    const bool in = t < f.kb && r <= t;
-    f.c[r] = in ? (UPPER ? A[(size_t)(j0 + t) * lda + j0 + r] : A[(size_t)(j0 + r) * lda + j0 + t])
-                : T(0);
+  for (int q = 0; q < 16; ++q) {
+    int r, c;
+    pb_coord<UPPER>(q, r, c);
+    v[q] = c < ncol ? *gptr(pb_at<T, UPPER>(const_cast<T*>(A), lda, r0 + r, c0 + c)) : T(0);
   }
-  rowb[64 + t] = T(0);
-  if (t == 0) *pv_ = f.c[0];
-  __builtin_amdgcn_wave_barrier();
-  f.d = *pv_;
-  sqrt_inv(f.d, f.sd, f.inv);
-  __builtin_amdgcn_wave_barrier();  // every lane has read pv before step 0 rewrites it
-  int fail = f.template phase<PW>(0);
-  if (!fail && PW > 16) fail = f.template phase<PW - 16>(16);
-  if (PW == 64) {
-    if (!fail) fail = f.template phase<(PW > 32 ? PW - 32 : 16)>(32);
-    if (!fail) fail = f.template phase<(PW > 48 ? PW - 48 : 16)>(48);
+}
+// The upper triangle of the kb x kb diagonal block at j0; the rest of the
+// 64 x 64 block is the identity's (so a narrow block factors like a full one).
+template <typename T, bool UPPER>
+__device__ __forceinline__ void pb_load_diag(const T* A, int lda, int j0, int kb, T (&v)[16]) {
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    int r, c;
+    pb_coord<UPPER>(q, r, c);
+    v[q] = (r <= c && c < kb) ? *gptr(pb_at<T, UPPER>(const_cast<T*>(A), lda, j0 + r, j0 + c))
+                              : (r == c ? T(1) : T(0));
   }
-  if (t == 0 && fail) {
-    if (info) *info = j0 + fail;
-    if (abort) *abort = global_base + j0 + fail;
+}
+template <typename T, bool UPPER>
+__device__ __forceinline__ void pb_put(T* M, const T (&v)[16]) {
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    int r, c;
+    pb_coord<UPPER>(q, r, c);
+    M[r * PBS + c] = v[q];
+  }
+}
+template <typename T, bool UPPER>
+__device__ __forceinline__ void pb_store(T* A, int lda, int r0, int c0, int ncol, const T* M) {
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    int r, c;
+    pb_coord<UPPER>(q, r, c);
+    if (c < ncol) *gptr(pb_at<T, UPPER>(A, lda, r0 + r, c0 + c)) = M[r * PBS + c];
+  }
+}
+// Upper triangle of the first nrow rows of a factored kb x kb block.
+template <typename T, bool UPPER>
+__device__ __forceinline__ void pb_store_diag(T* A, int lda, int j0, int kb, int nrow, const T* M) {
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    int r, c;
+    pb_coord<UPPER>(q, r, c);
+    if (r <= c && c < kb && r < nrow)
+      *gptr(pb_at<T, UPPER>(A, lda, j0 + r, j0 + c)) = M[r * PBS + c];
   }
 }
 
-// Panel row beside a factored full PW x PW block at (j0, j0): U12 :=
-// U11^-T A12 (U) or A21 := A21 L11^-T (L), one column of A12 (row of A21)
-// per lane.  potrf_row_stage (every thread of a one-wave workgroup) puts
-// the block in LDS as its upper view with row stride PW -- so reading row p
-// past column PW-1 lands in the (zero) strictly lower part of row p+1,
-// followed by PW zeros -- and the reciprocals of its diagonal in invd.
-// Us: PW * PW + PW elements, invd: PW.
-template <typename T, bool UPPER, int PW>
-__device__ __forceinline__ void potrf_row_stage(const T* __restrict__ A, int lda, int j0,
-                                                T* Us, T* invd) {
-  static_assert(PW == 32 || PW == 64, "panel width");
-  const int t = threadIdx.x;
-  if (t < PW) {
-    // lane = column c; U: element (r, c) = A[j0+r, j0+c]; L: A[j0+c, j0+r]
-    for (int r = 0; r < PW; ++r) {
-      T v = T(0);
-      if (r <= t) v = UPPER ? A[(size_t)(j0 + t) * lda + j0 + r] : A[(size_t)(j0 + r) * lda + j0 + t];
-      Us[r * PW + t] = v;
-    }
-    Us[PW * PW + t] = T(0);
+// Cholesky of the 64 x 64 block in M (upper triangle; columns from kb on are
+// the identity's), in place.  Returns 0, or the failed column + 1 (its row
+// and the later ones are then not final).  fail: one LDS int.
+//
+// Bound by the serial chain of 64 pivots.  Eight rows at a time (pb_chain):
+// wave 0 holds them with one column per lane, so a step is a readlane of the
+// pivot, the reciprocal square root, a scaling and at most seven rank-1
+// updates whose multipliers are readlanes too -- no LDS trip and no branch
+// inside the chain (pivots outside the normal range are noticed at the end of
+// the eight rows, which are then done again in the exact form).  The rows
+// below get the eight rows' update on the matrix cores: wave w keeps the
+// blocks of the 16 columns from 16 w on in its accumulators all the way down
+// (acc[q]: block row blk + q) and hands the next eight rows to wave 0 through
+// M; the blocks below those are updated while wave 0 is already at its next
+// eight rows.
+// Measured per block (cycles): the chain 1280 of 2500 per eight rows, the
+// hand-over the rest; one column per lane and all 64 steps from LDS rows, as
+// this step was done before, took 75000 for the block, this 19000.
+template <typename T>
+__device__ __forceinline__ int pb_chain(T* M, int base, T& diag) {
+  const int lane = threadIdx.x & 63;
+  T v[8];
+  T* rows = M + base * PBS + lane;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) v[r] = rows[r * PBS];
+  unsigned far = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const T d = lane_bcast(v[j], base + j);
+    const unsigned e = PivotBits<T>::of(d);
+    far = e > far ? e : far;
+    if (lane == base + j) diag = d;
+    const T u = v[j] = v[j] * inv_sqrt(d);
+#pragma unroll
+    for (int i = j + 1; i < 8; ++i) v[i] -= lane_bcast(u, base + i) * u;
   }
-  __syncthreads();
-  if (t < PW) invd[t] = T(1) / Us[t * PW + t];
-  __syncthreads();
-}
-
-// U11^T x = b for one column per lane, forward over the rows of the staged
-// block; x[i] holds row p + i at step p, and row p's result goes to
-// base[p * step].
-template <typename T, int PW>
-__device__ __forceinline__ void potrf_row_phases(T (&x)[PW], T* base, size_t step, const T* Us,
-                                                 const T* invd) {
-  auto phase = [&](auto len, int ps) {
-    constexpr int L = decltype(len)::value;
+  if (__builtin_expect(far <= PivotBits<T>::span, 1)) {  // uniform
+#pragma unroll
+    for (int r = 0; r < 8; ++r) rows[r * PBS] = v[r];
+    return 0;
+  }
 #pragma unroll 1
-    for (int p = ps; p < ps + 16; ++p) {
-      const T xp = x[0] * invd[p];
-      base[p * step] = xp;
-      const T* u = Us + p * PW + p + 1;
+  for (int j = 0; j < 8; ++j) {
+    const T w = rows[j * PBS], d = lane_bcast(w, base + j);
+    if (!(d > T(0))) return base + j + 1;
+    // tiny, huge or infinite: the exact forms
+    const T sd = sqrt(d), u = w * (T(1) / sd);
+    rows[j * PBS] = lane == base + j ? sd : u;
+    if (lane == base + j) diag = T(0);  // already final
+#pragma unroll 1
+    for (int i = j + 1; i < 8; ++i) rows[i * PBS] -= lane_bcast(u, base + i) * u;
+  }
+  return 0;
+}
+
+template <typename T>
+__device__ __forceinline__ int pb_factor(T* M, int kb, int* fail) {
+  typedef typename PMfma<T>::v4 v4;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int lr = lane & 15, lk = lane >> 4;
+  v4 acc[4];
 #pragma unroll
-      for (int i = 0; i < L - 1; ++i) x[i] = x[i + 1] - u[i] * xp;
-      x[L - 1] = T(0);
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      acc[q][r] = M[(16 * q + PMfma<T>::row(lk, r)) * PBS + 16 * wave + lr];
+  T diag = T(0);  // lane c: pivot c
+  int bad = 0;
+#pragma unroll 1
+  for (int blk = 0; 16 * blk < kb; ++blk) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int base = 16 * blk + 8 * half;
+      if (wave == 0) {
+        const int f = pb_chain<T>(M, base, diag);
+        if (lane == 0) *fail = f;
+      }
+      __syncthreads();
+      const int q0 = half;  // block row of the next eight rows
+      const T* row = M + (base + lk) * PBS + lr;
+      auto update = [&](int q) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          acc[q] = PMfma<T>::mac(-row[4 * s * PBS + 16 * (blk + q)], row[4 * s * PBS + 16 * wave],
+                                 acc[q]);
+      };
+      if (wave >= blk + q0) {
+        update(q0);
+        T* out = M + (base + 8) * PBS + 16 * wave + lr;
+        // half 0: rows 8 .. 15 of the block, half 1: rows 0 .. 7 of the next
+        if (sizeof(T) == 8) {
+          out[lk * PBS] = acc[q0][half ? 0 : 2];
+          out[(4 + lk) * PBS] = acc[q0][half ? 1 : 3];
+        } else if ((lk >> 1) == 1 - half) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) out[(4 * (lk & 1) + r) * PBS] = acc[q0][r];
+        }
+      }
+      bad = *fail;
+      __syncthreads();
+      if (bad || base + 8 >= kb) break;
+#pragma unroll
+      for (int q = q0 + 1; q < 4; ++q)
+        if (wave >= blk + q) update(q);
     }
-  };
-  phase(std::integral_constant<int, PW>{}, 0);
-  phase(std::integral_constant<int, PW - 16>{}, 16);
-  if constexpr (PW == 64) {
-    phase(std::integral_constant<int, 32>{}, 32);
-    phase(std::integral_constant<int, 16>{}, 48);
+    if (bad) break;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) acc[q] = acc[q + 1];
   }
+  if (wave == 0 && diag > T(0)) M[lane * PBS + lane] = sqrt_of(diag);
+  __syncthreads();
+  return bad;
 }
 
-// Columns c0 + lane of A12 (rows of A21), counted from j0 + PW, after
-// potrf_row_stage.  Lanes past the panel return (no barrier follows).
-template <typename T, bool UPPER, int PW>
-__device__ __forceinline__ void potrf_row_solve(T* __restrict__ A, int n, int lda, int j0, int c0,
-                                                const T* Us, const T* invd) {
-  const int t = threadIdx.x;
-  const int c_begin = j0 + PW, rest = n - c_begin;
-  if (c0 + t >= rest) return;
-  const int cc = c_begin + c0 + t;
-  const size_t step = UPPER ? 1 : (size_t)lda;
-  T* const base = UPPER ? A + (size_t)cc * lda + j0 : A + (size_t)j0 * lda + cc;
-  T x[PW];
-  const T* px = base;
+// W_g = (U_gg)^-T (lower triangular, 16 x 16) of the four diagonal blocks of
+// the factored block in M: W_g(r, c) at Wi[g * 16 * PIS + r * PIS + c].  Wave
+// g inverts block g: its two 8 x 8 diagonal blocks by substitution (one
+// column per lane), then W21 = -V1 (L21 V0).  The caller's barrier follows.
+template <typename T>
+__device__ __forceinline__ void pb_inv16(const T* M, T* Wi) {
+  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const T* Mg = M + (g * 16) * PBS + g * 16;  // U_gg(p, r) = Mg[p * PBS + r] = L(r, p)
+  T* W = Wi + g * 16 * PIS;
+  T* dinv = Wi + 4 * 16 * PIS + g * 16;
+  if (lane < 16) dinv[lane] = T(1) / Mg[lane * PBS + lane];
+  for (int e = lane; e < 256; e += 64) W[(e >> 4) * PIS + (e & 15)] = T(0);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const int o = (lane >> 3) * 8, c = lane & 7;
+  if (lane < 16) {
+    T x[8];
 #pragma unroll
-  for (int r = 0; r < PW; ++r) {
-    x[r] = *px;
-    px += step;
-    if ((r & 15) == 15) __builtin_amdgcn_sched_barrier(0);  // bound the loads in flight
+    for (int r = 0; r < 8; ++r) x[r] = r == c ? T(1) : T(0);
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      x[r] *= dinv[o + r];
+#pragma unroll
+      for (int i = r + 1; i < 8; ++i) x[i] -= Mg[(o + r) * PBS + o + i] * x[r];
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r) W[(o + r) * PIS + o + c] = x[r];
   }
-  potrf_row_phases<T, PW>(x, base, step, Us, invd);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  // Z = L21 V0 in W's (otherwise zero) upper right block
+  const int r8 = lane >> 3;
+  T z = T(0);
+#pragma unroll
+  for (int p = 0; p < 8; ++p) z += Mg[p * PBS + 8 + r8] * W[p * PIS + c];
+  W[r8 * PIS + 8 + c] = z;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  T y = T(0);
+#pragma unroll
+  for (int p = 0; p < 8; ++p) y -= W[(8 + r8) * PIS + 8 + p] * W[p * PIS + 8 + c];
+  __builtin_amdgcn_wave_barrier();  // every lane has read the block
+  W[(8 + r8) * PIS + c] = y;
+  W[r8 * PIS + 8 + c] = T(0);
 }
 
-// W = U11^-T (PW x PW, column-major, leading dimension ldw) of the block
-// staged by potrf_row_stage (upper view): lane c solves U11^T w = e_c.
-template <typename T, int PW>
-__device__ __forceinline__ void potrf_row_inverse(T* __restrict__ W, int ldw, const T* Us,
-                                                  const T* invd) {
-  const int t = threadIdx.x;
-  if (t >= PW) return;
-  T x[PW];
+// Columns c0 .. c0+15 of X := U^-T X for the factored block M (with pb_inv16's
+// Wi), by one wave on matrix cores: block row b needs sum_{i<b} U_ib^T X_i and
+// then a product with W_b.  An accumulator of the matrix core holds rows
+// row(lk, r) of a column in item r, and the next product's operand of k-step
+// s is rows row(lk, s): the same lane and item, so the chain of 40 products
+// stays in registers.
+template <typename T>
+__device__ __forceinline__ void pb_solve(const T* M, const T* Wi, T* X, int c0) {
+  typedef typename PMfma<T>::v4 v4;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  v4 x[4];
 #pragma unroll
-  for (int r = 0; r < PW; ++r) x[r] = (r == t) ? T(1) : T(0);
-  potrf_row_phases<T, PW>(x, W + (size_t)t * ldw, 1, Us, invd);
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) x[b][r] = X[(16 * b + PMfma<T>::row(lk, r)) * PBS + c0 + lr];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+#pragma unroll
+    for (int i = 0; i < b; ++i)
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        x[b] = PMfma<T>::mac(-M[(16 * i + PMfma<T>::row(lk, s)) * PBS + 16 * b + lr], x[i][s], x[b]);
+    v4 y = v4{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      y = PMfma<T>::mac(Wi[b * 16 * PIS + lr * PIS + PMfma<T>::row(lk, s)], x[b][s], y);
+    x[b] = y;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) X[(16 * b + PMfma<T>::row(lk, r)) * PBS + c0 + lr] = y[r];
+  }
 }
 
 }  // namespace dm

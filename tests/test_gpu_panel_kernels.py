@@ -1,0 +1,90 @@
+"""The panel kernels of the factorizations at the sizes and values where they
+branch: block edges, ragged last blocks, pivots outside the range of the fast
+reciprocal square root, failed pivots.  References are numpy in FP64."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+class Dev:
+    """A host array's device copy (column-major)."""
+
+    def __init__(self, dm, a):
+        self.dm = dm
+        self.a = np.asfortranarray(a)
+        self.buf = dm.DeviceBuffer(max(self.a.nbytes, 8))
+        if self.a.nbytes:
+            dm._lib.call("dm_memcpy_h2d", C.c_void_p(self.buf.ptr),
+                         self.a.ctypes.data_as(C.c_void_p), C.c_size_t(self.a.nbytes), None)
+
+    @property
+    def p(self):
+        return C.c_void_p(self.buf.ptr)
+
+    def get(self):
+        out = np.empty_like(self.a, order="F")
+        if out.nbytes:
+            self.dm._lib.call("dm_memcpy_d2h", out.ctypes.data_as(C.c_void_p), self.p,
+                              C.c_size_t(out.nbytes), None)
+        return out
+
+
+def _spd(n, dtype, seed):
+    rng = np.random.default_rng(seed)
+    G = rng.standard_normal((n, n))
+    return (G @ G.T / n + np.eye(n)).astype(dtype).astype(np.float64)
+
+
+def _potrf(dm, A, uplo, dtype):
+    n = A.shape[0]
+    d, info = Dev(dm, A.astype(dtype)), dm.DeviceInt(1)
+    fn = "dm_dpotrf" if dtype == np.float64 else "dm_spotrf"
+    dm._lib.call(fn, uplo.encode(), n, d.p, max(n, 1), C.c_void_p(info.ptr), None)
+    return d.get(), int(info.get()[0])
+
+
+# factor error of a well-conditioned matrix: a few n eps, n <= 200
+TOL = {np.float64: 2e-13, np.float32: 1e-4}
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 56, 57, 63, 64, 65, 127, 128, 129, 200])
+@pytest.mark.parametrize("scaling", ["none", "tiny", "huge", "mixed"])
+def test_potrf_panel(dm, dtype, uplo, n, scaling):
+    """D A D has the factor U D for a diagonal D of powers of two: with huge or
+    tiny D the pivots leave the fast range, with a mixed one only some do.  The
+    other triangle stays as it was."""
+    A = _spd(n, dtype, n)
+    e = {"none": 0, "tiny": -1, "huge": 1, "mixed": 1}[scaling] * (485 if dtype == np.float64 else 49)
+    k = np.full(n, e)
+    if scaling == "mixed":
+        k = np.where(np.arange(n) % 11 == 3, e, np.where(np.arange(n) % 13 == 5, -e, 0))
+    D = np.ldexp(1.0, k)
+    got, info = _potrf(dm, A * D[:, None] * D[None, :], uplo, dtype)
+    assert info == 0
+    U = np.linalg.cholesky(A).T
+    # undo the scaling (exact): U D -> U
+    F = got.astype(np.float64)
+    F = np.triu(F) / D[None, :] if uplo == "U" else (np.tril(F) / D[:, None]).T
+    assert np.abs(F - U).max() <= TOL[dtype] * np.abs(U).max()
+    other = np.tril(got, -1) if uplo == "U" else np.triu(got, 1)
+    want = (A * D[:, None] * D[None, :]).astype(dtype)
+    assert np.array_equal(other, np.tril(want, -1) if uplo == "U" else np.triu(want, 1))
+
+
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n,bad", [(1, 0), (64, 0), (64, 63), (70, 66), (150, 64), (150, 100),
+                                   (200, 199)])
+@pytest.mark.parametrize("value", [0.0, -3.0, np.nan])
+def test_potrf_failed_pivot(dm, uplo, n, bad, value):
+    """info is the 1-based order of the first pivot that is not positive, and
+    the rows of the factor before it are final."""
+    A = np.diag(np.arange(1.0, n + 1))
+    A[bad, bad] = value
+    got, info = _potrf(dm, A, uplo, np.float64)
+    assert info == bad + 1
+    assert np.allclose(np.diag(got)[:bad], np.sqrt(np.arange(1.0, bad + 1)), rtol=1e-15, atol=0)
