@@ -28,13 +28,6 @@ struct Region {
   std::vector<int> readers;  // readers since last_writer
 };
 
-struct InvSrc {
-  const void* A;
-  int lda, L;
-  size_t off;
-  void* dev = nullptr;
-};
-
 struct Group {
   int level = 0, crit = 1, op = 0, dtype = DM_F64, stream = 0;
   std::vector<int> tasks;
@@ -42,14 +35,12 @@ struct Group {
   // batched GEMM/SYRK
   bool ta = false, tb = false, vec = false;
   GemmCfgId cfg{0, 128, 128};
-  // batched TRSM: inverse blocks per distinct triangle, then the recursive
-  // solve's launches (leaf solves and GEMM updates) in order
+  // TRSM and TRSV: the recursive solve's launches (leaf solves and GEMM
+  // updates) in order
   TrsmShape shape{};
-  bool batched_trsm = false;
-  std::vector<InvSrc> inv_src;
   struct Step {
     bool leaf = true;
-    int njobs = 0, maxL = 0;
+    int njobs = 0, nb = 1;  // leaf solves: 16-vector blocks per workgroup
     long total_wg = 0;
     bool ta = false, tb = false, vec = false;  // GEMM updates
     GemmCfgId cfg{0, 128, 128};
@@ -89,7 +80,6 @@ struct Dag {
   // device state owned by the plan
   void* dev_mem = nullptr;
   int* abort_dev = nullptr;  // 0, or the global order of the first failed pivot
-  size_t inv_bytes = 0;
   std::vector<size_t> task_ws_off;  // byte offset in dev_mem, or SIZE_MAX
   std::vector<hipStream_t> streams;
   hipStream_t origin = nullptr;

@@ -51,6 +51,29 @@ void mat_span(const void* p, long rows, long cols, long ld, size_t es, uintptr_t
   hi = lo + (size_t)((cols - 1) * ld + rows) * es;
 }
 
+bool is_solve(int op) { return op == DM_OP_TRSM || op == DM_OP_TRSV; }
+
+// A solve task as a trsm call.  TRSV (x := op(A)^-1 x): a contiguous x is the
+// n x 1 right-hand side; x with stride incx is the single row of a 1 x n
+// matrix with ld = incx, solved from the right by the opposite transpose.
+struct SolveTask {
+  char side, uplo, trans, diag;
+  int m, n, ldb;
+  double alpha;
+  explicit SolveTask(const dm_task& t)
+      : side(t.side), uplo(t.uplo), trans(t.transa), diag(t.diag), m(t.m), n(t.n), ldb(t.ldc),
+        alpha(t.alpha) {
+    if (t.op != DM_OP_TRSV) return;
+    const bool row = t.ldc != 1;
+    side = row ? 'R' : 'L';
+    if (row) trans = is_trans(t.transa) ? 'N' : 'T';
+    m = row ? 1 : t.n;
+    n = row ? t.n : 1;
+    ldb = row ? t.ldc : t.n;
+    alpha = 1.0;
+  }
+};
+
 }  // namespace
 
 int Dag::add(const dm_task& t) {
@@ -337,7 +360,7 @@ int Dag::build_device_tables() {
   auto align = [&](size_t a) { while (blob.size() % a) blob.push_back(0); };
   for (Group& G : groups) {
     if (is_cplx(G.dtype)) continue;  // complex tasks need no job tables
-    if (G.tasks.size() <= 1 && G.op != DM_OP_TRSM && G.op != DM_OP_GEMM) continue;
+    if (G.op != DM_OP_GEMM && !is_solve(G.op)) continue;
     if (G.op == DM_OP_GEMM) {
       const dm_task& t0 = tasks[G.tasks[0]].t;
       bool ta, tb;
@@ -391,45 +414,24 @@ int Dag::build_device_tables() {
       };
       int rc = G.dtype == DM_F64 ? fill((double*)nullptr) : fill((float*)nullptr);
       if (rc) return rc;
-    } else if (G.op == DM_OP_TRSM) {
-      const dm_task& t0 = tasks[G.tasks[0]].t;
-      G.shape = trsm_shape(t0.side, t0.uplo, t0.transa, t0.diag);
+    } else {
+      const SolveTask s0(tasks[G.tasks[0]].t);
+      G.shape = trsm_shape(s0.side, s0.uplo, s0.trans, s0.diag);
       auto fill = [&](auto* dummy) -> int {
         typedef std::remove_pointer_t<decltype(dummy)> T;
-        // one inverse-block buffer per distinct (A, L); job inv pointers
-        // hold offsets into the inverse area until the allocation exists
-        std::map<std::pair<const void*, int>, int> invidx;
         std::vector<TrsmJob<T>> jobs;
         for (int ti : G.tasks) {
           const dm_task& t = tasks[ti].t;
-          const int L = G.shape.side_l ? t.m : t.n;
-          const int NV = G.shape.side_l ? t.n : t.m;
+          const SolveTask v(t);
+          const int L = G.shape.side_l ? v.m : v.n;
+          const int NV = G.shape.side_l ? v.n : v.m;
           if (L <= 0 || NV <= 0) continue;
-          auto key = std::make_pair(t.a, L);
-          auto it = invidx.find(key);
-          int ii;
-          if (it == invidx.end()) {
-            ii = (int)G.inv_src.size();
-            invidx.emplace(key, ii);
-            InvSrc src;
-            src.A = t.a;
-            src.lda = t.lda;
-            src.L = L;
-            src.off = inv_bytes;
-            inv_bytes += sizeof(T) * (size_t)((L + TRSM_BS - 1) / TRSM_BS) * TRSM_BS * TRSM_BS;
-            inv_bytes = (inv_bytes + 255) & ~(size_t)255;
-            G.inv_src.push_back(src);
-          } else {
-            ii = it->second;
-          }
           TrsmJob<T> j{};
           j.A = (const T*)t.a; j.B = (T*)t.c;
-          j.inv = (const T*)(uintptr_t)G.inv_src[ii].off;  // patched after allocation
-          j.L = L; j.NV = NV; j.lda = t.lda; j.ldb = t.ldc;
-          j.alpha = (T)t.alpha;
+          j.L = L; j.NV = NV; j.lda = t.lda; j.ldb = v.ldb;
+          j.alpha = (T)v.alpha;
           jobs.push_back(j);
         }
-        G.batched_trsm = true;
         std::vector<TrsmStep<T>> steps;
         trsm_plan_steps<T>(G.shape, jobs, steps);
         for (TrsmStep<T>& st : steps) {
@@ -439,7 +441,7 @@ int Dag::build_device_tables() {
           rec.table_off = blob.size();
           if (st.leaf) {
             rec.njobs = (int)st.tjobs.size();
-            rec.maxL = st.maxL;
+            rec.nb = st.nb;
             for (const TrsmJob<T>& j : st.tjobs) rec.flops += (double)j.L * j.L * j.NV;
             rec.total_wg = st.total_wg;
             const unsigned char* p = (const unsigned char*)st.tjobs.data();
@@ -477,9 +479,8 @@ int Dag::build_device_tables() {
       if (rc) return rc;
     }
   }
-  // per-task workspace for launches that solve through trsm_full
-  // (POTRF recursion, unbatched TRSM/TRSV): allocated here so nothing is
-  // allocated while a run is issued or captured.
+  // per-task workspaces, allocated here so nothing is allocated while a run
+  // is issued or captured
   task_ws_off.assign(tasks.size(), (size_t)-1);
   size_t ws_bytes = 0;
   // LU panels share one workspace: they are ordered by their data (each
@@ -492,19 +493,8 @@ int Dag::build_device_tables() {
                                               : getrf_panel_ws_bytes<float>(r.t.m, r.t.n));
   if (getrf_bytes) {
     for (size_t i = 0; i < tasks.size(); ++i)
-      if (tasks[i].t.op == DM_OP_GETRF) task_ws_off[i] = 256 + inv_bytes;
+      if (tasks[i].t.op == DM_OP_GETRF) task_ws_off[i] = 256;
     ws_bytes = (getrf_bytes + 255) / 256 * 256;
-  }
-  for (Group& G : groups) {
-    const bool needs = !is_cplx(G.dtype) &&
-                       (G.op == DM_OP_TRSV || (G.op == DM_OP_TRSM && !G.batched_trsm));
-    if (!needs) continue;
-    const size_t per = G.dtype == DM_F64 ? trsm_ws_elems<double>() * sizeof(double)
-                                         : trsm_ws_elems<float>() * sizeof(float);
-    for (int ti : G.tasks) {
-      task_ws_off[ti] = 256 + inv_bytes + ws_bytes;
-      ws_bytes += per;
-    }
   }
   // FP32 POTRF tasks factored in FP64 (opts.f64_diag): an n x n FP64 tile
   // each, so concurrent POTRFs of independent matrices never share one
@@ -512,34 +502,17 @@ int Dag::build_device_tables() {
     for (size_t i = 0; i < tasks.size(); ++i) {
       const dm_task& t = tasks[i].t;
       if (t.op != DM_OP_POTRF || t.dtype != DM_F32) continue;
-      task_ws_off[i] = 256 + inv_bytes + ws_bytes;
+      task_ws_off[i] = 256 + ws_bytes;
       ws_bytes += ((size_t)t.n * t.n * sizeof(double) + 255) / 256 * 256;
     }
-  // device memory: [abort int (256 B)] [inverse blocks] [workspaces] [job tables]
-  const size_t tab_base = 256 + inv_bytes + ws_bytes;
+  // device memory: [abort int (256 B)] [workspaces] [job tables]
+  const size_t tab_base = 256 + ws_bytes;
   const size_t total = tab_base + blob.size();
   DM_HIP(hipMalloc(&dev_mem, total));
   abort_dev = (int*)dev_mem;
   unsigned char* base = (unsigned char*)dev_mem;
-  // patch inverse pointers inside the leaf tables of TRSM groups
-  for (Group& G : groups) {
-    if (G.op != DM_OP_TRSM) continue;
-    for (Group::Step& st : G.tsteps) {
-      if (!st.leaf) continue;
-      if (G.dtype == DM_F64) {
-        auto* jobs = (TrsmJob<double>*)(blob.data() + st.table_off);
-        for (int i = 0; i < st.njobs; ++i)
-          jobs[i].inv = (const double*)(base + 256 + (uintptr_t)jobs[i].inv);
-      } else {
-        auto* jobs = (TrsmJob<float>*)(blob.data() + st.table_off);
-        for (int i = 0; i < st.njobs; ++i)
-          jobs[i].inv = (const float*)(base + 256 + (uintptr_t)jobs[i].inv);
-      }
-    }
-  }
   for (Group& G : groups) {
     G.table_dev = base + tab_base + G.table_off;
-    for (InvSrc& s : G.inv_src) s.dev = base + 256 + s.off;
     for (Group::Step& st : G.tsteps) st.table_dev = base + tab_base + st.table_off;
   }
   if (!blob.empty()) DM_HIP(hipMemcpy(base + tab_base, blob.data(), blob.size(), hipMemcpyHostToDevice));
@@ -599,22 +572,16 @@ int Dag::launch_group_t(const Group& G, hipStream_t s) {
     return gemm_launch<T>(G.ta, G.tb, G.vec, G.cfg, (const GemmJob<T>*)G.table_dev, G.njobs, dummy,
                           G.total_wg, ab, s);
   }
-  if (G.op == DM_OP_TRSM && G.batched_trsm) {
-    for (const InvSrc& src : G.inv_src) {
-      int rc = trinv_blocks_launch<T>(G.shape, (const T*)src.A, src.lda, src.L, (T*)src.dev, ab, s,
-                                      prio);
-      if (rc) return rc;
-    }
+  if (is_solve(G.op)) {
     const bool prof = opts.profile && !capturing;
     for (const Group::Step& st : G.tsteps) {
       int rc;
       if (prof && st.ev0) DM_HIP(hipEventRecord(st.ev0, s));
       if (st.leaf) {
         TrsmJob<T> dummy{};
-        dummy.L = st.maxL;
         dummy.prio = prio;
         rc = trsm_launch<T>(G.shape, (const TrsmJob<T>*)st.table_dev, st.njobs, dummy, st.total_wg,
-                            ab, s);
+                            ab, s, st.nb);
       } else {
         GemmJob<T> dummy{};
         dummy.prio = prio;
@@ -644,10 +611,6 @@ int Dag::launch_group_t(const Group& G, hipStream_t s) {
         rc = potrf_full<T>(is_upper(t.uplo), t.n, (T*)t.c, t.ldc, t.info, abort_dev, gofs, ws, s);
         break;
       }
-      case DM_OP_TRSM:
-        rc = trsm_full<T>(t.side, t.uplo, t.transa, t.diag, t.m, t.n, (T)t.alpha, (const T*)t.a,
-                          t.lda, (T*)t.c, t.ldc, ws, ab, s);
-        break;
       case DM_OP_GEMM:
         rc = gemm_single<T>(is_trans(t.transa), is_trans(t.transb), t.m, t.n, t.k, (T)t.alpha,
                             (const T*)t.a, t.lda, (const T*)t.b, t.ldb, (T)t.beta, (T*)t.c, t.ldc,
@@ -670,14 +633,6 @@ int Dag::launch_group_t(const Group& G, hipStream_t s) {
         break;
       case DM_OP_LASWP:
         rc = laswp_tiled<T>((T*)t.c, t.m, t.n, t.k, (const int*)t.b, t.lda, t.ldb, ab, s);
-        break;
-      case DM_OP_TRSV:
-        if (t.ldc == 1)
-          rc = trsm_full<T>('L', t.uplo, t.transa, t.diag, t.n, 1, T(1), (const T*)t.a, t.lda,
-                            (T*)t.c, t.n, ws, ab, s);
-        else
-          rc = trsm_full<T>('R', t.uplo, is_trans(t.transa) ? 'N' : 'T', t.diag, 1, t.n, T(1),
-                            (const T*)t.a, t.lda, (T*)t.c, t.ldc, ws, ab, s);
         break;
     }
     if (rc) return rc;
@@ -778,7 +733,7 @@ int Dag::launches() const {
   int n = 0;
   for (const Group& G : groups) {
     if (G.op == DM_OP_GEMM) n += G.njobs > 0 ? 1 : 0;
-    else if (G.op == DM_OP_TRSM && G.batched_trsm) n += (int)(G.inv_src.size() + G.tsteps.size());
+    else if (is_solve(G.op) && !is_cplx(G.dtype)) n += (int)G.tsteps.size();
     else n += (int)G.tasks.size();
   }
   return n;
@@ -892,7 +847,7 @@ int dm_dag_profile(dm_dag_t dag, dm_group_profile* out, int* count) {
   for (int g : d.order) {
     const Group& G = d.groups[g];
     int rc;
-    if (G.op == DM_OP_TRSM && G.batched_trsm && !G.tsteps.empty() && G.tsteps[0].ev0) {
+    if (is_solve(G.op) && !G.tsteps.empty() && G.tsteps[0].ev0) {
       // one record per launch of the batched solve: leaf solves (TRSM) and
       // the GEMM updates between them
       for (const Group::Step& st : G.tsteps) {

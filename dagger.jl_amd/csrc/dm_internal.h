@@ -174,7 +174,6 @@ template <typename T>
 struct TrsmJob {
   const T* A;
   T* B;
-  const T* inv;  // inverted 32x32 diagonal blocks of Tm (device)
   int L, NV;
   int lda, ldb;
   T alpha;
@@ -190,53 +189,40 @@ struct TrsmShape {
 };
 TrsmShape trsm_shape(char side, char uplo, char transa, char diag);
 
-constexpr int TRSM_BS = 32;     // diagonal block inverted up front
-constexpr int TRSM_LEAF = 256;  // longest solve held in LDS (longer ones recurse)
-int trsm_leaf_len();            // recursion leaf length in use (128)
-constexpr int TRSM_VPW = 64;    // vectors per workgroup of the leaf kernel (16 per wave)
-// Workspace (elements) for any trsm_full / potrf_full call: the inverted
-// diagonal blocks of one leaf solve.
-template <typename T>
-constexpr size_t trsm_ws_elems() {
-  return (size_t)(TRSM_LEAF / TRSM_BS) * TRSM_BS * TRSM_BS;
-}
-
-// Inverts the 32x32 diagonal blocks of Tm into inv (ceil(L/32)*1024 elems).
-template <typename T>
-int trinv_blocks_launch(const TrsmShape& sh, const T* A, int lda, int L, T* inv,
-                        const int* abort, hipStream_t s, int prio = 0);
-// Batched / single leaf solve (L <= TRSM_LEAF; jobs' inv point at the
-// inverted blocks of their own triangle).  single.L: longest L of the launch.
+constexpr int TRSM_LEAF = 512;  // longest solve of one launch (longer ones recurse)
+// 16-vector blocks per workgroup of the leaf kernel: two when that still gives
+// every CU a workgroup (the triangle is read once per workgroup and its steps'
+// fixed costs are shared; 512 rows, 16384 vectors from the right: FP64 139 us
+// with two and about 200 with one, FP32 95 and 131), else one: a CU left without a
+// workgroup would cost more (512 rows, 4096 vectors take 46 us with one)
+inline int trsm_vec_blocks(long vectors) { return vectors >= 32 * 256 ? 2 : 1; }
+inline int trsm_wgs(int NV, int nb) { return (NV + 16 * nb - 1) / (16 * nb); }
+// Batched / single leaf solve (L <= TRSM_LEAF) over total_wg workgroups of nb
+// 16-vector blocks each.
 template <typename T>
 int trsm_launch(const TrsmShape& sh, const TrsmJob<T>* jobs_dev, int njobs,
                 const TrsmJob<T>& single, long total_wg, const int* abort,
-                hipStream_t s, long max_wg = 0);
-int trsm_init_attributes();
-inline int trsm_wgs(int NV) { return (NV + TRSM_VPW - 1) / TRSM_VPW; }
+                hipStream_t s, long nb);
 
 // Recursive batched solve: the launches (leaf solves and GEMM updates, in
-// issue order) that solve every job of `jobs` (any lengths).  Split points
-// are multiples of TRSM_BS from the top of each triangle, so a job's inverse
-// blocks (computed once over its full triangle) serve every leaf.
+// issue order) that solve every job of `jobs` (any lengths).
 template <typename T>
 struct TrsmStep {
   bool leaf = true;
   std::vector<TrsmJob<T>> tjobs;  // leaf solves (wg_begin filled)
   std::vector<GemmJob<T>> gjobs;  // update C = alpha_j V2 - Tm21 X1
   bool ta = false, tb = false;    // update operand transposes
-  int maxL = 0;
+  int nb = 1;  // leaf solves: 16-vector blocks per workgroup
   long total_wg = 0;
 };
-// leaf: recursion leaf length (0: trsm_leaf_len())
 template <typename T>
 void trsm_plan_steps(const TrsmShape& sh, const std::vector<TrsmJob<T>>& jobs,
-                     std::vector<TrsmStep<T>>& steps, int leaf = 0);
+                     std::vector<TrsmStep<T>>& steps);
 
-// Full BLAS trsm (any size; host recursion above TRSM_LEAF, inverse blocks
-// formed per leaf in ws).
+// Full BLAS trsm (any size; host recursion above TRSM_LEAF).
 template <typename T>
 int trsm_full(char side, char uplo, char transa, char diag, int m, int n,
-              T alpha, const T* A, int lda, T* B, int ldb, T* ws,
+              T alpha, const T* A, int lda, T* B, int ldb,
               const int* abort, hipStream_t s);
 
 // ------------------------------------------------------------ POTRF

@@ -191,7 +191,7 @@ unsigned blocks_of(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 // getrf2's recursion on columns [c0, c0 + nc) of the contiguous panel.
 template <typename T>
-int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, T* ws, int* abort,
+int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, int* abort,
               bool pivot, hipStream_t s) {
   if (nc <= LU_LEAF) {
     hipLaunchKernelGGL((getf2_leaf_kernel<T>), dim3(1), dim3(LU_THREADS), 0, s, P, Mp, c0, nc, piv,
@@ -200,7 +200,7 @@ int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, T* ws, int
     return 0;
   }
   const int n1 = ((nc / 2 + LU_LEAF - 1) / LU_LEAF) * LU_LEAF, n2 = nc - n1;
-  int rc = getrf_rec<T>(P, Mp, c0, n1, piv, linfo, ws, abort, pivot, s);
+  int rc = getrf_rec<T>(P, Mp, c0, n1, piv, linfo, abort, pivot, s);
   if (rc) return rc;
   const int64_t ld = Mp;
   if (pivot) {  // left half's swaps on the right half
@@ -212,7 +212,7 @@ int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, T* ws, int
   T* A12 = P + (int64_t)(c0 + n1) * ld + c0;
   T* A21 = P + (int64_t)c0 * ld + c0 + n1;
   T* A22 = P + (int64_t)(c0 + n1) * ld + c0 + n1;
-  rc = trsm_full<T>('L', 'L', 'N', 'U', n1, n2, T(1), A11, (int)ld, A12, (int)ld, ws, abort, s);
+  rc = trsm_full<T>('L', 'L', 'N', 'U', n1, n2, T(1), A11, (int)ld, A12, (int)ld, abort, s);
   if (rc) return rc;
   if (Mp > c0 + n1) {
     rc = gemm_single<T>(false, false, (int)(Mp - c0 - n1), n2, n1, T(-1), A21, (int)ld, A12,
@@ -220,7 +220,7 @@ int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, T* ws, int
     if (rc) return rc;
   }
   if (Mp > c0 + n1) {
-    rc = getrf_rec<T>(P, Mp, c0 + n1, n2, piv, linfo, ws, abort, pivot, s);
+    rc = getrf_rec<T>(P, Mp, c0 + n1, n2, piv, linfo, abort, pivot, s);
     if (rc) return rc;
     if (pivot) {  // right half's swaps on the left half
       hipLaunchKernelGGL((laswp_contig_kernel<T>), dim3(blocks_of(n1, 64)), dim3(64), 0, s, P, ld,
@@ -232,13 +232,12 @@ int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, T* ws, int
 }
 }  // namespace
 
-// Workspace elements of a panel factorization: the contiguous panel, the
-// TRSM's inverted diagonal blocks, then W + 1 ints (pivots, local info).
+// Workspace bytes of a panel factorization: the contiguous panel, then W + 1
+// ints (pivots, local info).
 template <typename T>
 size_t getrf_panel_ws_bytes(int64_t Mp, int W) {
   const size_t panel = sizeof(T) * (size_t)Mp * W;
-  const size_t trsm = sizeof(T) * trsm_ws_elems<T>();
-  return ((panel + 255) / 256) * 256 + ((trsm + 255) / 256) * 256 + 4 * ((size_t)W + 64);
+  return ((panel + 255) / 256) * 256 + 4 * ((size_t)W + 64);
 }
 
 // LU of a tiled panel: the tiles (k..mt-1, k) starting at `tiles` (Mp rows
@@ -251,8 +250,7 @@ int getrf_panel(T* tiles, int64_t Mp, int W, int mb, int64_t row0, int* ipiv, in
   char* w = (char*)wsp;
   T* P = (T*)w;
   const size_t panel = ((sizeof(T) * (size_t)Mp * W + 255) / 256) * 256;
-  T* tws = (T*)(w + panel);
-  int* piv = (int*)(w + panel + ((sizeof(T) * trsm_ws_elems<T>() + 255) / 256) * 256);
+  int* piv = (int*)(w + panel);
   int* linfo = piv + W;
   const int npiv = (int)std::min<int64_t>(Mp, W);
   int rc = fill_i32_launch(linfo, 0, 1, s);
@@ -260,7 +258,7 @@ int getrf_panel(T* tiles, int64_t Mp, int W, int mb, int64_t row0, int* ipiv, in
   hipLaunchKernelGGL((panel_pack_kernel<T>), dim3(blocks_of(Mp * W, 256)), dim3(256), 0, s, P,
                      tiles, Mp, W, mb, 0);
   DM_LAUNCH_CHECK("panel_pack_kernel");
-  rc = getrf_rec<T>(P, Mp, 0, npiv, piv, linfo, tws, abort, pivot, s);
+  rc = getrf_rec<T>(P, Mp, 0, npiv, piv, linfo, abort, pivot, s);
   if (rc) return rc;
   if (W > npiv) {  // a panel wider than tall: the rest gets the swaps and L11^-1
     if (pivot) {
@@ -269,7 +267,7 @@ int getrf_panel(T* tiles, int64_t Mp, int W, int mb, int64_t row0, int* ipiv, in
       DM_LAUNCH_CHECK("laswp_contig_kernel");
     }
     rc = trsm_full<T>('L', 'L', 'N', 'U', npiv, W - npiv, T(1), P, (int)Mp,
-                      P + (int64_t)npiv * Mp, (int)Mp, tws, abort, s);
+                      P + (int64_t)npiv * Mp, (int)Mp, abort, s);
     if (rc) return rc;
   }
   hipLaunchKernelGGL((panel_pack_kernel<T>), dim3(blocks_of(Mp * W, 256)), dim3(256), 0, s, P,

@@ -8,17 +8,10 @@
 //     transposed, lower or upper triangular;
 //   * the right-hand-side vectors are the columns (side L) or rows (side R)
 //     of B, solved in place.
-// Solves longer than 256 are split on the host at a multiple of 32 from the
-// top of the triangle: solve the first part, update the second part with one
-// (batched) GEMM on the MFMA GEMM kernel, solve the second part -- so most of
-// the flops of a long solve run at GEMM speed.
-// A leaf (L <= 256) is one kernel: a workgroup owns 64 vectors, each of its
-// four waves 16 of them, with no cross-wave synchronisation.  A wave keeps its
-// solved part in LDS and walks 32-row blocks of Tm in solve order: MFMA
-// products of the block's rows with the solved part, then one MFMA product
-// with the pre-inverted 32x32 diagonal block.  The diagonal blocks are
-// inverted up front by a small kernel (one thread per column, exact
-// substitution), so the serial part of each block is a short MFMA chain.
+// Solves longer than TRSM_LEAF are split on the host: solve the first part,
+// update the second part with one (batched) GEMM on the MFMA GEMM kernel,
+// solve the second part -- so most of the flops of a long solve run at GEMM
+// speed.  A leaf is one launch of trsm_kernel; it needs no workspace.
 #include "dm_internal.h"
 #include "trsm_plan.h"
 
@@ -43,50 +36,32 @@ template <> struct MfmaT<float> {
   }
 };
 
-template <typename T, bool TTRANS>
-__device__ __forceinline__ T tm_at(const T* __restrict__ A, int lda, int i, int k) {
-  const auto g = gptr(A);
-  return TTRANS ? g[(size_t)i * lda + k] : g[(size_t)k * lda + i];
-}
+// Two elements at an address aligned to one.
+template <typename T> struct Pair;
+template <> struct Pair<double> { typedef double t __attribute__((ext_vector_type(2), aligned(8))); };
+template <> struct Pair<float> { typedef float t __attribute__((ext_vector_type(2), aligned(4))); };
 
-// inv[b*1024 + c*32 + r] = (Tm_bb^-1)(r, c); rows/cols past L act as identity.
-// One workgroup per diagonal block, one thread per column of the inverse.
-template <typename T, bool LOWER, bool TTRANS, bool UNIT>
-__global__ __launch_bounds__(32) void trinv_blocks_kernel(const T* __restrict__ A, int lda, int L,
-                                                          T* __restrict__ inv,
-                                                          const int* __restrict__ abort,
-                                                          int prio) {
-  __shared__ T tb[TRSM_BS][TRSM_BS + 1];  // Tm_bb, row-major
-  __shared__ T xs[TRSM_BS][TRSM_BS + 1];  // column c of the inverse in xs[.][c]
-  if (abort && *abort) return;
-  if (prio) raise_wave_priority();
-  const int b = blockIdx.x;
-  const int c = threadIdx.x;
-  const int r0 = b * TRSM_BS;
-  const int nb = min(TRSM_BS, L - r0);
-  for (int r = 0; r < TRSM_BS; ++r) {
-    T v = (r == c) ? T(1) : T(0);
-    if (r < nb && c < nb) v = tm_at<T, TTRANS>(A, lda, r0 + r, r0 + c);
-    tb[r][c] = v;
-    xs[r][c] = T(0);
-  }
-  __syncthreads();
-  if (LOWER) {
-    for (int r = c; r < TRSM_BS; ++r) {
-      T s = (r == c) ? T(1) : T(0);
-      for (int p = c; p < r; ++p) s -= tb[r][p] * xs[p][c];
-      xs[r][c] = (UNIT || r >= nb) ? s : s / tb[r][r];
-    }
-  } else {
-    for (int r = c; r >= 0; --r) {
-      T s = (r == c) ? T(1) : T(0);
-      for (int p = r + 1; p <= c; ++p) s -= tb[r][p] * xs[p][c];
-      xs[r][c] = (UNIT || r >= nb) ? s : s / tb[r][r];
-    }
-  }
-  __syncthreads();
-  T* out = inv + (size_t)b * TRSM_BS * TRSM_BS;
-  for (int r = 0; r < TRSM_BS; ++r) out[(size_t)c * TRSM_BS + r] = xs[r][c];
+constexpr int TB = 16;                 // block row
+constexpr int TW = 16;                 // waves of a workgroup
+constexpr int TQ = TRSM_LEAF / (TB * TW);  // block rows per wave
+// Steps of the triangle in flight, as many as the registers of 16 waves hold.
+template <typename T, int NB> constexpr int trsm_depth() {
+  return sizeof(T) == 4 ? 4 : NB == 1 ? 2 : 1;
+}
+constexpr int TIS = TB + 1;            // LDS row stride of an inverted diagonal block
+
+// A wave-uniform element offset, kept out of the optimizer's sight: it would
+// otherwise turn every (step, row, column) of the unrolled loop into a vector
+// pointer of its own and spill.  In 32-bit halves: as one 64-bit asm operand
+// the compiler puts a negative constant such as -32 into an s_mov_b64 with a
+// 32-bit literal, which the hardware extends with zeros.
+__device__ __forceinline__ ptrdiff_t uniform_offset(ptrdiff_t o) {
+#ifdef __HIP_DEVICE_COMPILE__
+  int lo = (int)o, hi = (int)(o >> 32);
+  asm volatile("" : "+s"(lo), "+s"(hi));
+  o = (ptrdiff_t)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+#endif
+  return o;
 }
 
 // Orders this wave's LDS writes before its later LDS reads.
@@ -96,250 +71,327 @@ __device__ __forceinline__ void trsm_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <typename T, bool LOWER, bool TTRANS, bool SIDE_L>
-__global__ __launch_bounds__(256) void trsm_kernel(const TrsmJob<T>* __restrict__ jobs, int njobs,
-                                                   TrsmJob<T> single, int total,
-                                                   const int* __restrict__ abort) {
+// One leaf solve.  A workgroup owns 16 NB vectors and the whole triangle; an
+// upper triangle is solved as the lower one that reversing both axes gives,
+// so everything below is forward substitution over 16-row blocks.  Wave w
+// owns block rows w, w + 16, ...: their right-hand sides, their sums
+// sum_k T_pk X_k in matrix-core accumulators, and W_p, the inverse of their
+// diagonal blocks (16 x 16, formed first, in LDS):
+//   X_p = W_p (alpha V_p - sum_{k<p} T_pk X_k).
+// The chain from X_J to X_{J+1} is two block products, a trip through LDS and
+// a barrier; the other waves' products (T_pJ X_J, p > J + 1) run beside it.
+// (W_p T_{p,p-1} formed ahead would halve the chain, but it measured no faster
+// and loses accuracy where a diagonal block is badly conditioned.)  T comes
+// straight from global memory as matrix-core operands, loaded a few steps
+// ahead.
+//
+// Bound by three things in turn: 512 rows and 16 vectors in FP64 are 13 us of
+// matrix-core work for one CU, and the 32 steps cost about 0.2 us each for the
+// barrier and 0.4 us each for the chain.  Measured with the launch, 512 rows
+// (left side, A^T; A; right side): 16 vectors FP64 51, 45 and 41 us, FP32 44,
+// 32 and 29; 16384 vectors FP64 158, 150 and 139 us, FP32 127, 104 and 95.  The
+// launches this replaces took about 210 us for 16 vectors (four solves of 128
+// rows at 31 us that kept a whole 32-row chain in one wave, the products
+// between them and the inversion of the diagonal blocks).  Loads made
+// unconditional or a deeper prefetch measured slower or the same.
+template <typename T, bool LOWER, bool TTRANS, bool SIDE_L, int NB>
+__global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restrict__ jobs,
+                                                       int njobs, TrsmJob<T> single, int unit,
+                                                       const int* __restrict__ abort) {
   typedef typename MfmaT<T>::v4 v4;
-  DM_DYNAMIC_LDS(dm_trsm_smem);
+  constexpr int TD = trsm_depth<T, NB>();
+  __shared__ T Wd[TRSM_LEAF / TB][TB * TIS];   // diagonal blocks, then their inverses
+  __shared__ T Xs[2][TB * TB * NB];            // X_J: [k][vector]
   if (abort && *abort) return;
   if (single.prio) raise_wave_priority();
-  // A launch may have fewer workgroups than units of 64 vectors: each
-  // workgroup then loops over its share (waves never synchronise, so a wave
-  // simply moves on to its next unit).
-  for (int wg = blockIdx.x; wg < total; wg += gridDim.x) {
   TrsmJob<T> job;
-  int local;
+  int local = blockIdx.x;
   if (njobs == 0) {
     job = single;
-    local = wg;
   } else {
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
-      if (jobs[mid].wg_begin <= wg) lo = mid; else hi = mid - 1;
+      if (jobs[mid].wg_begin <= local) lo = mid; else hi = mid - 1;
     }
     job = jobs[lo];
-    local = wg - job.wg_begin;
+    local -= job.wg_begin;
   }
-  // The LDS layout follows the launch's longest solve (single.L).
-  const int Lmax = ((single.L + TRSM_BS - 1) / TRSM_BS) * TRSM_BS;
-  const int L = job.L, NV = job.NV;
-  const int nblk = (L + TRSM_BS - 1) / TRSM_BS;
-  const int Lp = nblk * TRSM_BS;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lr = lane & 15, lk = lane >> 4;
-  T* X = reinterpret_cast<T*>(dm_trsm_smem) + (size_t)wave * (Lmax + TRSM_BS) * 16;  // [Lp][16]
-  T* bt = X + (size_t)Lmax * 16;                                                     // [32][16]
-  const int j0 = local * TRSM_VPW + wave * 16;  // first vector of this wave
-  if (j0 >= NV) continue;                       // waves never synchronise with each other
-  const T* __restrict__ A = job.A;
+  const int L = job.L, NV = job.NV, nblk = (L + TB - 1) / TB;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int wave = __builtin_amdgcn_readlane((int)threadIdx.x >> 6, 0);
+  const int j0 = local * TB * NB;
+  const auto A = gptr(job.A);
   const auto B = gptr(job.B);
-  const int lda = job.lda, ldb = job.ldb;
-  const T alpha = job.alpha;
-  const int gj = j0 + lr;  // this lane's vector in the MFMA output layout
+  const size_t lda = job.lda, ldb = job.ldb;
+  // element (i, k) of the lower triangle, element i of vector j
+  auto a_off = [&](int i, int k) -> size_t {
+    if (!LOWER) {
+      i = L - 1 - i;
+      k = L - 1 - k;
+    }
+    return TTRANS ? (size_t)i * lda + k : (size_t)k * lda + i;
+  };
+  // this lane's element of block row 0 and the steps along rows and vectors
+  const ptrdiff_t bstep = (LOWER ? 1 : -1) * (SIDE_L ? 1 : (ptrdiff_t)ldb);
+  const ptrdiff_t vstep = SIDE_L ? (ptrdiff_t)ldb : 1;
+  const auto brow = B + (LOWER ? 0 : (L - 1) * (SIDE_L ? 1 : (ptrdiff_t)ldb)) +
+                    MfmaT<T>::row(lk, 0) * bstep + (j0 + lr) * vstep;
+  constexpr int RS = sizeof(T) == 8 ? 4 : 1;  // row(lk, r) = row(lk, 0) + RS r
+  auto b_at = [&](int p, int r, int n) {
+    return brow + uniform_offset((TB * p + RS * r) * bstep + TB * n * vstep);
+  };
+  // T_pJ as the operand of four k-steps: row 16 p + lr, columns 16 J + tk(lk, s)
+  // (rows past the triangle repeat its last one; their results are dropped).
+  // tk makes the lanes of a row read whole 64-byte pieces of it.
+  auto tk = [](int k, int s) { return 2 * k + (s & 1) + 8 * (s >> 1); };
+  // trow[q]: this lane's row of the wave's block row q at column tk(lk, 0)
+  decltype(gptr(job.A)) trow[TQ];
+#pragma unroll
+  for (int q = 0; q < TQ; ++q)
+    trow[q] = A + a_off(min(TB * (wave + TW * q) + lr, L - 1),
+                        2 * lk + (TTRANS && !LOWER ? 1 : 0));
+  const ptrdiff_t kstep = (LOWER ? 1 : -1) * (TTRANS ? 1 : (ptrdiff_t)lda);
+  auto load_t = [&](int q, int J, T (&t)[4]) {
+    const int p = wave + TW * q;
+    if (J >= p || p >= nblk) return;
+    const auto src = trow[q] + uniform_offset((ptrdiff_t)(TB * J) * kstep);
+    if (TTRANS) {
+      typedef typename Pair<T>::t V2;
+      const V2 u = *(const DM_GLOBAL_AS V2*)src, v = *(const DM_GLOBAL_AS V2*)(src + 8 * kstep);
+      t[0] = LOWER ? u[0] : u[1];
+      t[1] = LOWER ? u[1] : u[0];
+      t[2] = LOWER ? v[0] : v[1];
+      t[3] = LOWER ? v[1] : v[0];
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) t[s] = src[tk(0, s) * kstep];
+    }
+  };
 
-  for (int e = lane; e < Lp * 16; e += 64) X[e] = T(0);
+  // ---- inverses of the diagonal blocks, the wave's all at once: lane group g
+  // of 16 inverts block wave + 16 g (its two 8 x 8 diagonal blocks by
+  // substitution, one column per lane, then the coupling block -V1 (L21 V0))
+#pragma unroll
+  for (int q = 0; q < TQ; ++q) {
+    const int p = wave + TW * q;
+    if (p >= nblk) continue;
+    T d[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int x = lr, y = 4 * e + lk;  // x along the contiguous axis
+      const int r = TTRANS ? y : x, c = TTRANS ? x : y;
+      const bool in = TB * p + r < L && TB * p + c < L && r >= c;
+      d[e] = A[in ? a_off(TB * p + r, TB * p + c) : 0];
+      if (!in || (unit && r == c)) d[e] = r == c ? T(1) : T(0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int x = lr, y = 4 * e + lk;
+      Wd[p][(TTRANS ? y : x) * TIS + (TTRANS ? x : y)] = d[e];
+    }
+  }
   trsm_wave_sync();
-
-  for (int bi = 0; bi < nblk; ++bi) {
-    const int b = LOWER ? bi : nblk - 1 - bi;
-    const int r0 = b * TRSM_BS;
-    // ---- acc = Tm[I, solved] X[solved]  (rows r0 + 0..15 and r0 + 16..31)
-    const int kbeg = LOWER ? 0 : r0 + TRSM_BS;
-    const int kend = LOWER ? r0 : L;
-    const int nsteps = (kend - kbeg + 3) >> 2;
-    v4 acc[2][2];
+  static_assert(TQ <= 4, "one lane group of 16 per diagonal block");
+  {
+    const int p = wave + TW * lk;
+    const bool on = lk < TQ && p < nblk;
+    T* W = Wd[on ? p : wave % nblk];
+    const int o = lr & 8, c = lr & 7;
+    T x[8], z[4];
+    const T dinv = T(1) / W[lr * TIS + lr];
+    // the block's two 8 x 8 triangles, columns by lane
 #pragma unroll
-    for (int h = 0; h < 2; ++h) acc[h][0] = acc[h][1] = v4{0, 0, 0, 0};
-    const int ra = r0 + lr, rb = r0 + 16 + lr;
-    const bool raok = ra < L, rbok = rb < L;
-    int st = 0;
-    // four k-steps per iteration: eight Tm loads in flight per lane (a leaf
-    // workgroup runs one wave per SIMD, so latency is hidden by ILP only)
-    for (; st + 4 <= nsteps; st += 4) {
-      T ta[4], tb[4], xv[4];
+    for (int r = 0; r < 8; ++r) x[r] = r == c ? T(1) : T(0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = kbeg + 4 * (st + q) + lk;
-        const bool ok = k < kend;
-        ta[q] = (ok && raok) ? tm_at<T, TTRANS>(A, lda, ra, k) : T(0);
-        tb[q] = (ok && rbok) ? tm_at<T, TTRANS>(A, lda, rb, k) : T(0);
-        xv[q] = ok ? X[k * 16 + lr] : T(0);
-      }
+    for (int r = 0; r < 8; ++r) {
+      x[r] *= __shfl(dinv, (lane & 56) + r, 64);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        acc[0][q & 1] = MfmaT<T>::mac(ta[q], xv[q], acc[0][q & 1]);
-        acc[1][q & 1] = MfmaT<T>::mac(tb[q], xv[q], acc[1][q & 1]);
-      }
+      for (int i = r + 1; i < 8; ++i) x[i] -= W[(o + i) * TIS + o + r] * x[r];
     }
-    for (; st + 2 <= nsteps; st += 2) {
-      const int k0 = kbeg + 4 * st + lk, k1 = k0 + 4;
-      const bool ok0 = k0 < kend, ok1 = k1 < kend;
-      const T t00 = (ok0 && raok) ? tm_at<T, TTRANS>(A, lda, ra, k0) : T(0);
-      const T t10 = (ok0 && rbok) ? tm_at<T, TTRANS>(A, lda, rb, k0) : T(0);
-      const T t01 = (ok1 && raok) ? tm_at<T, TTRANS>(A, lda, ra, k1) : T(0);
-      const T t11 = (ok1 && rbok) ? tm_at<T, TTRANS>(A, lda, rb, k1) : T(0);
-      const T x0 = ok0 ? X[k0 * 16 + lr] : T(0);
-      const T x1 = ok1 ? X[k1 * 16 + lr] : T(0);
-      acc[0][0] = MfmaT<T>::mac(t00, x0, acc[0][0]);
-      acc[1][0] = MfmaT<T>::mac(t10, x0, acc[1][0]);
-      acc[0][1] = MfmaT<T>::mac(t01, x1, acc[0][1]);
-      acc[1][1] = MfmaT<T>::mac(t11, x1, acc[1][1]);
-    }
-    if (st < nsteps) {
-      const int k0 = kbeg + 4 * st + lk;
-      const bool ok0 = k0 < kend;
-      const T t00 = (ok0 && raok) ? tm_at<T, TTRANS>(A, lda, ra, k0) : T(0);
-      const T t10 = (ok0 && rbok) ? tm_at<T, TTRANS>(A, lda, rb, k0) : T(0);
-      const T x0 = ok0 ? X[k0 * 16 + lr] : T(0);
-      acc[0][0] = MfmaT<T>::mac(t00, x0, acc[0][0]);
-      acc[1][0] = MfmaT<T>::mac(t10, x0, acc[1][0]);
-    }
-    // ---- bt = alpha V_I - acc  (lane: rows h*16 + row(lk, r), vector lr)
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = h * 16 + MfmaT<T>::row(lk, r);
-        const int gi = r0 + i;
-        T v = T(0);
-        if (gi < L && gj < NV) {
-          const T bv = SIDE_L ? B[(size_t)gj * ldb + gi] : B[(size_t)gi * ldb + gj];
-          v = alpha * bv - (acc[h][0][r] + acc[h][1][r]);
-        }
-        bt[i * 16 + lr] = v;
-      }
     trsm_wave_sync();
-    // ---- X_I = inv(Tm_II) bt
-    const auto iv = gptr(job.inv + (size_t)b * TRSM_BS * TRSM_BS);
+    if (on)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      v4 xa = v4{0, 0, 0, 0}, xb = v4{0, 0, 0, 0};
+      for (int r = 0; r < 8; ++r) W[(o + r) * TIS + o + c] = x[r];
+    trsm_wave_sync();
+    // Z = L21 V0 (rows 4 (lr / 8) + y, column c), through the upper block
 #pragma unroll
-      for (int kk = 0; kk < TRSM_BS / 4; kk += 2) {
-        const int c0 = 4 * kk + lk, c1 = 4 * (kk + 1) + lk;
-        xa = MfmaT<T>::mac(iv[c0 * TRSM_BS + h * 16 + lr], bt[c0 * 16 + lr], xa);
-        xb = MfmaT<T>::mac(iv[c1 * TRSM_BS + h * 16 + lr], bt[c1 * 16 + lr], xb);
-      }
+    for (int y = 0; y < 4; ++y) {
+      z[y] = T(0);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = h * 16 + MfmaT<T>::row(lk, r);
-        const int gi = r0 + i;
-        const T v = xa[r] + xb[r];
-        X[gi * 16 + lr] = v;
-        if (gi < L && gj < NV) {
-          if (SIDE_L) B[(size_t)gj * ldb + gi] = v;
-          else B[(size_t)gi * ldb + gj] = v;
-        }
-      }
+      for (int k = 0; k < 8; ++k) z[y] += W[(8 + (o >> 1) + y) * TIS + k] * W[k * TIS + c];
     }
+    trsm_wave_sync();
+    if (on)
+#pragma unroll
+      for (int y = 0; y < 4; ++y) W[((o >> 1) + y) * TIS + 8 + c] = z[y];
+    trsm_wave_sync();
+    T w21[4];
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+      w21[y] = T(0);
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        w21[y] -= W[(8 + (o >> 1) + y) * TIS + 8 + k] * W[k * TIS + 8 + c];
+    }
+    trsm_wave_sync();
+    if (on)
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        W[(8 + (o >> 1) + y) * TIS + c] = w21[y];
+        W[((o >> 1) + y) * TIS + 8 + c] = T(0);
+      }
     trsm_wave_sync();
   }
+
+  // (no load is moved above this point: the registers are needed above)
+  asm volatile("" ::: "memory");
+  // ---- this wave's right-hand sides (accumulator layout)
+  T vals[TQ][NB][4];
+#pragma unroll
+  for (int q = 0; q < TQ; ++q) {
+    const int p = wave + TW * q;
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = TB * p + MfmaT<T>::row(lk, r), j = j0 + TB * n + lr;
+        const bool in = i < L && j < NV;
+        vals[q][n][r] = *(in ? b_at(p, r, n) : B);
+        if (!in) vals[q][n][r] = T(0);
+      }
+  }
+  // the triangle's first TD steps
+  T t[TD][TQ][4];
+#pragma unroll
+  for (int u = 0; u < TD; ++u)
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) {
+      if (nblk > 1) load_t(q, u, t[u][q]);
+    }
+  // ---- forward substitution
+  v4 acc[TQ][NB];
+#pragma unroll
+  for (int q = 0; q < TQ; ++q)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[q][n] = v4{0, 0, 0, 0};
+  const T alpha = job.alpha;
+  // X_p of block row p = wave + 16 q: to B, and to LDS for the later rows
+  auto finish = [&](int p, const v4 (&x)[NB]) {
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        Xs[p & 1][(MfmaT<T>::row(lk, r) * NB + n) * TB + lr] = x[n][r];
+    }
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = TB * p + MfmaT<T>::row(lk, r), j = j0 + TB * n + lr;
+        if (i < L && j < NV) *b_at(p, r, n) = x[n][r];
+      }
+  };
+  // X_p = W_p (alpha V_p - sum)
+  auto solve = [&](int p, const T (&v)[NB][4], const v4 (&sum)[NB]) {
+    T w[4];
+    v4 x[NB];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) w[s] = Wd[p][lr * TIS + MfmaT<T>::row(lk, s)];
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      x[n] = v4{0, 0, 0, 0};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        // the accumulator's item s is the operand of k-step s (same lane)
+        const T rhs =
+            TB * p + MfmaT<T>::row(lk, s) < L ? alpha * v[n][s] - sum[n][s] : T(0);
+        x[n] = MfmaT<T>::mac(w[s], rhs, x[n]);
+      }
+    }
+    finish(p, x);
+  };
+  if (wave == 0) solve(0, vals[0], acc[0]);
+  __syncthreads();
+  auto step = [&](int J, T (&tj)[TQ][4]) {
+    T x[NB][4];
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) x[n][s] = Xs[J & 1][(tk(lk, s) * NB + n) * TB + lr];
+    auto update = [&](int q) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[q][n] = MfmaT<T>::mac(tj[q][s], x[n][s], acc[q][n]);
+    };
+    // the next block row first, ahead of the other waves
+#pragma unroll
+    for (int q = 0; q < TQ; ++q)
+      if (wave + TW * q == J + 1 && J + 1 < nblk) {
+        __builtin_amdgcn_s_setprio(3);
+        update(q);
+        solve(J + 1, vals[q], acc[q]);
+        __builtin_amdgcn_s_setprio(0);
+      }
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) {
+      const int p = wave + TW * q;
+      if (p > J + 1 && p < nblk) update(q);
+    }
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) load_t(q, J + TD, tj[q]);
+    __syncthreads();
+  };
+  // steps past the last block row only load (again) and pass the barrier
+#pragma unroll 1
+  for (int J = 0; J + 1 < nblk; J += TD) {
+#pragma unroll
+    for (int u = 0; u < TD; ++u) step(J + u, t[u]);
   }
 }
 
 // ------------------------------------------------------------ host side
 template <typename T>
-int trinv_blocks_launch(const TrsmShape& sh, const T* A, int lda, int L, T* inv,
-                        const int* abort, hipStream_t s, int prio) {
-  const int nblk = (L + TRSM_BS - 1) / TRSM_BS;
-  if (nblk <= 0) return 0;
-#define DM_TRINV(LO, TT, UN)                                                          \
-  hipLaunchKernelGGL((trinv_blocks_kernel<T, LO, TT, UN>), dim3(nblk), dim3(TRSM_BS), 0, s, A, \
-                     lda, L, inv, abort, prio)
+int trsm_launch(const TrsmShape& sh, const TrsmJob<T>* jobs_dev, int njobs,
+                const TrsmJob<T>& single, long total_wg, const int* abort, hipStream_t s, long nb) {
+  if (total_wg <= 0) return 0;
+  if (total_wg > 0x7fffffffL) return arg_fail(0, "trsm: too many workgroups");
+#define DM_TRSM_NB(LO, TT, SL, N)                                                            \
+  hipLaunchKernelGGL((trsm_kernel<T, LO, TT, SL, N>), dim3((unsigned)total_wg), dim3(64 * TW), \
+                     0, s, jobs_dev, njobs, single, sh.unit ? 1 : 0, abort)
+#define DM_TRSM_GO(LO, TT, SL)              \
+  do {                                      \
+    if (nb == 2) DM_TRSM_NB(LO, TT, SL, 2); \
+    else DM_TRSM_NB(LO, TT, SL, 1);         \
+  } while (0)
   if (sh.lower) {
-    if (sh.ttrans) { if (sh.unit) DM_TRINV(true, true, true); else DM_TRINV(true, true, false); }
-    else { if (sh.unit) DM_TRINV(true, false, true); else DM_TRINV(true, false, false); }
+    if (sh.ttrans) { if (sh.side_l) DM_TRSM_GO(true, true, true); else DM_TRSM_GO(true, true, false); }
+    else { if (sh.side_l) DM_TRSM_GO(true, false, true); else DM_TRSM_GO(true, false, false); }
   } else {
-    if (sh.ttrans) { if (sh.unit) DM_TRINV(false, true, true); else DM_TRINV(false, true, false); }
-    else { if (sh.unit) DM_TRINV(false, false, true); else DM_TRINV(false, false, false); }
+    if (sh.ttrans) { if (sh.side_l) DM_TRSM_GO(false, true, true); else DM_TRSM_GO(false, true, false); }
+    else { if (sh.side_l) DM_TRSM_GO(false, false, true); else DM_TRSM_GO(false, false, false); }
   }
-#undef DM_TRINV
-  DM_LAUNCH_CHECK("trinv_blocks_kernel");
-  return 0;
-}
-
-namespace {
-template <typename T>
-size_t trsm_smem_bytes(int L) {
-  const int Lp = ((L + TRSM_BS - 1) / TRSM_BS) * TRSM_BS;
-  return sizeof(T) * 4 * (size_t)(Lp + TRSM_BS) * 16;  // per wave: X [Lp][16], bt [32][16]
-}
-template <typename T, bool LO, bool TT, bool SL>
-int trsm_go(const TrsmJob<T>* jobs, int njobs, const TrsmJob<T>& single, long total, long grid,
-            size_t smem, const int* abort, hipStream_t s) {
-  hipLaunchKernelGGL((trsm_kernel<T, LO, TT, SL>), dim3((unsigned)grid), dim3(256), smem, s, jobs,
-                     njobs, single, (int)total, abort);
+#undef DM_TRSM_GO
+#undef DM_TRSM_NB
   DM_LAUNCH_CHECK("trsm_kernel");
   return 0;
 }
-template <typename T, bool LO, bool TT, bool SL>
-int trsm_attr() {
-  DM_HIP(hipFuncSetAttribute((const void*)trsm_kernel<T, LO, TT, SL>,
-                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)trsm_smem_bytes<T>(TRSM_LEAF)));
-  return 0;
-}
-template <typename T>
-int trsm_attr_all() {
-  int rc = 0;
-  rc = rc ? rc : trsm_attr<T, true, true, true>();
-  rc = rc ? rc : trsm_attr<T, true, true, false>();
-  rc = rc ? rc : trsm_attr<T, true, false, true>();
-  rc = rc ? rc : trsm_attr<T, true, false, false>();
-  rc = rc ? rc : trsm_attr<T, false, true, true>();
-  rc = rc ? rc : trsm_attr<T, false, true, false>();
-  rc = rc ? rc : trsm_attr<T, false, false, true>();
-  rc = rc ? rc : trsm_attr<T, false, false, false>();
-  return rc;
-}
-}  // namespace
 
-// Raises the dynamic LDS limit of every trsm kernel (called once at init,
-// outside any stream capture).
-int trsm_init_attributes() {
-  int rc = trsm_attr_all<double>();
-  return rc ? rc : trsm_attr_all<float>();
-}
-
-template <typename T>
-int trsm_launch(const TrsmShape& sh, const TrsmJob<T>* jobs_dev, int njobs,
-                const TrsmJob<T>& single, long total_wg, const int* abort, hipStream_t s,
-                long max_wg) {
-  if (total_wg <= 0) return 0;
-  if (total_wg > 0x7fffffffL) return arg_fail(0, "trsm: too many workgroups");
-  const long grid = (max_wg > 0 && max_wg < total_wg) ? max_wg : total_wg;
-  // LDS is sized for the longest job; batched callers pass the max L in single.L.
-  const size_t smem = trsm_smem_bytes<T>(single.L);
-#define DM_TRSM_GO(LO, TT, SL) \
-  trsm_go<T, LO, TT, SL>(jobs_dev, njobs, single, total_wg, grid, smem, abort, s)
-  if (sh.lower) {
-    if (sh.ttrans) return sh.side_l ? DM_TRSM_GO(true, true, true) : DM_TRSM_GO(true, true, false);
-    return sh.side_l ? DM_TRSM_GO(true, false, true) : DM_TRSM_GO(true, false, false);
-  }
-  if (sh.ttrans) return sh.side_l ? DM_TRSM_GO(false, true, true) : DM_TRSM_GO(false, true, false);
-  return sh.side_l ? DM_TRSM_GO(false, false, true) : DM_TRSM_GO(false, false, false);
-#undef DM_TRSM_GO
-}
-
-// Unbatched solve with the diagonal blocks of each leaf inverted into ws.
+// Unbatched solve, recursive above one leaf.
 template <typename T>
 static int trsm_eff(const TrsmShape& sh, int L, int NV, T alpha, const T* A, int lda, T* B,
-                    int ldb, T* ws, const int* abort, hipStream_t s) {
+                    int ldb, const int* abort, hipStream_t s) {
   if (L <= 0 || NV <= 0) return 0;
-  if (L <= trsm_leaf_len()) {
-    if (!ws) return arg_fail(0, "trsm: no workspace");
-    T* inv = ws;
-    int rc = trinv_blocks_launch<T>(sh, A, lda, L, inv, abort, s);
-    if (rc) return rc;
+  if (L <= TRSM_LEAF) {
     TrsmJob<T> j{};
-    j.A = A; j.B = B; j.inv = inv; j.L = L; j.NV = NV; j.lda = lda; j.ldb = ldb; j.alpha = alpha;
-    return trsm_launch<T>(sh, nullptr, 0, j, trsm_wgs(NV), abort, s);
+    j.A = A; j.B = B; j.L = L; j.NV = NV; j.lda = lda; j.ldb = ldb; j.alpha = alpha;
+    const int nb = trsm_vec_blocks(NV);
+    return trsm_launch<T>(sh, nullptr, 0, j, trsm_wgs(NV, nb), abort, s, nb);
   }
   const TrsmSplit sp = trsm_split(sh, L);
   int rc = trsm_eff<T>(sh, sp.first_n, NV, alpha, tm_sub(sh, A, lda, sp.first_r, sp.first_r), lda,
-                       vsub(sh, B, ldb, sp.first_r), ldb, ws, abort, s);
+                       vsub(sh, B, ldb, sp.first_r), ldb, abort, s);
   if (rc) return rc;
   bool ta, tb;
   const GemmJob<T> g = trsm_update_job<T>(sh, sp, NV, alpha, A, lda, B, ldb, ta, tb);
@@ -347,12 +399,12 @@ static int trsm_eff(const TrsmShape& sh, int L, int NV, T alpha, const T* A, int
                       abort, s);
   if (rc) return rc;
   return trsm_eff<T>(sh, sp.second_n, NV, T(1), tm_sub(sh, A, lda, sp.second_r, sp.second_r), lda,
-                     vsub(sh, B, ldb, sp.second_r), ldb, ws, abort, s);
+                     vsub(sh, B, ldb, sp.second_r), ldb, abort, s);
 }
 
 template <typename T>
 int trsm_full(char side, char uplo, char transa, char diag, int m, int n, T alpha, const T* A,
-              int lda, T* B, int ldb, T* ws, const int* abort, hipStream_t s) {
+              int lda, T* B, int ldb, const int* abort, hipStream_t s) {
   const TrsmShape sh = trsm_shape(side, uplo, transa, diag);
   const int L = sh.side_l ? m : n;
   const int NV = sh.side_l ? n : m;
@@ -361,20 +413,16 @@ int trsm_full(char side, char uplo, char transa, char diag, int m, int n, T alph
     // B := 0 (BLAS: A not referenced)
     return gemm_single<T>(false, false, m, n, 0, T(0), B, ldb, B, ldb, T(0), B, ldb, 0, abort, s);
   }
-  return trsm_eff<T>(sh, L, NV, alpha, A, lda, B, ldb, ws, abort, s);
+  return trsm_eff<T>(sh, L, NV, alpha, A, lda, B, ldb, abort, s);
 }
 
-template int trinv_blocks_launch<double>(const TrsmShape&, const double*, int, int, double*,
-                                         const int*, hipStream_t, int);
-template int trinv_blocks_launch<float>(const TrsmShape&, const float*, int, int, float*,
-                                        const int*, hipStream_t, int);
 template int trsm_launch<double>(const TrsmShape&, const TrsmJob<double>*, int,
                                  const TrsmJob<double>&, long, const int*, hipStream_t, long);
 template int trsm_launch<float>(const TrsmShape&, const TrsmJob<float>*, int,
                                 const TrsmJob<float>&, long, const int*, hipStream_t, long);
 template int trsm_full<double>(char, char, char, char, int, int, double, const double*, int,
-                               double*, int, double*, const int*, hipStream_t);
+                               double*, int, const int*, hipStream_t);
 template int trsm_full<float>(char, char, char, char, int, int, float, const float*, int, float*,
-                              int, float*, const int*, hipStream_t);
+                              int, const int*, hipStream_t);
 
 }  // namespace dm

@@ -17,14 +17,14 @@ inline T* vsub(const TrsmShape& sh, T* B, int ldb, int r) {
   return sh.side_l ? B + r : B + (size_t)r * ldb;
 }
 
-// Split of a solve of length L > trsm_leaf_len() at P (a multiple of TRSM_BS from
-// the top of the triangle): rows [0, P) and [P, L).  Lower triangles solve
+// Split of a solve of length L > TRSM_LEAF at P (a multiple of 32 from the
+// top of the triangle): rows [0, P) and [P, L).  Lower triangles solve
 // [0, P) first, upper ones [P, L) first.
 struct TrsmSplit {
   int first_r, first_n, second_r, second_n;
 };
 inline TrsmSplit trsm_split(const TrsmShape& sh, int L) {
-  const int P = ((L / 2) + TRSM_BS - 1) / TRSM_BS * TRSM_BS;
+  const int P = ((L / 2) + 31) / 32 * 32;
   if (sh.lower) return TrsmSplit{0, P, P, L - P};
   return TrsmSplit{P, L - P, 0, P};
 }

@@ -6,13 +6,6 @@
 
 namespace dm {
 
-int trsm_leaf_len() {
-  // Leaves of 128 rows need half the LDS of 256-row leaves, so two leaf
-  // workgroups share a CU (measured at N = 32768: ldiv! 33.5 ms against
-  // 36.6 ms, cholesky! unchanged).
-  return 128;
-}
-
 TrsmShape trsm_shape(char side, char uplo, char transa, char diag) {
   TrsmShape s;
   s.side_l = is_left(side);
@@ -33,17 +26,19 @@ TrsmShape trsm_shape(char side, char uplo, char transa, char diag) {
 // Batched planning: jobs of equal length L.
 template <typename T>
 static void plan_rec(const TrsmShape& sh, int L, const std::vector<TrsmJob<T>>& jobs,
-                     std::vector<TrsmStep<T>>& steps, int leaf) {
+                     std::vector<TrsmStep<T>>& steps) {
   if (jobs.empty() || L <= 0) return;
-  if (L <= leaf) {
+  if (L <= TRSM_LEAF) {
     TrsmStep<T> st;
     st.leaf = true;
-    st.maxL = L;
+    long vectors = 0;
+    for (const TrsmJob<T>& j : jobs) vectors += j.NV;
+    st.nb = trsm_vec_blocks(vectors);
     long wg = 0;
     for (TrsmJob<T> j : jobs) {
       j.L = L;
       j.wg_begin = (int)wg;
-      wg += trsm_wgs(j.NV);
+      wg += trsm_wgs(j.NV, st.nb);
       st.tjobs.push_back(j);
     }
     st.total_wg = wg;
@@ -58,36 +53,33 @@ static void plan_rec(const TrsmShape& sh, int L, const std::vector<TrsmJob<T>>& 
     TrsmJob<T> a = j;
     a.A = tm_sub(sh, j.A, j.lda, sp.first_r, sp.first_r);
     a.B = vsub(sh, j.B, j.ldb, sp.first_r);
-    a.inv = j.inv + (size_t)(sp.first_r / TRSM_BS) * TRSM_BS * TRSM_BS;
     j1.push_back(a);
     up.gjobs.push_back(trsm_update_job<T>(sh, sp, j.NV, j.alpha, j.A, j.lda, j.B, j.ldb, up.ta,
                                           up.tb));
     TrsmJob<T> c = j;
     c.A = tm_sub(sh, j.A, j.lda, sp.second_r, sp.second_r);
     c.B = vsub(sh, j.B, j.ldb, sp.second_r);
-    c.inv = j.inv + (size_t)(sp.second_r / TRSM_BS) * TRSM_BS * TRSM_BS;
     c.alpha = T(1);
     j2.push_back(c);
   }
-  plan_rec<T>(sh, sp.first_n, j1, steps, leaf);
+  plan_rec<T>(sh, sp.first_n, j1, steps);
   steps.push_back(std::move(up));
-  plan_rec<T>(sh, sp.second_n, j2, steps, leaf);
+  plan_rec<T>(sh, sp.second_n, j2, steps);
 }
 
 template <typename T>
 void trsm_plan_steps(const TrsmShape& sh, const std::vector<TrsmJob<T>>& jobs,
-                     std::vector<TrsmStep<T>>& steps, int leaf) {
-  if (leaf < TRSM_BS || leaf > TRSM_LEAF || leaf % TRSM_BS) leaf = trsm_leaf_len();
+                     std::vector<TrsmStep<T>>& steps) {
   // one recursion per distinct length (a group normally has one)
   std::map<int, std::vector<TrsmJob<T>>> byL;
   for (const TrsmJob<T>& j : jobs)
     if (j.L > 0 && j.NV > 0) byL[j.L].push_back(j);
-  for (auto& kv : byL) plan_rec<T>(sh, kv.first, kv.second, steps, leaf);
+  for (auto& kv : byL) plan_rec<T>(sh, kv.first, kv.second, steps);
 }
 
 template void trsm_plan_steps<double>(const TrsmShape&, const std::vector<TrsmJob<double>>&,
-                                      std::vector<TrsmStep<double>>&, int);
+                                      std::vector<TrsmStep<double>>&);
 template void trsm_plan_steps<float>(const TrsmShape&, const std::vector<TrsmJob<float>>&,
-                                     std::vector<TrsmStep<float>>&, int);
+                                     std::vector<TrsmStep<float>>&);
 
 }  // namespace dm

@@ -88,3 +88,57 @@ def test_potrf_failed_pivot(dm, uplo, n, bad, value):
     got, info = _potrf(dm, A, uplo, np.float64)
     assert info == bad + 1
     assert np.allclose(np.diag(got)[:bad], np.sqrt(np.arange(1.0, bad + 1)), rtol=1e-15, atol=0)
+
+
+def _trsm(dm, dtype, side, uplo, trans, diag, L, nv, alpha, pad):
+    """One tile solve against its residual.  Substitution through inverted
+    16 x 16 blocks is backward stable up to those blocks' condition (below 4
+    here): |T X - alpha B| <= 4 (L + 16) eps |T| |X|."""
+    rng = np.random.default_rng(1000 * L + nv)
+    A = 0.5 * rng.standard_normal((L + pad, L)) / np.sqrt(L)
+    A[np.arange(L), np.arange(L)] = 1.5 + rng.random(L)
+    A = A.astype(dtype)
+    m, n = (L, nv) if side == "L" else (nv, L)
+    B = rng.standard_normal((m + pad, n)).astype(dtype)
+    dA, dB = Dev(dm, A), Dev(dm, B)
+    p = "d" if dtype == np.float64 else "s"
+    a = C.c_double(alpha) if p == "d" else C.c_float(alpha)
+    dm._lib.call(f"dm_{p}trsm", side.encode(), uplo.encode(), trans.encode(), diag.encode(), m, n,
+                 a, dA.p, L + pad, dB.p, m + pad, None)
+    got = dB.get()
+    assert np.array_equal(got[m:], B[m:])
+    T = A[:L].astype(np.float64)
+    T = np.triu(T) if uplo == "U" else np.tril(T)
+    if diag == "U":
+        np.fill_diagonal(T, 1)
+    op = T.T if trans == "T" else T
+    X, R = got[:m].astype(np.float64), alpha * B[:m].astype(np.float64)
+    if side == "R":
+        op, X, R = op.T, X.T, R.T
+    bound = 4 * (L + 16) * np.finfo(dtype).eps * (np.abs(op) @ np.abs(X))
+    assert (np.abs(op @ X - R) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("diag", ["N", "U"])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("side", ["L", "R"])
+def test_trsm_leaf(dm, dtype, side, uplo, trans, diag):
+    """Around the block rows of 16, the 256 rows a wave set covers once and the
+    512 of a leaf; vectors around the 16 a workgroup takes; odd strides."""
+    for L, nv, pad in [(1, 1, 0), (15, 3, 1), (16, 16, 0), (17, 17, 3), (33, 1, 0), (255, 31, 0),
+                       (256, 1, 1), (257, 5, 0), (300, 16, 1), (496, 33, 0), (511, 2, 3),
+                       (512, 48, 0), (513, 7, 0), (1041, 18, 1)]:
+        _trsm(dm, dtype, side, uplo, trans, diag, L, nv, 0.75, pad)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("side", ["L", "R"])
+@pytest.mark.parametrize("nv", [8191, 8192, 8193, 8223])
+def test_trsm_wide(dm, dtype, side, trans, nv):
+    """From 8192 vectors on a workgroup takes two blocks of 16, the last of
+    them partly or wholly past the end."""
+    for L in (16, 48, 290):
+        _trsm(dm, dtype, side, "U", trans, "N", L, nv, -1.0, 1)
