@@ -12,17 +12,19 @@
 //   left half (recursively); its row swaps applied to the right half;
 //   A12 := L11^-1 A12 (unit lower TRSM); A22 -= A21 A12 (GEMM);
 //   right half (recursively); its row swaps applied to the left half,
-// with leaves of 32 columns factored column by column in one workgroup.
-// Row swaps of the other block columns (swaprows_trail!, :239-262) apply
-// the panel's pivots in order p = 1..npiv, one thread per column.
+// with leaves of 32 columns factored in one workgroup, from registers where
+// the rows fit.  Row swaps of the other block columns (swaprows_trail!,
+// :239-262) apply the permutation that the panel's pivots amount to.
 #include <algorithm>
 #include <limits>
+#include <type_traits>
 #include "dm_internal.h"
 
 namespace dm {
 
 constexpr int LU_LEAF = 32;       // columns of a leaf panel
-constexpr int LU_THREADS = 1024;  // the leaf's one workgroup
+constexpr int LU_THREADS = 1024;  // the one workgroup of a leaf in memory
+constexpr int LR_THREADS = 512;   // and of a leaf in registers
 
 // Global row r of a tiled block column starting at tile row 0 of `base`
 // (tiles of mb rows, all `cols` wide, each with ld = its row count).
@@ -48,12 +50,14 @@ __global__ void panel_pack_kernel(T* __restrict__ dst, T* __restrict__ tiles, in
   else dst[i] = *t;
 }
 
-// Factor columns [c0, c0 + nc) of the contiguous panel P (Mp x W, ld = Mp),
-// rows [c0, Mp): for each column j, pick the pivot (maximum |P[r, j]|,
-// r >= j, first on ties) when `pivot`, swap rows j and p within the leaf's
-// columns, scale the column below the diagonal by the pivot's reciprocal
-// (skipped for a zero pivot, which sets *info to j + 1 if unset) and update
-// the rest of the leaf.  piv[j] receives p (0-based, panel rows).
+// A leaf with more rows than registers hold: factor columns [c0, c0 + nc) of
+// the contiguous panel P (Mp x W, ld = Mp), rows [c0, Mp), in memory (32
+// columns of 32000 rows: 5.95 ms in FP64, bound by the passes over the leaf).
+// For each column j, pick the pivot (maximum |P[r, j]|, r >= j, first on ties)
+// when `pivot`, swap rows j and p within the leaf's columns, scale the column
+// below the diagonal by the pivot's reciprocal (skipped for a zero pivot, which
+// sets *info to j + 1 if unset) and update the rest of the leaf.  piv[j]
+// receives p (0-based, panel rows).
 template <typename T>
 __global__ __launch_bounds__(LU_THREADS) void getf2_leaf_kernel(T* __restrict__ P, int64_t Mp,
                                                                 int c0, int nc,
@@ -132,22 +136,317 @@ __global__ __launch_bounds__(LU_THREADS) void getf2_leaf_kernel(T* __restrict__ 
   }
 }
 
-// Row swaps of a contiguous panel: for p in [p0, p1) in order, swap rows p
-// and piv[p] of columns [c0, c1).  One thread per column.
-template <typename T>
-__global__ void laswp_contig_kernel(T* __restrict__ P, int64_t ld, int c0, int c1, int p0, int p1,
-                                    const int* __restrict__ piv, const int* __restrict__ abort) {
-  if (abort && *abort) return;
-  const int c = c0 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (c >= c1) return;
-  T* a = P + (int64_t)c * ld;
-  for (int p = p0; p < p1; ++p) {
-    const int q = piv[p];
-    if (q != p) {
-      const T t = a[p];
-      a[p] = a[q];
-      a[q] = t;
+// Value of lane l (uniform) in every lane.
+template <typename T> __device__ __forceinline__ T wave_bcast(T v, int l) {
+  if (sizeof(T) == 8) {
+    const long long b = __builtin_bit_cast(long long, (double)v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return (T)__builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+  }
+  return (T)__builtin_bit_cast(float,
+                               __builtin_amdgcn_readlane(__builtin_bit_cast(int, (float)v), l));
+}
+
+// Largest of the 64 lanes' values, in every lane (emulated lane by lane on the host).
+template <typename T> __device__ __forceinline__ T wave_max(T v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  auto step = [&](auto ctrl) {
+    T o;
+    if (sizeof(T) == 8) {
+      const long long b = __builtin_bit_cast(long long, (double)v);
+      const int lo = __builtin_amdgcn_update_dpp((int)b, (int)b, ctrl.value, 0xf, 0xf, false);
+      const int hi = __builtin_amdgcn_update_dpp((int)(b >> 32), (int)(b >> 32), ctrl.value, 0xf,
+                                                 0xf, false);
+      o = (T)__builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+    } else {
+      const int b = __builtin_bit_cast(int, (float)v);
+      o = (T)__builtin_bit_cast(
+          float, __builtin_amdgcn_update_dpp(b, b, ctrl.value, 0xf, 0xf, false));
     }
+    v = fmax(v, o);
+  };
+  step(std::integral_constant<int, 0x111>{});  // row_shr 1, 2, 4, 8: lane 15 of each row of 16
+  step(std::integral_constant<int, 0x112>{});
+  step(std::integral_constant<int, 0x114>{});
+  step(std::integral_constant<int, 0x118>{});
+  step(std::integral_constant<int, 0x142>{});  // row_bcast 15, 31: lane 63
+  step(std::integral_constant<int, 0x143>{});
+  return wave_bcast(v, 63);
+#else
+  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl(v, (threadIdx.x & 63) ^ off, 64));
+  return v;
+#endif
+}
+
+// Smallest key of the wave, in every lane; lanes without one hold INT_MAX.
+__device__ __forceinline__ int wave_first(int key) {
+#ifdef __HIP_DEVICE_COMPILE__
+  unsigned long long m = __builtin_amdgcn_ballot_w64(key != std::numeric_limits<int>::max());
+  int best = std::numeric_limits<int>::max();
+  while (m) {  // one lane but for ties
+    best = std::min(best, __builtin_amdgcn_readlane(key, __builtin_ctzll(m)));
+    m &= m - 1;
+  }
+  return best;
+#else
+  for (int off = 32; off > 0; off >>= 1)
+    key = std::min(key, __shfl(key, (threadIdx.x & 63) ^ off, 64));
+  return key;
+#endif
+}
+
+// f(i) for the uniform i in [I, I + N) that equals `at`, by halves.  (The asm
+// keeps the compiler from merging the cases into one that indexes an array of
+// registers by a variable, which would put the array into memory.)
+template <int I, int N, typename F> __device__ __forceinline__ void at_index(int at, F&& f) {
+  if constexpr (N == 1) {
+    f(std::integral_constant<int, I>{});
+#ifdef __HIP_DEVICE_COMPILE__
+    asm volatile("; %0" ::"n"(I));
+#endif
+  } else if (at < I + N / 2) {
+    at_index<I, N / 2>(at, f);
+  } else {
+    at_index<I + N / 2, N - N / 2>(at, f);
+  }
+}
+
+// The same leaf, rows [c0, c0 + 512 R): C columns at a time live in the
+// registers of the one workgroup, thread t holding rows t, t + 512, ... .
+// Every element sees the operations of the kernel above in the same order, so
+// the results are the same bits; the leaf's earlier columns reach a chunk as
+// products (their rows of U first, by wave 0), and the chunk's swaps reach the
+// leaf's other columns at its end, all at once.  A column costs one barrier:
+// each wave offers its largest element with that row of the chunk, the owner
+// of row j offers row j, and then every thread finds the winner by itself.
+//
+// Bound by the chain of a column (maximum, exchange, reciprocal: about 2 us on
+// few rows) and by the products on one CU.  32 columns of 512, 1024, 2048, 4096,
+// 8192 and 16384 rows, FP64: 72, 72, 87, 125, 335 and 1070 us, against 203, 308,
+// 502, 893, 1669 and 3225 for the kernel above (a pass over the leaf in memory
+// per column and three barriers with a single thread between them); FP32: 64,
+// 64, 72, 92, 143 and 296 against 171, 180, 263, 423, 743 and 1412.
+template <typename T, int R, int C>
+__global__ __launch_bounds__(LR_THREADS) void getf2_reg_kernel(T* __restrict__ P, int64_t Mp,
+                                                               int c0, int nc,
+                                                               int* __restrict__ piv,
+                                                               int* __restrict__ info,
+                                                               const int* __restrict__ abort,
+                                                               int pivot) {
+  constexpr int NW = LR_THREADS / 64;
+  __shared__ T candv[2][NW], cand[2][NW][C], rowj[2][C], U[LU_LEAF][C];
+  __shared__ T L11[LU_LEAF][LU_LEAF];
+  __shared__ int candr[2][NW], q[C], tgt[2 * C], src[2 * C];
+  if (abort && *abort) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readlane(tid >> 6, 0);
+  const int64_t ld = Mp;
+  T* const base = P + (int64_t)c0 * ld + c0;  // row 0, column 0 of the leaf
+  const int M = (int)(Mp - c0);
+  T a[R][C];
+  // this thread's rows; those past the end are zeros that no comparison picks
+  // (their products may turn them to NaN) and that are never stored
+  unsigned ro[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) ro[i] = std::min(tid + LR_THREADS * i, M - 1);
+#pragma unroll 1
+  for (int k0 = 0; k0 < nc; k0 += C) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      const T* const col = base + (int64_t)std::min(k0 + c, nc - 1) * ld;
+#pragma unroll
+      for (int i = 0; i < R; ++i) a[i][c] = col[ro[i]];
+    }
+    if (k0 > 0) {
+      for (int e = tid; e < k0 * LU_LEAF; e += LR_THREADS) {
+        const int k = e / LU_LEAF, r = e % LU_LEAF;
+        if (r < k0) L11[k][r] = base[(int64_t)k * ld + r];
+      }
+      T l[2][R];
+      auto load_l = [&](int k, T (&x)[R]) {
+        const T* const col = base + (int64_t)std::min(k, k0 - 1) * ld;
+#pragma unroll
+        for (int i = 0; i < R; ++i) x[i] = col[ro[i]];
+      };
+      if (R <= 4) load_l(0, l[0]);
+      __syncthreads();
+      if (wave == 0) {
+        T lk = L11[0][lane & (LU_LEAF - 1)];
+        for (int k = 0; k < k0; ++k) {
+          const T lv = lk;
+          lk = L11[std::min(k + 1, k0 - 1)][lane & (LU_LEAF - 1)];
+          T u[C];
+#pragma unroll
+          for (int c = 0; c < C; ++c) u[c] = wave_bcast(a[0][c], k);
+          if (lane > k && lane < k0)
+#pragma unroll
+            for (int c = 0; c < C; ++c) a[0][c] -= lv * u[c];
+        }
+        if (lane < k0)
+#pragma unroll
+          for (int c = 0; c < C; ++c) U[lane][c] = a[0][c];
+      }
+      __syncthreads();
+      auto update = [&](int k, const T (&x)[R]) {
+        T u[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) u[c] = U[k][c];
+        if (tid >= k0)
+#pragma unroll
+          for (int c = 0; c < C; ++c) a[0][c] -= x[0] * u[c];
+#pragma unroll
+        for (int i = 1; i < R; ++i)
+#pragma unroll
+          for (int c = 0; c < C; ++c) a[i][c] -= x[i] * u[c];
+      };
+      static_assert(C % 2 == 0, "the earlier columns are taken in pairs");
+      if (R <= 4) {  // registers for a column ahead
+        for (int k = 0; k < k0; k += 2) {
+          load_l(k + 1, l[1]);
+          update(k, l[0]);
+          load_l(k + 2, l[0]);
+          update(k + 1, l[1]);
+        }
+      } else {
+#pragma unroll 1
+        for (int k = 0; k < k0; ++k) {
+          load_l(k, l[0]);
+          update(k, l[0]);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+      if (tid + LR_THREADS * i >= M)
+#pragma unroll
+        for (int c = 0; c < C; ++c) a[i][c] = T(0);
+#pragma unroll
+    for (int jj = 0; jj < C; ++jj) {
+      const int j = k0 + jj, par = jj & 1;
+      if (j >= nc) break;
+      if (pivot) {
+        // the wave's maximum over rows >= j (NaN never wins), then its first row
+        T best = tid >= j ? fmax(T(-1), fabs(a[0][jj])) : T(-1);
+#pragma unroll
+        for (int i = 1; i < R; ++i) best = fmax(best, fabs(a[i][jj]));
+        best = wave_max(best);
+        int br = std::numeric_limits<int>::max();
+#pragma unroll
+        for (int i = R - 1; i > 0; --i)
+          if (fabs(a[i][jj]) == best) br = tid + LR_THREADS * i;
+        if (tid >= j && fabs(a[0][jj]) == best) br = tid;
+        br = wave_first(br);
+        const int bi = __builtin_amdgcn_readlane(br / LR_THREADS, 0);
+        if (tid == (br & (LR_THREADS - 1)))
+          at_index<0, R>(bi, [&](auto i) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) cand[par][wave][c] = a[i.value][c];
+          });
+        if (lane == 0) { candv[par][wave] = best; candr[par][wave] = br; }
+      }
+      if (tid == j)
+#pragma unroll
+        for (int c = 0; c < C; ++c) rowj[par][c] = a[0][c];
+      __syncthreads();
+      int p = j;
+      const T* pr = rowj[par];
+      if (pivot) {
+        T b = candv[par][0];
+        int x = candr[par][0], w = 0;
+#pragma unroll
+        for (int o = 1; o < NW; ++o) {
+          const T v = candv[par][o];
+          const int r = candr[par][o];
+          if (v > b || (v == b && r < x)) { b = v; x = r; w = o; }
+        }
+        if (x < M && x != j) {  // (an all-NaN column keeps its row)
+          p = x;
+          pr = cand[par][w];
+        }
+      }
+      T u[C];
+#pragma unroll
+      for (int c = 0; c < C; ++c) u[c] = pr[c];
+      if (p != j) {
+        const int pi = __builtin_amdgcn_readlane(p / LR_THREADS, 0);
+        if (tid == (p & (LR_THREADS - 1)))
+          at_index<0, R>(pi, [&](auto i) {
+#pragma unroll
+            for (int c = 0; c < C; ++c) a[i.value][c] = rowj[par][c];
+          });
+        if (tid == j)
+#pragma unroll
+          for (int c = 0; c < C; ++c) a[0][c] = u[c];
+      }
+      const T d = u[jj];
+      if (tid == 0) {
+        piv[c0 + j] = c0 + p;
+        q[jj] = p;
+        if (d == T(0) && info && *info == 0) *info = c0 + j + 1;
+      }
+      if (fabs(d) >= std::numeric_limits<T>::min()) {
+        const T inv = T(1) / d;  // LAPACK getf2: scale by the reciprocal
+        if (tid > j) a[0][jj] *= inv;
+#pragma unroll
+        for (int i = 1; i < R; ++i) a[i][jj] *= inv;
+      } else if (d != T(0)) {    // ... or divide when it would overflow
+        if (tid > j) a[0][jj] /= d;
+#pragma unroll
+        for (int i = 1; i < R; ++i) a[i][jj] /= d;
+      }
+      if (tid > j)
+#pragma unroll
+        for (int c = jj + 1; c < C; ++c) a[0][c] -= a[0][jj] * u[c];
+#pragma unroll
+      for (int i = 1; i < R; ++i)
+#pragma unroll
+        for (int c = jj + 1; c < C; ++c) a[i][c] -= a[i][jj] * u[c];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      if (k0 + c >= nc) break;
+      T* const col = base + (int64_t)(k0 + c) * ld;
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        if (tid + LR_THREADS * i < M) col[ro[i]] = a[i][c];
+    }
+    const int cc = std::min(C, nc - k0);
+    if (pivot && nc > cc) {
+      // the chunk's swaps on the leaf's other columns: row tgt[] takes what
+      // row src[] held (rows that stay where they are: -1)
+      __syncthreads();
+      if (tid < C) {
+        int row[2] = {-1, -1}, from[2] = {-1, -1};
+        if (tid < cc) {
+          bool last = q[tid] >= k0 + cc;
+          for (int t = tid + 1; t < cc; ++t) last = last && q[t] != q[tid];
+          row[0] = k0 + tid;
+          from[0] = q[tid];
+          if (last) { row[1] = q[tid]; from[1] = k0 + tid; }
+          // what row `from` held before step tid: trace it back
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            for (int t = tid - 1; t >= 0; --t)
+              if (q[t] == from[e]) from[e] = k0 + t;
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          tgt[2 * tid + e] = row[e] != from[e] ? row[e] : -1;
+          src[2 * tid + e] = from[e];
+        }
+      }
+      __syncthreads();
+      const int e = tid % (2 * C);
+      int c = tid / (2 * C);
+      if (c >= k0) c += cc;
+      const bool moves = c < nc && tgt[e] >= 0;
+      T v = T(0);
+      if (moves) v = base[(int64_t)c * ld + src[e]];
+      __syncthreads();
+      if (moves) base[(int64_t)c * ld + tgt[e]] = v;
+    }
+    __syncthreads();
   }
 }
 
@@ -164,49 +463,160 @@ __global__ void lu_ipiv_kernel(const int* __restrict__ piv, int npiv, int64_t ro
   }
 }
 
-// Row swaps of a tiled block-column region (rows row0.. of the matrix): for
-// p = 0..npiv-1 in order, swap region row p with region row ipiv[p] - 1 -
-// row0.  One thread per column (the order of the swaps is kept per column).
+// Row swaps of a tiled block-column region (a contiguous panel is one with
+// mb = Mr): for p = p0..p1-1 in order, swap rows p and piv[p - p0] - off (an
+// index out of range swaps nothing).
+//
+// The pivots of up to 512 steps are turned into the permutation they amount to
+// and every element moves once: thread t takes the new row p0 + t and, if its
+// step is the last to name a row below the steps' own, that row.  A step
+// names its own row or a later one, so what comes to rest at row p is what
+// row piv[p] held before step p, and before step b a row holds what the last
+// earlier step that names it had as its own row then (a chain of such steps
+// back to a row that none names).  A list with a step that names an earlier
+// row is applied one swap at a time.
+//
+// Bound by the latency of three phases (the lists, the loads, the stores);
+// four columns a workgroup spread the elements over the chip.  512 steps on
+// 512 columns of 4096 rows, FP64: 33 us, against 215 us with one thread a
+// column that made the swaps one after the other; the swaps within a panel
+// 6 against 23 us.
+constexpr int LS_THREADS = 512, LS_COLS = 4;
 template <typename T>
-__global__ void laswp_tiled_kernel(T* __restrict__ base, int64_t Mr, int W, int mb,
-                                   const int* __restrict__ ipiv, int npiv, int64_t row0,
-                                   const int* __restrict__ abort) {
+__global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base, int64_t Mr, int W,
+                                                           int mb, int c0, int c1, int p0, int p1,
+                                                           const int* __restrict__ piv,
+                                                           int64_t off,
+                                                           const int* __restrict__ abort) {
+  __shared__ int q[LS_THREADS], home[LS_THREADS];
+  __shared__ int backward;
   if (abort && *abort) return;
-  const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (c >= W) return;
-  for (int p = 0; p < npiv; ++p) {
-    const int64_t q = (int64_t)ipiv[p] - 1 - row0;
-    if (q != p && q >= 0 && q < Mr) {
-      T* a = tiled_at(base, Mr, mb, W, p, c);
-      T* b = tiled_at(base, Mr, mb, W, q, c);
-      const T t = *a;
-      *a = *b;
-      *b = t;
+  const int t = threadIdx.x;
+  c0 += blockIdx.x * LS_COLS;
+  for (int b0 = p0; b0 < p1; b0 += LS_THREADS) {
+    const int n = std::min(LS_THREADS, p1 - b0), p = b0 + t;
+    int mine = -1;
+    if (t < n) {
+      const int64_t to = (int64_t)piv[p - p0] - off;
+      mine = to >= 0 && to < Mr ? (int)to : p;
     }
+    if (t == 0) backward = 0;
+    q[t] = mine;
+    __syncthreads();
+    if (t < n && mine < p) backward = 1;
+    // the last earlier step that names this step's row, the last earlier one
+    // that names the same row, whether a later one does
+    int own = -1, same = -1;
+    bool later = false;
+#pragma unroll 8
+    for (int i = 0; i < n; ++i) {
+      const int x = q[i];
+      if (i < t && x == p) own = i;
+      if (i < t && x == mine) same = i;
+      if (i > t && x == mine) later = true;
+    }
+    home[t] = own;
+    __syncthreads();
+    if (backward) {
+      if (t < LS_COLS && c0 + t < c1)
+        for (int i = 0; i < n; ++i)
+          if (q[i] != b0 + i) {
+            T* a = tiled_at(base, Mr, mb, W, b0 + i, c0 + t);
+            T* b = tiled_at(base, Mr, mb, W, q[i], c0 + t);
+            const T v = *a;
+            *a = *b;
+            *b = v;
+          }
+      __syncthreads();
+      continue;
+    }
+    int to[2] = {-1, -1}, from[2] = {-1, -1};
+    if (t < n) {
+      to[0] = p;
+      from[0] = mine;
+      for (int i = same; i >= 0; i = home[i]) from[0] = b0 + i;
+      if (mine >= b0 + n && !later) {
+        to[1] = mine;
+        from[1] = p;
+        for (int i = own; i >= 0; i = home[i]) from[1] = b0 + i;
+      }
+    }
+    T v[2][LS_COLS];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      if (to[e] != from[e]) {
+        const int64_t k = from[e] / mb, l = std::min<int64_t>(mb, Mr - k * mb);
+        const T* a = base + k * (int64_t)mb * W + (from[e] - k * mb);
+#pragma unroll
+        for (int c = 0; c < LS_COLS; ++c)
+          if (c0 + c < c1) v[e][c] = a[(c0 + c) * l];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      if (to[e] != from[e]) {
+        const int64_t k = to[e] / mb, l = std::min<int64_t>(mb, Mr - k * mb);
+        T* a = base + k * (int64_t)mb * W + (to[e] - k * mb);
+#pragma unroll
+        for (int c = 0; c < LS_COLS; ++c)
+          if (c0 + c < c1) a[(c0 + c) * l] = v[e][c];
+      }
+    __syncthreads();
   }
 }
 
 namespace {
 unsigned blocks_of(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
+// Columns [c0, c1) of a tiled region or contiguous panel (mb = Mr).
+template <typename T>
+int laswp_launch(T* base, int64_t Mr, int W, int mb, int c0, int c1, int p0, int p1,
+                 const int* piv, int64_t off, const int* abort, hipStream_t s) {
+  hipLaunchKernelGGL((laswp_kernel<T>), dim3(blocks_of(c1 - c0, LS_COLS)), dim3(LS_THREADS), 0, s,
+                     base, Mr, W, mb, c0, c1, p0, p1, piv, off, abort);
+  DM_LAUNCH_CHECK("laswp_kernel");
+  return 0;
+}
+
+// A leaf: C columns of all its rows in at most 128 of a thread's 256 registers,
+// fewer columns for more rows (8 while they fit: each chunk passes over the
+// leaf's earlier columns again); beyond 16384 rows, where a chunk would be one
+// column, it is factored in memory.
+template <typename T, int R, int C>
+int getf2_reg_launch(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, int* abort,
+                     bool pivot, hipStream_t s) {
+  hipLaunchKernelGGL((getf2_reg_kernel<T, R, C>), dim3(1), dim3(LR_THREADS), 0, s, P, Mp, c0, nc,
+                     piv, linfo, abort, pivot ? 1 : 0);
+  DM_LAUNCH_CHECK("getf2_reg_kernel");
+  return 0;
+}
+template <typename T>
+int getf2_leaf(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, int* abort, bool pivot,
+               hipStream_t s) {
+  const int64_t r = (Mp - c0 + LR_THREADS - 1) / LR_THREADS;
+  if (r <= 2) return getf2_reg_launch<T, 2, 8>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
+  if (r <= 4) return getf2_reg_launch<T, 4, 8>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
+  if (r <= 8) return getf2_reg_launch<T, 8, 8>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
+  if (r <= 16) return getf2_reg_launch<T, 16, 4>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
+  if (r <= 32) return getf2_reg_launch<T, 32, 2>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
+  hipLaunchKernelGGL((getf2_leaf_kernel<T>), dim3(1), dim3(LU_THREADS), 0, s, P, Mp, c0, nc, piv,
+                     linfo, abort, pivot ? 1 : 0);
+  DM_LAUNCH_CHECK("getf2_leaf_kernel");
+  return 0;
+}
+
 // getrf2's recursion on columns [c0, c0 + nc) of the contiguous panel.
 template <typename T>
 int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, int* abort,
               bool pivot, hipStream_t s) {
-  if (nc <= LU_LEAF) {
-    hipLaunchKernelGGL((getf2_leaf_kernel<T>), dim3(1), dim3(LU_THREADS), 0, s, P, Mp, c0, nc, piv,
-                       linfo, abort, pivot ? 1 : 0);
-    DM_LAUNCH_CHECK("getf2_leaf_kernel");
-    return 0;
-  }
+  if (nc <= LU_LEAF) return getf2_leaf<T>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
   const int n1 = ((nc / 2 + LU_LEAF - 1) / LU_LEAF) * LU_LEAF, n2 = nc - n1;
   int rc = getrf_rec<T>(P, Mp, c0, n1, piv, linfo, abort, pivot, s);
   if (rc) return rc;
   const int64_t ld = Mp;
   if (pivot) {  // left half's swaps on the right half
-    hipLaunchKernelGGL((laswp_contig_kernel<T>), dim3(blocks_of(n2, 64)), dim3(64), 0, s, P, ld,
-                       c0 + n1, c0 + nc, c0, c0 + n1, piv, abort);
-    DM_LAUNCH_CHECK("laswp_contig_kernel");
+    rc = laswp_launch<T>(P, Mp, 0, (int)Mp, c0 + n1, c0 + nc, c0, c0 + n1, piv + c0, 0, abort, s);
+    if (rc) return rc;
   }
   T* A11 = P + (int64_t)c0 * ld + c0;
   T* A12 = P + (int64_t)(c0 + n1) * ld + c0;
@@ -223,9 +633,9 @@ int getrf_rec(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, int* abort
     rc = getrf_rec<T>(P, Mp, c0 + n1, n2, piv, linfo, abort, pivot, s);
     if (rc) return rc;
     if (pivot) {  // right half's swaps on the left half
-      hipLaunchKernelGGL((laswp_contig_kernel<T>), dim3(blocks_of(n1, 64)), dim3(64), 0, s, P, ld,
-                         c0, c0 + n1, c0 + n1, (int)std::min<int64_t>(c0 + nc, Mp), piv, abort);
-      DM_LAUNCH_CHECK("laswp_contig_kernel");
+      rc = laswp_launch<T>(P, Mp, 0, (int)Mp, c0, c0 + n1, c0 + n1,
+                           (int)std::min<int64_t>(c0 + nc, Mp), piv + c0 + n1, 0, abort, s);
+      if (rc) return rc;
     }
   }
   return 0;
@@ -262,9 +672,8 @@ int getrf_panel(T* tiles, int64_t Mp, int W, int mb, int64_t row0, int* ipiv, in
   if (rc) return rc;
   if (W > npiv) {  // a panel wider than tall: the rest gets the swaps and L11^-1
     if (pivot) {
-      hipLaunchKernelGGL((laswp_contig_kernel<T>), dim3(blocks_of(W - npiv, 64)), dim3(64), 0, s,
-                         P, Mp, npiv, W, 0, npiv, piv, abort);
-      DM_LAUNCH_CHECK("laswp_contig_kernel");
+      rc = laswp_launch<T>(P, Mp, 0, (int)Mp, npiv, W, 0, npiv, piv, 0, abort, s);
+      if (rc) return rc;
     }
     rc = trsm_full<T>('L', 'L', 'N', 'U', npiv, W - npiv, T(1), P, (int)Mp,
                       P + (int64_t)npiv * Mp, (int)Mp, abort, s);
@@ -283,10 +692,7 @@ template <typename T>
 int laswp_tiled(T* base, int64_t Mr, int W, int mb, const int* ipiv, int npiv, int64_t row0,
                 const int* abort, hipStream_t s) {
   if (Mr <= 0 || W <= 0 || npiv <= 0) return 0;
-  hipLaunchKernelGGL((laswp_tiled_kernel<T>), dim3(blocks_of(W, 64)), dim3(64), 0, s, base, Mr, W,
-                     mb, ipiv, npiv, row0, abort);
-  DM_LAUNCH_CHECK("laswp_tiled_kernel");
-  return 0;
+  return laswp_launch<T>(base, Mr, W, mb, 0, W, 0, npiv, ipiv, row0 + 1, abort, s);
 }
 
 template size_t getrf_panel_ws_bytes<double>(int64_t, int);

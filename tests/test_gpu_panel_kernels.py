@@ -142,3 +142,85 @@ def test_trsm_wide(dm, dtype, side, trans, nv):
     them partly or wholly past the end."""
     for L in (16, 48, 290):
         _trsm(dm, dtype, side, "U", trans, "N", L, nv, -1.0, 1)
+
+
+def _getf2(A, pivot):
+    """Column by column, the operations of the panel in their order."""
+    A, piv = A.astype(np.float64).copy(), []
+    for k in range(min(A.shape)):
+        p = k + int(np.argmax(np.abs(A[k:, k]))) if pivot else k
+        piv.append(p + 1)
+        A[[k, p]] = A[[p, k]]
+        if A[k, k] != 0:
+            A[k + 1:, k] /= A[k, k]
+        A[k + 1:, k + 1:] -= np.outer(A[k + 1:, k], A[k, k + 1:])
+    return A, np.array(piv)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("pivot", [True, False])
+@pytest.mark.parametrize("m,n", [(1, 1), (7, 7), (33, 32), (63, 40), (512, 9), (513, 33), (1024, 8),
+                                 (1025, 31), (2048, 17), (2049, 32), (4096, 32), (4097, 7),
+                                 (8193, 5), (16384, 3), (16385, 3), (20, 50)])
+def test_lu_panel(dm, dtype, pivot, m, n):
+    """One tile of m x n around the rows at which a leaf changes its kernel:
+    the pivots exactly, ties (small integers) included, the factors within
+    32 n eps of the growth that partial pivoting (or a dominant diagonal)
+    bounds on these inputs."""
+    rng = np.random.default_rng(m + n)
+    A = rng.integers(-3, 4, (m, n)).astype(dtype) if n <= 9 else rng.standard_normal((m, n))
+    A = (A if pivot else A + 4 * n * np.eye(m, n)).astype(dtype)
+    if n <= 9:
+        A[:, 1:] += rng.standard_normal((m, n - 1)).astype(dtype) / 4  # ties in the first column
+    b = max(m, n)
+    DA = dm.DArray.from_array(A, dm.Blocks(b, b))
+    F = dm.lu_(DA, dm.RowMaximum() if pivot else dm.NoPivot(), check=False, allowsingular=True)
+    want, piv = _getf2(A, pivot)
+    assert np.array_equal(F.ipiv, piv)
+    assert np.abs(DA.collect() - want).max() <= 32 * n * np.finfo(dtype).eps * np.abs(want).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_lu_panel_values(dm, dtype):
+    """Columns of zeros, NaN and infinities, pivots too small to invert."""
+    rng = np.random.default_rng(3)
+    A = rng.standard_normal((600, 12)).astype(dtype)
+    A[:, 5] = 0
+    DA = dm.DArray.from_array(A, dm.Blocks(600, 600))
+    F = dm.lu_(DA, dm.RowMaximum(), check=False, allowsingular=True)
+    want, piv = _getf2(A, True)
+    assert F.info == 6 and np.array_equal(F.ipiv[:5], piv[:5]) and F.ipiv[5] == 6
+    T = np.finfo(dtype)
+    B = np.full((40, 1), T.smallest_subnormal * 4, dtype)  # 1 / pivot overflows
+    B[17] = T.smallest_subnormal * 16
+    DB = dm.DArray.from_array(B, dm.Blocks(40, 40))
+    F = dm.lu_(DB, dm.RowMaximum(), check=False)
+    assert F.ipiv[0] == 18 and np.array_equal(DB.collect()[1:, 0], np.full(39, 0.25, dtype))
+    N = np.full((40, 1), np.nan, dtype)                    # no candidate: the row stays
+    DN = dm.DArray.from_array(N, dm.Blocks(40, 40))
+    assert dm.lu_(DN, dm.RowMaximum(), check=False, allowsingular=True).ipiv[0] == 1
+    N[30], N[35] = -np.inf, np.inf                         # NaN never wins, the first tie does
+    DN = dm.DArray.from_array(N, dm.Blocks(40, 40))
+    assert dm.lu_(DN, dm.RowMaximum(), check=False, allowsingular=True).ipiv[0] == 31
+
+
+@pytest.mark.parametrize("m,n,nb,steps", [(1, 1, 1, 1), (1300, 9, 100, 1300), (600, 5, 64, 37),
+                                          (700, 3, 700, 512), (1025, 6, 256, 513)])
+@pytest.mark.parametrize("kind", ["pivots", "one row", "any"])
+def test_row_swaps(dm, m, n, nb, steps, kind):
+    """The swaps in order, exactly: the rows a pivoted panel names, all steps
+    naming one row, and lists with earlier rows and indices out of range."""
+    rng = np.random.default_rng(m)
+    B = rng.standard_normal((m, n))
+    piv = np.array([rng.integers(p, m) for p in range(steps)]) + 1
+    if kind == "one row":
+        piv[:] = m
+    elif kind == "any":
+        piv = rng.integers(-3, m + 5, steps)
+    D, ip = dm.DArray.from_array(B, dm.Blocks(nb, nb)), Dev(dm, piv.astype(np.int32))
+    t = D.tiled()
+    dm._lib.call("dm_tiled_laswp", C.byref(t), ip.p, steps, None)
+    for p, q in enumerate(piv - 1):
+        if 0 <= q < m:
+            B[[p, q]] = B[[q, p]]
+    assert np.array_equal(D.collect(), B)
