@@ -5,7 +5,7 @@
 // through to its GEMM tasks (src/array/trsm.jl:103-111,157-163).
 //
 // Elements are (re, im) pairs of R (Julia's layout).  Design:
-//  * GEMM/HERK: 64 x 64 tiles of C, 4 waves of 32 x 32, on the real matrix
+//  * GEMM/HERK: tiles of C of 64 x 64 or 32 x 32, 4 waves, on the real matrix
 //    cores (v_mfma_f64_16x16x4f64 / v_mfma_f32_16x16x4f32): each complex
 //    product takes four real ones, re += ar*br - ai*bi, im += ar*bi + ai*br.
 //    op(A) and op(B) are staged into LDS as separate re/im planes with the
@@ -14,58 +14,40 @@
 //    set to zero (BLAS herk semantics).
 //  * POTRF: the recursion n -> (n1, n2) of LAPACK's potrf2 (factor A11;
 //    A12 := A11^-H A12 / A21 := A21 A11^-H; A22 -= herk; factor A22) down to
-//    64 x 64 leaves factored in LDS by one workgroup.
+//    64 x 64 leaves factored in the registers of one workgroup.
 //  * TRSM: the same recursion on the triangle (solve, GEMM update, solve)
-//    down to 64 x 64 leaves, where one thread solves one right-hand-side
-//    vector by substitution against the triangle in LDS.
+//    down to 256 x 256 leaves, where a workgroup solves 16 right-hand-side
+//    vectors by block rows of 16 on the matrix cores.
 // Every kernel returns at once when the abort word is set (a failed pivot),
 // so the rest of a failed factorization becomes a no-op.
 #include "dm_internal.h"
 #include "complex_ops.h"
+#include "potrf_diag.h"
 
 namespace dm {
 
 namespace {
 
-template <typename R> struct Mf;
-// output layout (lane l, item r; 16x16 block D[i][j], j = l%16):
-//   f64 16x16x4: i = 4*r + l/16        f32 16x16x4: i = 4*(l/16) + r
-template <> struct Mf<double> {
-  typedef double v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * r + lk; }
-  static __device__ __forceinline__ v4 mac(double a, double b, v4 c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mf<float> {
-  typedef float v4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ int row(int lk, int r) { return 4 * lk + r; }
-  static __device__ __forceinline__ v4 mac(float a, float b, v4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
+template <typename R> using Mf = PMfma<R>;
 
-constexpr int ZT = 64;        // C tile
-constexpr int ZBK = 8;        // k per step
-constexpr int ZS = ZT + 4;    // LDS row stride of the [k][mn] planes
-constexpr int ZLEAF = 64;     // POTRF / TRSM leaf size
+constexpr int ZLEAF = 64;         // POTRF leaf
+constexpr int ZTB = 16;           // TRSM block row
+constexpr int ZTRSM_LEAF = 256;   // TRSM leaf: one block row per wave of a workgroup
 
-// element (r, c) of op(X) for a column-major X with leading dimension ld:
-// op 0 'N' X[r, c], 1 'T' X[c, r], 2 'C' conj(X[c, r]), 3 conj(X[r, c])
-template <typename R>
-__device__ __forceinline__ void op_elem(const R* __restrict__ X, int64_t ld, int op, int r, int c,
-                                        R& re, R& im) {
-  const int64_t idx = (op == 0 || op == 3) ? (int64_t)c * ld + r : (int64_t)r * ld + c;
-  typedef R v2 __attribute__((ext_vector_type(2)));
-  const v2 v = *gptr((const v2*)(X + 2 * idx));
-  re = v.x;
-  im = (op >= 2) ? -v.y : v.y;
-}
-
-// C = alpha op(A) op(B) + beta C on one 64 x 64 tile per workgroup.
-template <typename R>
+// C = alpha op(A) op(B) + beta C on one ZT x ZT tile per workgroup, k by ZBK
+// steps.  A step's elements are loaded into registers a step ahead and written
+// to LDS as separate re/im planes (the other buffer) after the products.
+//
+// Bound by the matrix cores on tiles of 64 (2048 x 2048 x 256 FP64: 191 us, 262
+// before the loads were taken a step ahead); a launch with too few of those to
+// fill the chip takes tiles of 32 (zgemm_launch; 256 x 256 x 256: 20 us, 74 in
+// tiles of 64 without the prefetch).
+template <typename R, int ZT, int ZBK>
 __global__ __launch_bounds__(256) void zgemm_kernel(ZGemmArgs<R> g, const int* __restrict__ abort) {
   typedef typename Mf<R>::v4 v4;
+  typedef R v2 __attribute__((ext_vector_type(2)));
+  constexpr int ZS = ZT + 4;        // LDS row stride of the [k][mn] planes
+  constexpr int W = ZT / 2, MI = W / 16, NQ = ZT * ZBK / 256;
   __shared__ R As[2][2][ZBK * ZS];  // [buffer][re/im][k * ZS + m]
   __shared__ R Bs[2][2][ZBK * ZS];  // [buffer][re/im][k * ZS + n]
   if (abort && *abort) return;
@@ -75,74 +57,97 @@ __global__ __launch_bounds__(256) void zgemm_kernel(ZGemmArgs<R> g, const int* _
   if (g.tri == 2 && n0 > m0 + ZT - 1) return;  // tile above the lower triangle
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lr = lane & 15, lk = lane >> 4;
-  const int wm0 = (wave & 1) * 32, wn0 = (wave >> 1) * 32;
-  v4 cre[2][2], cim[2][2];
+  const int wm0 = (wave & 1) * W, wn0 = (wave >> 1) * W;
+  v4 cre[MI][MI], cim[MI][MI];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) cre[i][j] = cim[i][j] = v4{0, 0, 0, 0};
+    for (int j = 0; j < MI; ++j) cre[i][j] = cim[i][j] = v4{0, 0, 0, 0};
 
-  // staging: 64 x 8 elements of each operand per step, two per thread.  For
-  // an op that reads X[c, r] (k contiguous in memory) lanes walk k first.
-  auto stage = [&](int buf, int k0) {
+  // this thread's NQ elements of each operand per step: op(A)[m, k] reads
+  // X[k, m] for 'T' and 'C' (k contiguous in memory: lanes walk k first), X[m, k]
+  // else; op(B)[k, n] the other way round.  Rows and columns past the end read
+  // the last ones (their results are dropped), k past the end gives zero.
+  const bool kfa = g.opa == 1 || g.opa == 2, kfb = g.opb == 0 || g.opb == 3;
+  const R sa = g.opa >= 2 ? R(-1) : R(1), sb = g.opb >= 2 ? R(-1) : R(1);
+  int ak[NQ], bk[NQ], as[NQ], bs[NQ];
+  const v2* ap[NQ];
+  const v2* bp[NQ];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int e = tid + 256 * q;
-      const bool kfa = g.opa == 1 || g.opa == 2;
-      const int am = kfa ? e / ZBK : e % ZT, ak = kfa ? e % ZBK : e / ZT;
-      R re = 0, im = 0;
-      if (m0 + am < g.M && k0 + ak < g.K) op_elem(g.A, g.lda, g.opa, m0 + am, k0 + ak, re, im);
-      As[buf][0][ak * ZS + am] = re;
-      As[buf][1][ak * ZS + am] = im;
-      // op(B)[k, n]: 'N' reads B[k, n] (k contiguous)
-      const bool kfb = g.opb == 0 || g.opb == 3;
-      const int bn = kfb ? e / ZBK : e % ZT, bk = kfb ? e % ZBK : e / ZT;
-      re = 0; im = 0;
-      if (n0 + bn < g.N && k0 + bk < g.K) op_elem(g.B, g.ldb, g.opb, k0 + bk, n0 + bn, re, im);
-      Bs[buf][0][bk * ZS + bn] = re;
-      Bs[buf][1][bk * ZS + bn] = im;
+  for (int q = 0; q < NQ; ++q) {
+    const int e = tid + 256 * q;
+    const int am = kfa ? e / ZBK : e % ZT, bn = kfb ? e / ZBK : e % ZT;
+    ak[q] = kfa ? e % ZBK : e / ZT;
+    bk[q] = kfb ? e % ZBK : e / ZT;
+    as[q] = ak[q] * ZS + am;
+    bs[q] = bk[q] * ZS + bn;
+    const int m = min(m0 + am, g.M - 1), n = min(n0 + bn, g.N - 1);
+    ap[q] = (const v2*)g.A + (kfa ? (int64_t)m * g.lda : m);
+    bp[q] = (const v2*)g.B + (kfb ? (int64_t)n * g.ldb : n);
+  }
+  const int64_t astep = kfa ? 1 : g.lda, bstep = kfb ? 1 : g.ldb;
+  v2 av[NQ], bv[NQ];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      av[q] = *gptr(ap[q] + min(k0 + ak[q], g.K - 1) * astep);
+      bv[q] = *gptr(bp[q] + min(k0 + bk[q], g.K - 1) * bstep);
+    }
+  };
+  auto store = [&](int buf, int k0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const bool a = k0 + ak[q] < g.K, b = k0 + bk[q] < g.K;
+      As[buf][0][as[q]] = a ? av[q].x : R(0);
+      As[buf][1][as[q]] = a ? sa * av[q].y : R(0);
+      Bs[buf][0][bs[q]] = b ? bv[q].x : R(0);
+      Bs[buf][1][bs[q]] = b ? sb * bv[q].y : R(0);
     }
   };
   const int nk = (g.K + ZBK - 1) / ZBK;
-  if (nk > 0) stage(0, 0);
+  if (nk > 0) {
+    load(0);
+    store(0, 0);
+  }
   __syncthreads();
   for (int kt = 0; kt < nk; ++kt) {
     const int cur = kt & 1;
-    if (kt + 1 < nk) stage(cur ^ 1, (kt + 1) * ZBK);  // the other buffer: read in step kt-1, ended by its barrier
+    const bool more = kt + 1 < nk;
+    if (more) load((kt + 1) * ZBK);
 #pragma unroll
     for (int kk = 0; kk < ZBK / 4; ++kk) {
       const int k = kk * 4 + lk;
-      R ar[2], ai[2], br[2], bi[2], nbi[2];
+      R ar[MI], ai[MI], br[MI], bi[MI], nbi[MI];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < MI; ++i) {
         ar[i] = As[cur][0][k * ZS + wm0 + i * 16 + lr];
         ai[i] = As[cur][1][k * ZS + wm0 + i * 16 + lr];
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int j = 0; j < MI; ++j) {
         br[j] = Bs[cur][0][k * ZS + wn0 + j * 16 + lr];
         bi[j] = Bs[cur][1][k * ZS + wn0 + j * 16 + lr];
         nbi[j] = -bi[j];
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
+        for (int j = 0; j < MI; ++j) {
           cre[i][j] = Mf<R>::mac(br[j], ar[i], cre[i][j]);
-          cre[i][j] = Mf<R>::mac(nbi[j], ai[i], cre[i][j]);
           cim[i][j] = Mf<R>::mac(bi[j], ar[i], cim[i][j]);
+          cre[i][j] = Mf<R>::mac(nbi[j], ai[i], cre[i][j]);
           cim[i][j] = Mf<R>::mac(br[j], ai[i], cim[i][j]);
         }
     }
+    if (more) store(cur ^ 1, (kt + 1) * ZBK);  // read in step kt-1, ended by its barrier
     __syncthreads();
   }
   // lane holds C[m][n], m = m0 + wm0 + 16i + lr, n = n0 + wn0 + 16j + row(lk, r)
-  typedef R v2 __attribute__((ext_vector_type(2)));
   const bool bz = g.beta_re == R(0) && g.beta_im == R(0);
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < MI; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wm0 + i * 16 + lr, n = n0 + wn0 + j * 16 + Mf<R>::row(lk, r);
@@ -172,126 +177,270 @@ __global__ __launch_bounds__(256) void zgemm_kernel(ZGemmArgs<R> g, const int* _
 // *info is 0) and the abort word to global_base + info_off + j + 1 (the
 // global column, as the real kernels report it), and leaves the block
 // partly factored.
+//
+// Thread (tx, ty) of 16 x 16 holds the elements (ty + 16 i, tx + 16 k) of the
+// upper view (A, or A^T for 'L': both factor as M[x][y] -= conj(M[j][x]) M[j][y])
+// in registers.  A column is one barrier: the owners of row j put it into LDS
+// unscaled, and every thread scales it by the pivot's reciprocal root itself.
+// Bound by that chain.  64 columns: 34 us FP64, against 101 us with the block in
+// LDS (three barriers a column, an integer division per element).
 template <typename R, bool UPPER>
 __global__ __launch_bounds__(256) void zpotrf_leaf_kernel(R* __restrict__ A, int n, int lda,
                                                           int* __restrict__ info, int info_off,
                                                           int* __restrict__ abort,
                                                           int global_base) {
-  __shared__ R t[2][ZLEAF][ZLEAF + 1];  // [re/im][row][col]
-  __shared__ int failed;
-  if (abort && *abort) return;
-  const int tid = threadIdx.x;
   typedef R v2 __attribute__((ext_vector_type(2)));
-  for (int e = tid; e < n * n; e += 256) {
-    const int r = e % n, c = e / n;
-    const v2 v = *gptr((const v2*)(A + 2 * ((int64_t)c * lda + r)));
-    t[0][r][c] = v.x;
-    t[1][r][c] = v.y;
-  }
-  if (tid == 0) failed = 0;
-  __syncthreads();
-  for (int j = 0; j < n; ++j) {
-    if (tid == 0) {
-      const R d = t[0][j][j];
+  constexpr int NB = ZLEAF / 16;
+  __shared__ v2 row[2][ZLEAF];
+  if (abort && *abort) return;
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  v2 m[NB][NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int x = ty + 16 * i, y = tx + 16 * k;
+      const int r = UPPER ? x : y, c = UPPER ? y : x;
+      m[i][k] = v2{x == y ? R(1) : R(0), R(0)};
+      if (x <= y && y < n) m[i][k] = *gptr((const v2*)A + (int64_t)c * lda + r);
+    }
+  bool failed = false;
+#pragma unroll
+  for (int jb = 0; jb < NB; ++jb)
+#pragma unroll 1
+    for (int jj = 0; jj < 16; ++jj) {
+      const int j = 16 * jb + jj;
+      if (failed || j >= n) break;
+      v2* const s = row[j & 1];
+      if (ty == jj)
+#pragma unroll
+        for (int k = jb; k < NB; ++k) s[tx + 16 * k] = m[jb][k];
+      __syncthreads();
+      const R d = s[j].x;
       if (!(d > R(0))) {
-        failed = 1;
-        if (info && *info == 0) *info = info_off + j + 1;
-        if (abort) *abort = global_base + info_off + j + 1;
-      } else {
-        t[0][j][j] = sqrt(d);
-        t[1][j][j] = R(0);
+        if (tid == 0) {
+          if (info && *info == 0) *info = info_off + j + 1;
+          if (abort) *abort = global_base + info_off + j + 1;
+        }
+        failed = true;
+        break;
       }
-    }
-    __syncthreads();
-    if (failed) break;
-    const R d = t[0][j][j];
-    // scale the rest of row j (U) / column j (L)
-    for (int k = j + 1 + tid; k < n; k += 256) {
-      if (UPPER) { t[0][j][k] /= d; t[1][j][k] /= d; }
-      else { t[0][k][j] /= d; t[1][k][j] /= d; }
-    }
-    __syncthreads();
-    // trailing update of the stored triangle
-    const int w = n - j - 1;
-    for (int e = tid; e < w * w; e += 256) {
-      const int a = j + 1 + e % w, b = j + 1 + e / w;  // a row, b column
-      if (UPPER) {
-        if (a > b) continue;
-        // A[a][b] -= conj(U[j][a]) U[j][b]
-        const R ur = t[0][j][a], ui = t[1][j][a], vr = t[0][j][b], vi = t[1][j][b];
-        t[0][a][b] -= ur * vr + ui * vi;
-        t[1][a][b] -= ur * vi - ui * vr;
-      } else {
-        if (a < b) continue;
-        // A[a][b] -= L[a][j] conj(L[b][j])
-        const R lr = t[0][a][j], li = t[1][a][j], mr = t[0][b][j], mi = t[1][b][j];
-        t[0][a][b] -= lr * mr + li * mi;
-        t[1][a][b] -= li * mr - lr * mi;
+      const bool fast = PivotBits<R>::of(d) <= PivotBits<R>::span;
+      const R inv = fast ? inv_sqrt(d) : R(1) / R(sqrt(d));
+      v2 u[NB], v[NB];
+#pragma unroll
+      for (int k = jb; k < NB; ++k) {
+        u[k] = s[ty + 16 * k] * inv;
+        v[k] = s[tx + 16 * k] * inv;
       }
+      if (ty == jj) {
+#pragma unroll
+        for (int k = jb; k < NB; ++k) m[jb][k] = v[k];
+        if (tx == jj) m[jb][jb] = v2{fast ? sqrt_of(d) : R(sqrt(d)), R(0)};
+      }
+#pragma unroll
+      for (int i = jb; i < NB; ++i)
+        if (i > jb || ty > jj)
+#pragma unroll
+          for (int k = i; k < NB; ++k) {
+            m[i][k].x -= u[i].x * v[k].x + u[i].y * v[k].y;
+            m[i][k].y -= u[i].x * v[k].y - u[i].y * v[k].x;
+          }
     }
-    __syncthreads();
-  }
-  __syncthreads();
-  for (int e = tid; e < n * n; e += 256) {
-    const int r = e % n, c = e / n;
-    if (UPPER ? r > c : r < c) continue;
-    *gptr((v2*)(A + 2 * ((int64_t)c * lda + r))) = v2{t[0][r][c], t[1][r][c]};
-  }
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int x = ty + 16 * i, y = tx + 16 * k;
+      const int r = UPPER ? x : y, c = UPPER ? y : x;
+      if (x <= y && y < n) *gptr((v2*)A + (int64_t)c * lda + r) = m[i][k];
+    }
 }
 
-// Solves op(T) x = alpha b for the vectors of B, T an n x n (n <= 64)
-// triangle: one thread per vector, the triangle in LDS.  Vector v's element
-// i is B[v * vstride + i * estride].  op: 0 T, 1 T^T, 2 T^H, 3 conj(T).
+// Solves op(T) x = alpha b for the vectors of B, T an L x L (L <= 256)
+// triangle.  Vector v's element i is B[v * vstride + i * estride].  op: 0 T,
+// 1 T^T, 2 T^H, 3 conj(T).  A workgroup owns 16 vectors and the whole triangle,
+// its wave p block row p of 16; an upper op(T) is solved as the lower triangle
+// that reversing both axes gives.  As in the real kernel, right-hand sides stay
+// in registers, sums in accumulators, the diagonal blocks' inverses W_p in LDS:
+//   X_p = W_p (alpha V_p - sum_{k<p} T_pk X_k),
+// each complex product four real ones, T straight from global memory.
+//
+// Bound by the matrix cores (256 rows are 13 us of products on one CU) and the
+// chain from block to block (two block products and a barrier, about 1 us
+// each).  256 rows, up to 4096 vectors: 40-45 us FP64, against about 700 us for the
+// launches this replaces (four leaves of 64 rows at 145 us, one thread a vector
+// walking the triangle in LDS, and the products between them).
 template <typename R>
-__global__ __launch_bounds__(64) void ztrsm_leaf_kernel(const R* __restrict__ T, int n, int ldt,
-                                                        bool lower, int op, bool unit, R alpha_re,
-                                                        R alpha_im, R* __restrict__ B,
-                                                        int64_t estride, int64_t vstride,
-                                                        int nvec, const int* __restrict__ abort) {
-  __shared__ R t[2][ZLEAF][ZLEAF + 1];  // op(T)[i][k]
-  __shared__ R x[2][ZLEAF][64];         // this workgroup's vectors
-  if (abort && *abort) return;
-  const int tid = threadIdx.x;
-  for (int e = tid; e < n * n; e += 64) {
-    const int i = e % n, k = e / n;
-    R re, im;
-    op_elem(T, ldt, op, i, k, re, im);
-    t[0][i][k] = re;
-    t[1][i][k] = im;
-  }
-  __syncthreads();
-  const int v = blockIdx.x * 64 + tid;
-  if (v >= nvec) return;
+__global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ T, int L, int ldt,
+                                                          bool lower, int op, bool unit,
+                                                          R alpha_re, R alpha_im,
+                                                          R* __restrict__ B, int64_t estride,
+                                                          int64_t vstride, int nvec,
+                                                          const int* __restrict__ abort) {
+  typedef typename Mf<R>::v4 v4;
   typedef R v2 __attribute__((ext_vector_type(2)));
-  R* bv = B + 2 * (int64_t)v * vstride;
-  for (int i = 0; i < n; ++i) {
-    const v2 b = *gptr((const v2*)(bv + 2 * (int64_t)i * estride));
-    x[0][i][tid] = alpha_re * b.x - alpha_im * b.y;
-    x[1][i][tid] = alpha_re * b.y + alpha_im * b.x;
+  constexpr int S = ZTB + 1, D = 2;             // LDS row stride; steps of T in flight
+  __shared__ v2 Wd[ZTRSM_LEAF / ZTB][ZTB * S];  // diagonal blocks, then their inverses
+  __shared__ v2 Xs[2][ZTB * ZTB];               // X_J: [row][vector]
+  if (abort && *abort) return;
+  const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+  const int p = __builtin_amdgcn_readlane((int)threadIdx.x >> 6, 0);
+  const int nblk = (L + ZTB - 1) / ZTB, j0 = blockIdx.x * ZTB;
+  const bool tt = op == 1 || op == 2, lo = tt ? !lower : lower;
+  const R sg = op >= 2 ? R(-1) : R(1);  // conjugation
+  // element (i, k) of the lower triangle: t0[i * rs + k * cs]
+  int64_t rs = tt ? ldt : 1, cs = tt ? 1 : ldt, es = estride;
+  const v2* t0 = (const v2*)T;
+  v2* b0 = (v2*)B;
+  if (!lo) {
+    t0 += (L - 1) * (rs + cs);
+    b0 += (L - 1) * es;
+    rs = -rs;
+    cs = -cs;
+    es = -es;
   }
-  // op(T) is lower for (lower, N / conj) and (upper, T / H)
-  const bool lo = (op == 0 || op == 3) ? lower : !lower;
-  for (int s = 0; s < n; ++s) {
-    const int i = lo ? s : n - 1 - s;
-    R sr = x[0][i][tid], si = x[1][i][tid];
-    const int kb = lo ? 0 : i + 1, ke = lo ? i : n;
-    for (int k = kb; k < ke; ++k) {
-      const R tr = t[0][i][k], ti = t[1][i][k], xr = x[0][k][tid], xi = x[1][k][tid];
-      sr -= tr * xr - ti * xi;
-      si -= tr * xi + ti * xr;
+  // T_pJ as the operand of four k-steps: row 16 p + lr, columns 16 J + 2 lk + tk(s)
+  auto tk = [](int s) { return (s & 1) + 8 * (s >> 1); };
+  const v2* const trow = t0 + min(ZTB * p + lr, L - 1) * rs + 2 * lk * cs;
+  auto load_t = [&](int J, v2 (&t)[4]) {
+    if (J >= p) return;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) t[s] = *gptr(trow + (ZTB * J + tk(s)) * cs);
+  };
+  // ---- the inverse of the diagonal block: its two 8 x 8 triangles by
+  // substitution, a column per lane, then the coupling block -V1 (L21 V0)
+  v2* const W = Wd[p];
+  {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int x = lr, y = 4 * e + lk;  // x along the contiguous axis
+      const int r = tt ? y : x, c = tt ? x : y;
+      const bool in = ZTB * p + r < L && ZTB * p + c < L && r >= c;
+      v2 d = v2{r == c ? R(1) : R(0), R(0)};
+      if (in && !(unit && r == c)) {
+        d = *gptr(t0 + (ZTB * p + r) * rs + (ZTB * p + c) * cs);
+        d.y *= sg;
+      }
+      W[r * S + c] = d;
     }
-    if (!unit) {  // s / d by the textbook complex quotient
-      const R dr = t[0][i][i], di = t[1][i][i];
-      const R den = dr * dr + di * di;
-      const R qr = (sr * dr + si * di) / den, qi = (si * dr - sr * di) / den;
-      sr = qr;
-      si = qi;
+    auto sync = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // a - b c
+    auto sub = [](v2 a, v2 b, v2 c) {
+      a.x -= b.x * c.x;
+      a.x += b.y * c.y;
+      a.y -= b.x * c.y;
+      a.y -= b.y * c.x;
+      return a;
+    };
+    sync();
+    const int o = lr & 8, c = lr & 7, y = (o >> 1) + lk;
+    v2 x[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) x[r] = v2{r == c ? R(1) : R(0), R(0)};
+    // each lane group of 16 forms all columns (the four hold the same)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const v2 d = W[(o + r) * S + o + r];
+      const R den = R(1) / (d.x * d.x + d.y * d.y);
+      const v2 q = v2{d.x * den, -d.y * den}, b = x[r];
+      x[r] = v2{b.x * q.x - b.y * q.y, b.x * q.y + b.y * q.x};
+#pragma unroll
+      for (int i = r + 1; i < 8; ++i) x[i] = sub(x[i], W[(o + i) * S + o + r], x[r]);
     }
-    x[0][i][tid] = sr;
-    x[1][i][tid] = si;
+    sync();
+    if (lk == 0)
+#pragma unroll
+      for (int r = 0; r < 8; ++r) W[(o + r) * S + o + c] = x[r];
+    sync();
+    v2 z = v2{0, 0};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) z = sub(z, W[(8 + y) * S + k], W[k * S + c]);
+    sync();
+    W[y * S + 8 + c] = z;  // -L21 V0, through the upper block
+    sync();
+    z = v2{0, 0};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const v2 a = W[(8 + y) * S + 8 + k];
+      z = sub(z, v2{-a.x, -a.y}, W[k * S + 8 + c]);
+    }
+    sync();
+    W[(8 + y) * S + c] = z;
+    W[y * S + 8 + c] = v2{0, 0};
+    sync();
   }
-  for (int i = 0; i < n; ++i)
-    *gptr((v2*)(bv + 2 * (int64_t)i * estride)) = v2{x[0][i][tid], x[1][i][tid]};
+  // (no load is moved above this point: the registers are needed above)
+  asm volatile("" ::: "memory");
+  v2 t[D][4];
+#pragma unroll
+  for (int u = 0; u < D; ++u) load_t(u, t[u]);
+  // the right-hand side in the accumulator layout
+  v2 v[4];
+  v2* const bvec = b0 + (j0 + lr) * vstride;
+  const bool mine = j0 + lr < nvec;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int i = ZTB * p + Mf<R>::row(lk, r);
+    v[r] = v2{0, 0};
+    if (mine && i < L) v[r] = *gptr((const v2*)bvec + i * es);
+  }
+  // ---- forward substitution
+  v4 ar = v4{0, 0, 0, 0}, ai = v4{0, 0, 0, 0};
+  auto solve = [&] {
+    v4 xr = v4{0, 0, 0, 0}, xi = v4{0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      // the accumulator's item s is the operand of k-step s (same lane)
+      const int k = Mf<R>::row(lk, s);
+      const v2 w = W[lr * S + k];
+      const bool in = ZTB * p + k < L;
+      const R br = in ? alpha_re * v[s].x - alpha_im * v[s].y - ar[s] : R(0);
+      const R bi = in ? alpha_re * v[s].y + alpha_im * v[s].x - ai[s] : R(0);
+      xr = Mf<R>::mac(w.x, br, xr);
+      xi = Mf<R>::mac(w.x, bi, xi);
+      xr = Mf<R>::mac(-w.y, bi, xr);
+      xi = Mf<R>::mac(w.y, br, xi);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = Mf<R>::row(lk, r), i = ZTB * p + k;
+      const v2 x = v2{xr[r], xi[r]};
+      Xs[p & 1][k * ZTB + lr] = x;
+      if (mine && i < L) *gptr(bvec + i * es) = x;
+    }
+  };
+  if (p == 0) solve();
+  __syncthreads();
+  auto step = [&](int J, v2 (&tj)[4]) {
+    if (J < p && J + 1 < nblk) {
+      if (p == J + 1) __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const v2 x = Xs[J & 1][(2 * lk + tk(s)) * ZTB + lr];
+        const R tr = tj[s].x, ti = sg * tj[s].y;
+        ar = Mf<R>::mac(tr, x.x, ar);
+        ai = Mf<R>::mac(tr, x.y, ai);
+        ar = Mf<R>::mac(-ti, x.y, ar);
+        ai = Mf<R>::mac(ti, x.x, ai);
+      }
+      if (p == J + 1) {
+        solve();
+        __builtin_amdgcn_s_setprio(0);
+      }
+      load_t(J + D, tj);
+    }
+    __syncthreads();
+  };
+#pragma unroll 1
+  for (int J = 0; J + 1 < nblk; J += D) {
+#pragma unroll
+    for (int u = 0; u < D; ++u) step(J + u, t[u]);
+  }
 }
 
 int op_code(char t) { return is_notrans(t) ? 0 : (t == 'T' || t == 't') ? 1 : 2; }
@@ -303,9 +452,15 @@ int split_point(int n) { return ((n / 2 + 31) / 32) * 32; }
 template <typename R>
 int zgemm_launch(const ZGemmArgs<R>& g, const int* abort, hipStream_t s) {
   if (g.M <= 0 || g.N <= 0) return 0;
-  const long tiles = (long)((g.M + ZT - 1) / ZT) * ((g.N + ZT - 1) / ZT);
-  if (tiles > 0x7fffffffL) return arg_fail(0, "zgemm: too many tiles");
-  hipLaunchKernelGGL((zgemm_kernel<R>), dim3((unsigned)tiles), dim3(256), 0, s, g, abort);
+  // tiles of 64 once they fill the 256 CUs, else four times as many of 32
+  auto tiles = [&](long t) { return ((g.M + t - 1) / t) * ((g.N + t - 1) / t); };
+  const bool big = tiles(64) >= 256;
+  const long n = tiles(big ? 64 : 32);
+  if (n > 0x7fffffffL) return arg_fail(0, "zgemm: too many tiles");
+  if (big)
+    hipLaunchKernelGGL((zgemm_kernel<R, 64, 8>), dim3((unsigned)n), dim3(256), 0, s, g, abort);
+  else
+    hipLaunchKernelGGL((zgemm_kernel<R, 32, 16>), dim3((unsigned)n), dim3(256), 0, s, g, abort);
   DM_LAUNCH_CHECK("zgemm_kernel");
   return 0;
 }
@@ -329,13 +484,14 @@ template <typename R>
 int ztrsm_rec(bool left, bool lower, int op, bool unit, int L, R ar, R ai, const R* T, int ldt,
               R* B, int ldb, int nv, const int* abort, hipStream_t s) {
   if (L <= 0 || nv <= 0) return 0;
-  if (L <= ZLEAF) {
+  if (L <= ZTRSM_LEAF) {
     // left: vectors are B's columns; right: x op(T) = b as op(T)^T x^T = b^T
     // on B's rows (op N<->T, H<->conj)
     const int lop = left ? op : (op == 0 ? 1 : op == 1 ? 0 : op == 2 ? 3 : 2);
     const int64_t es = left ? 1 : ldb, vs = left ? ldb : 1;
-    hipLaunchKernelGGL((ztrsm_leaf_kernel<R>), dim3((nv + 63) / 64), dim3(64), 0, s, T, L, ldt,
-                       lower, lop, unit, ar, ai, B, es, vs, nv, abort);
+    hipLaunchKernelGGL((ztrsm_leaf_kernel<R>), dim3((nv + ZTB - 1) / ZTB),
+                       dim3(64 * ((L + ZTB - 1) / ZTB)), 0, s, T, L, ldt, lower, lop, unit, ar, ai,
+                       B, es, vs, nv, abort);
     DM_LAUNCH_CHECK("ztrsm_leaf_kernel");
     return 0;
   }

@@ -224,3 +224,94 @@ def test_row_swaps(dm, m, n, nb, steps, kind):
         if 0 <= q < m:
             B[[p, q]] = B[[q, p]]
     assert np.array_equal(D.collect(), B)
+
+
+def _crand(rng, *shape):
+    return rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 129])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -55, 2.0 ** 55])
+def test_complex_potrf_leaf(dm, dtype, uplo, n, scale):
+    """Blocks around the 16 x 16 threads and the leaf of 64; the scaled ones
+    have FP32 pivots outside the range of the fast reciprocal root.  Factor
+    error a few n eps of a well-conditioned matrix."""
+    rng = np.random.default_rng(n)
+    G = _crand(rng, n, n)
+    A = (G @ G.conj().T / n + np.eye(n)).astype(dtype)
+    U = np.linalg.cholesky(A.astype(complex)).conj().T * scale
+    A = (A.astype(complex) * scale * scale).astype(dtype)
+    d, info = Dev(dm, A), dm.DeviceInt(1)
+    p = "z" if dtype == np.complex128 else "c"
+    dm._lib.call(f"dm_{p}potrf", uplo.encode(), n, d.p, n, C.c_void_p(info.ptr), None)
+    got = d.get()
+    assert int(info.get()[0]) == 0
+    F = np.triu(got) if uplo == "U" else np.tril(got).conj().T
+    tol = 2e-13 if dtype == np.complex128 else 1e-4
+    assert np.abs(F - U).max() <= tol * np.abs(U).max()
+    assert not np.diag(got).imag.any()
+    other = (lambda M: np.tril(M, -1)) if uplo == "U" else (lambda M: np.triu(M, 1))
+    assert np.array_equal(other(got), other(A))
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("trans", ["N", "T", "C"])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("side", ["L", "R"])
+def test_complex_trsm_leaf(dm, dtype, side, uplo, trans):
+    """Around the block rows of 16 and the leaf of 256, by the residual:
+    |T X - alpha B| <= 8 (L + 16) eps |T| |X|, as for the real kernel with the
+    two products of each part."""
+    eps = np.finfo(dtype).eps
+    for L, nv, diag in [(1, 1, "N"), (15, 3, "U"), (16, 16, "N"), (17, 17, "N"), (64, 1, "U"),
+                        (65, 33, "N"), (255, 2, "N"), (256, 31, "U"), (257, 16, "N"),
+                        (530, 5, "N")]:
+        rng = np.random.default_rng(L)
+        A = (0.5 * _crand(rng, L + 1, L) / np.sqrt(2 * L)).astype(dtype)
+        A[np.arange(L), np.arange(L)] = 1.5 + rng.random(L) + 0.5j * rng.random(L)
+        m, n = (L, nv) if side == "L" else (nv, L)
+        B = _crand(rng, m + 2, n).astype(dtype)
+        dA, dB = Dev(dm, A), Dev(dm, B)
+        p, R = ("z", np.float64) if dtype == np.complex128 else ("c", np.float32)
+        alpha = np.array([0.75, -0.5], R)
+        dm._lib.call(f"dm_{p}trsm", side.encode(), uplo.encode(), trans.encode(), diag.encode(),
+                     m, n, alpha.ctypes.data_as(C.c_void_p), dA.p, L + 1, dB.p, m + 2, None)
+        got = dB.get()
+        assert np.array_equal(got[m:], B[m:])
+        T = A[:L].astype(complex)
+        T = np.triu(T) if uplo == "U" else np.tril(T)
+        if diag == "U":
+            np.fill_diagonal(T, 1)
+        op = {"N": T, "T": T.T, "C": T.conj().T}[trans]
+        X, rhs = got[:m].astype(complex), (0.75 - 0.5j) * B[:m].astype(complex)
+        if side == "R":
+            op, X, rhs = op.T, X.T, rhs.T
+        bound = 8 * (L + 16) * eps * (np.abs(op) @ np.abs(X))
+        assert (np.abs(op @ X - rhs) <= bound).all(), (L, nv, diag)
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("ta", ["N", "T", "C"])
+@pytest.mark.parametrize("tb", ["N", "T", "C"])
+def test_complex_gemm_tiles(dm, dtype, ta, tb):
+    """Tiles of 32 and (from 256 of them on) of 64, remainders in every
+    direction, by the product's bound 4 (k + 4) eps (|A| |B| + |C|)."""
+    op = {"N": lambda M: M, "T": lambda M: M.T, "C": lambda M: M.conj().T}
+    p, R = ("z", np.float64) if dtype == np.complex128 else ("c", np.float32)
+    for m, n, k in [(1, 1, 1), (33, 31, 17), (64, 70, 0), (1024, 1024, 9), (1023, 1025, 8),
+                    (960, 1024, 16)]:
+        rng = np.random.default_rng(m + n)
+        A = _crand(rng, *((m, k) if ta == "N" else (k, m))).astype(dtype)
+        B = _crand(rng, *((k, n) if tb == "N" else (n, k))).astype(dtype)
+        Cm = _crand(rng, m, n).astype(dtype)
+        dA, dB, dC = Dev(dm, A), Dev(dm, B), Dev(dm, Cm)
+        al, be = np.array([0.75, -0.5], R), np.array([0.5, 0.25], R)
+        dm._lib.call(f"dm_{p}gemm", ta.encode(), tb.encode(), m, n, k,
+                     al.ctypes.data_as(C.c_void_p), dA.p, max(A.shape[0], 1), dB.p,
+                     max(B.shape[0], 1), be.ctypes.data_as(C.c_void_p), dC.p, m, None)
+        a, b, c = op[ta](A.astype(complex)), op[tb](B.astype(complex)), Cm.astype(complex)
+        ref = (0.75 - 0.5j) * (a @ b) + (0.5 + 0.25j) * c
+        bound = 4 * (k + 4) * np.finfo(dtype).eps * (np.abs(a) @ np.abs(b) + np.abs(c))
+        assert (np.abs(dC.get() - ref) <= bound).all(), (m, n, k)
