@@ -315,3 +315,36 @@ def test_complex_gemm_tiles(dm, dtype, ta, tb):
         ref = (0.75 - 0.5j) * (a @ b) + (0.5 + 0.25j) * c
         bound = 4 * (k + 4) * np.finfo(dtype).eps * (np.abs(a) @ np.abs(b) + np.abs(c))
         assert (np.abs(dC.get() - ref) <= bound).all(), (m, n, k)
+
+
+@pytest.mark.parametrize("inc", [1, 3])
+def test_gemv_n(dm, inc):
+    """Around the 32 rows of a workgroup and the 256 columns of one round of
+    loads, by the product's bound 4 (n + 4) eps (|A| |x| + |y|)."""
+    for m, n in [(1, 1), (31, 5), (32, 255), (33, 256), (70, 257), (512, 600), (64, 0)]:
+        rng = np.random.default_rng(m + n)
+        A = rng.standard_normal((m, max(n, 1)))
+        x, y = rng.standard_normal(max(n, 1) * inc), rng.standard_normal(m * inc)
+        dA, dx, dy = Dev(dm, A), Dev(dm, x), Dev(dm, y)
+        dm._lib.call("dm_dgemv", b"N", m, n, 0.5, dA.p, m, dx.p, inc, -2.0, dy.p, inc, None)
+        got, a, v, w = dy.get(), A[:, :n], x[::inc][:n], y[::inc]
+        bound = 4 * (n + 4) * np.finfo(float).eps * (np.abs(a) @ np.abs(v) + 2 * np.abs(w))
+        assert (np.abs(got[::inc] - (0.5 * (a @ v) - 2.0 * w)) <= bound).all(), (m, n)
+        rest = np.arange(len(y)) % inc != 0
+        assert np.array_equal(got[rest], y[rest])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n,nb", [(1, 1), (15, 15), (16, 16), (17, 17), (63, 63), (64, 64), (65, 65),
+                                  (200, 130), (129, 64)])
+def test_inverted_tiles(dm, dtype, uplo, n, nb):
+    """ldiv! through the inverted diagonal tiles around their leaf of 64 and its
+    blocks of 16; the matrix has condition about 5, the error bound is 64 n eps."""
+    A, rng = _spd(n, dtype, n), np.random.default_rng(n)
+    b = rng.standard_normal((n, 3)).astype(dtype)
+    DA = dm.DArray.from_array(A.astype(dtype), dm.Blocks(nb, nb))
+    DB = dm.DArray.from_array(b, dm.Blocks(nb, 3))
+    dm.ldiv_(dm.cholesky_(DA, uplo), DB)
+    want = np.linalg.solve(A, b.astype(np.float64))
+    assert np.abs(DB.collect() - want).max() <= 64 * n * np.finfo(dtype).eps * np.abs(want).max()
