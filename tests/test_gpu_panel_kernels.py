@@ -348,3 +348,43 @@ def test_inverted_tiles(dm, dtype, uplo, n, nb):
     dm.ldiv_(dm.cholesky_(DA, uplo), DB)
     want = np.linalg.solve(A, b.astype(np.float64))
     assert np.abs(DB.collect() - want).max() <= 64 * n * np.finfo(dtype).eps * np.abs(want).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("m,n,k", [(1793, 1800, 17), (1920, 1792, 16), (127, 129, 40), (65, 1, 3)])
+@pytest.mark.parametrize("beta", [0.0, 0.5])
+def test_gemm_ragged_tiles(dm, dtype, m, n, k, beta):
+    """Whole and ragged tiles of 128 and 64 (beta = 0 reads no C), by the
+    product's bound 4 (k + 4) eps (|A| |B| + |C|); rows past C stay."""
+    rng = np.random.default_rng(m + n)
+    A, B = rng.standard_normal((k, m)).astype(dtype), rng.standard_normal((k, n)).astype(dtype)
+    Cm = rng.standard_normal((m + 1, n)).astype(dtype)
+    if beta == 0.0:
+        Cm[:m] = np.nan
+    dA, dB, dC = Dev(dm, A), Dev(dm, B), Dev(dm, Cm)
+    p, real = ("d", C.c_double) if dtype == np.float64 else ("s", C.c_float)
+    dm._lib.call(f"dm_{p}gemm", b"T", b"N", m, n, k, real(-1.5), dA.p, k, dB.p, k, real(beta), dC.p,
+                 m + 1, None)
+    got, a, b = dC.get(), A.astype(np.float64), B.astype(np.float64)
+    c = np.nan_to_num(Cm[:m].astype(np.float64)) * beta
+    bound = 4 * (k + 4) * np.finfo(dtype).eps * (1.5 * np.abs(a.T) @ np.abs(b) + np.abs(c))
+    assert (np.abs(got[:m] - (c - 1.5 * (a.T @ b))) <= bound).all()
+    assert np.array_equal(got[m], Cm[m])
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n", [1, 129, 2433])
+def test_syrk_diagonal_tiles(dm, dtype, uplo, n):
+    """Tiles on the diagonal store their triangle and leave the other alone."""
+    rng, k = np.random.default_rng(n), 19
+    A, Cm = rng.standard_normal((k, n)).astype(dtype), rng.standard_normal((n, n)).astype(dtype)
+    dA, dC = Dev(dm, A), Dev(dm, Cm)
+    p, real = ("d", C.c_double) if dtype == np.float64 else ("s", C.c_float)
+    dm._lib.call(f"dm_{p}syrk", uplo.encode(), b"T", n, k, real(-1.0), dA.p, k, real(1.0), dC.p, n,
+                 None)
+    got, a = dC.get(), A.astype(np.float64)
+    tri = np.triu if uplo == "U" else np.tril
+    bound = 4 * (k + 4) * np.finfo(dtype).eps * (np.abs(a.T) @ np.abs(a) + np.abs(Cm))
+    assert (np.abs(tri(got - (Cm - a.T @ a))) <= bound).all()
+    assert np.array_equal(got - tri(got), Cm - tri(Cm))
