@@ -120,19 +120,20 @@ def _chol(A, uplo, via, options):
     """LinearAlgebra._chol!(A, UpperTriangular/LowerTriangular): returns info."""
     if A.ndim != 2 or A.m != A.n:
         raise ValueError("DimensionMismatch: matrix is not square")
-    # One info pair per matrix: the cached plan/graph is keyed on these
-    # device pointers, so reusing them keeps repeated factorizations on the
-    # captured graph.
+    # One info pair (tile-local, global) per matrix: the cached plan/graph is
+    # keyed on these device pointers, so reusing them keeps repeated
+    # factorizations on the captured graph.  Side by side, because a read
+    # costs about 24 us whatever its size.
     if getattr(A, "_chol_info", None) is None:
-        A._chol_info = (DeviceInt(1), DeviceInt(1))
-    info, ginfo = A._chol_info
+        A._chol_info = DeviceInt(2)
+    info = A._chol_info
 
     def run(Ab):
         if via == "native":
             t = Ab.tiled()
             o = options.c()
             call("dm_cholesky_tiled", uplo.encode(), C.byref(t), C.c_void_p(info.ptr),
-                 C.c_void_p(ginfo.ptr), C.byref(o), None)
+                 C.c_void_p(info.ptr + 4), C.byref(o), None)
             call("dm_stream_sync", None)
         elif via == "datadeps":
             _chol_datadeps(Ab.chunks, uplo, info, options)
@@ -140,9 +141,8 @@ def _chol(A, uplo, via, options):
             raise ValueError(f"unknown via={via!r}")
 
     _maybe_copy_buffered([(A, _square_blocks(A))], run)
-    loc = int(info.get()[0])
-    g = int(ginfo.get()[0]) if via == "native" else 0
-    return loc, g
+    loc, g = (int(v) for v in info.get())
+    return loc, g if via == "native" else 0
 
 
 def ishermitian(A):
@@ -154,11 +154,13 @@ def ishermitian(A):
     sq = _square_blocks(A)
     B = A if A.partitioning == sq else A.reblock(sq)
     mt = B.mt
-    work = DeviceInt(max(mt * (mt + 1) // 2, 1))
-    res = DeviceInt(1)
+    buf = DeviceBuffer(4 * (1 + max(mt * (mt + 1) // 2, 1)))  # the result, then a flag per pair
     t = B.tiled()
-    call("dm_ishermitian_tiled", C.byref(t), C.c_void_p(res.ptr), C.c_void_p(work.ptr), None)
-    ok = bool(res.get()[0])
+    call("dm_ishermitian_tiled", C.byref(t), C.c_void_p(buf.ptr), C.c_void_p(buf.ptr + 4), None)
+    res = np.zeros(1, np.int32)
+    call("dm_memcpy_d2h", res.ctypes.data_as(C.c_void_p), C.c_void_p(buf.ptr), C.c_size_t(4), None)
+    buf.free()
+    ok = bool(res[0])
     if B is not A:
         B.unsafe_free()
     return ok
