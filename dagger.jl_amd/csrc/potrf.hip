@@ -109,7 +109,7 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
       for (int r = 0; r < 4; ++r) {
         const int m = row_of(p, r), c = col_of(q, r);
         old[p][q][r] =
-            work && inside(m, c) ? *gptr(pb_at<T, UPPER>(A, lda, ci + m, cj + c)) : T(0);
+            *gptr(pb_at<T, UPPER>(A, lda, min(ci + m, n - 1), min(cj + c, n - 1)));
       }
   pb_put<T, UPPER>(M, v);
   __syncthreads();

@@ -120,27 +120,41 @@ __device__ __forceinline__ void pb_coord(int q, int& r, int& c) {
   c = UPPER ? b : a;
 }
 
-// v = rows r0.. and columns c0.. of the view, zero from column ncol on
-// (16 loads in flight per thread).
+// v = rows r0.. and columns c0.. of the view, zero from column ncol >= 1 on.
+// The loads carry no condition (past the end they repeat the last column):
+// with a branch around each the compiler waits between them, and the step of
+// the 1024-row FP32 tile took 21.4 us instead of 20.2.
 template <typename T, bool UPPER>
 __device__ __forceinline__ void pb_load(const T* A, int lda, int r0, int c0, int ncol, T (&v)[16]) {
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     int r, c;
     pb_coord<UPPER>(q, r, c);
-    v[q] = c < ncol ? *gptr(pb_at<T, UPPER>(const_cast<T*>(A), lda, r0 + r, c0 + c)) : T(0);
+    v[q] = *gptr(pb_at<T, UPPER>(const_cast<T*>(A), lda, r0 + r, c0 + min(c, ncol - 1)));
+  }
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    int r, c;
+    pb_coord<UPPER>(q, r, c);
+    if (c >= ncol) v[q] = T(0);
   }
 }
 // The upper triangle of the kb x kb diagonal block at j0; the rest of the
 // 64 x 64 block is the identity's (so a narrow block factors like a full one).
+// Loaded whole, for the same reason.
 template <typename T, bool UPPER>
 __device__ __forceinline__ void pb_load_diag(const T* A, int lda, int j0, int kb, T (&v)[16]) {
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     int r, c;
     pb_coord<UPPER>(q, r, c);
-    v[q] = (r <= c && c < kb) ? *gptr(pb_at<T, UPPER>(const_cast<T*>(A), lda, j0 + r, j0 + c))
-                              : (r == c ? T(1) : T(0));
+    v[q] = *gptr(pb_at<T, UPPER>(const_cast<T*>(A), lda, j0 + min(r, kb - 1), j0 + min(c, kb - 1)));
+  }
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    int r, c;
+    pb_coord<UPPER>(q, r, c);
+    if (r > c || c >= kb) v[q] = r == c ? T(1) : T(0);
   }
 }
 template <typename T, bool UPPER>
