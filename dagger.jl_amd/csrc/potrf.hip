@@ -22,8 +22,10 @@
 // columns of a 512 tile (FP64): one launch of 20 us, 8 of them the diagonal
 // block; the panel row and the update as two launches, with the block factored
 // by one lane per column from LDS rows, took 23 + 40 us.
-// Every launch first checks the abort flag (and info), so after a failed
-// pivot the remaining launches are no-ops.
+// After a failed pivot the remaining launches are no-ops.  A workgroup decides
+// that once, for all its waves (potrf_stop), and a launch heeds only failures
+// that earlier launches reported: its own workgroup 0 may report one while
+// others of its workgroups have yet to start.
 #include <type_traits>
 #include "dm_internal.h"
 #include "gemm_tiles.h"
@@ -45,21 +47,36 @@ __device__ __forceinline__ void potrf_block(T* M, int* fail, T* __restrict__ A, 
   }
 }
 
+// Whether a pivot of order at most `upto` in this tile has failed, by the
+// report of potrf_block; with `abort`, also whether one of an earlier tile or an
+// earlier task has (orders up to 0).  For one thread of a workgroup: the words
+// may change while it runs.
+__device__ __forceinline__ bool potrf_stop(const int* info, const int* abort, int global_base,
+                                           int upto) {
+  const int* const p = abort ? abort : info;
+  const int order = p ? *p : 0;
+  return order != 0 && order - (abort ? global_base : 0) <= upto;
+}
+
 template <typename T, bool UPPER>
 __global__ __launch_bounds__(256) void potrf_diag_kernel(T* __restrict__ A, int n, int lda,
                                                          int* __restrict__ info,
                                                          int* __restrict__ abort,
                                                          int global_base) {
   __shared__ T M[PBE];
-  __shared__ int fail;
-  if (abort && *abort) return;
-  if (info && *info) return;
+  __shared__ int fail, stop;
   raise_wave_priority();  // always on the critical path of a factorization
   const int kb = min(PB, n);
   T v[16];
   pb_load_diag<T, UPPER>(A, lda, 0, kb, v);
+  if (threadIdx.x == 0) {
+    stop = (abort && *abort) || (info && *info);
+    // an info word that was set before this call stops its other launches too
+    if (stop && abort && !*abort) *abort = global_base + 1;
+  }
   pb_put<T, UPPER>(M, v);
   __syncthreads();
+  if (stop) return;
   potrf_block<T, UPPER>(M, &fail, A, lda, 0, kb, info, abort, global_base);
 }
 
@@ -75,9 +92,7 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
   __shared__ T Xi_[PBE];
   __shared__ T Xj[PBE];
   __shared__ T Wi[PIE];
-  __shared__ int fail;
-  if (abort && *abort) return;
-  if (info && *info) return;
+  __shared__ int fail, stop;
   raise_wave_priority();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const int t = blockIdx.x;
@@ -111,8 +126,10 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
         old[p][q][r] =
             *gptr(pb_at<T, UPPER>(A, lda, min(ci + m, n - 1), min(cj + c, n - 1)));
       }
+  if (threadIdx.x == 0) stop = potrf_stop(info, abort, global_base, j0 + PB);
   pb_put<T, UPPER>(M, v);
   __syncthreads();
+  if (stop) return;
   pb_inv16<T>(M, Wi);
   pb_put<T, UPPER>(Xj, xj);
   if (two) pb_put<T, UPPER>(Xi_, xi);

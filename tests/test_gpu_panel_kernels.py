@@ -90,6 +90,27 @@ def test_potrf_failed_pivot(dm, uplo, n, bad, value):
     assert np.allclose(np.diag(got)[:bad], np.sqrt(np.arange(1.0, bad + 1)), rtol=1e-15, atol=0)
 
 
+def _leading_factor(dm, uplo, n, bad):
+    """potrf of a dense matrix whose pivot `bad` is negative: the factor of its
+    leading bad x bad minor, and numpy's."""
+    A = _spd(n, np.float64, n)
+    A[bad, bad] = -1.0
+    got, info = _potrf(dm, A, uplo, np.float64)
+    assert info == bad + 1
+    F = (np.triu(got) if uplo == "U" else np.tril(got).T)[:bad, :bad]
+    return F, np.linalg.cholesky(A[:bad, :bad]).T
+
+
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n,bad", [(200, 150), (200, 195), (330, 200), (330, 329)])
+def test_potrf_failed_pivot_earlier_rows(dm, uplo, n, bad):
+    """The panel before the last one that was factored is finished by the
+    launch in which the pivot fails, whichever of its workgroups is first."""
+    F, U = _leading_factor(dm, uplo, n, bad)
+    rows = bad // 64 * 64 - 64
+    assert np.abs(F - U)[:rows].max() <= TOL[np.float64] * np.abs(U).max()
+
+
 def _trsm(dm, dtype, side, uplo, trans, diag, L, nv, alpha, pad):
     """One tile solve against its residual.  Substitution through inverted
     16 x 16 blocks is backward stable up to those blocks' condition (below 4
