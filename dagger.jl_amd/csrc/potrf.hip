@@ -22,10 +22,11 @@
 // columns of a 512 tile (FP64): one launch of 20 us, 8 of them the diagonal
 // block; the panel row and the update as two launches, with the block factored
 // by one lane per column from LDS rows, took 23 + 40 us.
-// After a failed pivot the remaining launches are no-ops.  A workgroup decides
-// that once, for all its waves (potrf_stop), and a launch heeds only failures
-// that earlier launches reported: its own workgroup 0 may report one while
-// others of its workgroups have yet to start.
+// After a failed pivot the remaining launches do nothing but finish the rows
+// before it (the factor of the leading minor is whole, as LAPACK leaves it).  A
+// workgroup decides that once, for all its waves (potrf_stop), by the order of
+// the diagonal block it starts from: its own launch's workgroup 0 may report the
+// next one's failure while others have yet to start.
 #include <type_traits>
 #include "dm_internal.h"
 #include "gemm_tiles.h"
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
         old[p][q][r] =
             *gptr(pb_at<T, UPPER>(A, lda, min(ci + m, n - 1), min(cj + c, n - 1)));
       }
-  if (threadIdx.x == 0) stop = potrf_stop(info, abort, global_base, j0 + PB);
+  if (threadIdx.x == 0) stop = potrf_stop(info, abort, global_base, jp + PB);
   pb_put<T, UPPER>(M, v);
   __syncthreads();
   if (stop) return;

@@ -111,6 +111,16 @@ def test_potrf_failed_pivot_earlier_rows(dm, uplo, n, bad):
     assert np.abs(F - U)[:rows].max() <= TOL[np.float64] * np.abs(U).max()
 
 
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n,bad", [(150, 40), (150, 64), (150, 100), (200, 128), (200, 150),
+                                   (200, 199), (330, 256), (330, 300)])
+def test_potrf_failed_pivot_leading_factor(dm, uplo, n, bad):
+    """The factor of the leading minor before a failed pivot is whole, wherever
+    in the second, third or last panel the pivot fails."""
+    F, U = _leading_factor(dm, uplo, n, bad)
+    assert np.abs(F - U).max() <= TOL[np.float64] * np.abs(U).max()
+
+
 def _trsm(dm, dtype, side, uplo, trans, diag, L, nv, alpha, pad):
     """One tile solve against its residual.  Substitution through inverted
     16 x 16 blocks is backward stable up to those blocks' condition (below 4
