@@ -473,7 +473,7 @@ __global__ __launch_bounds__(256) void bpotrf_row_kernel(T* __restrict__ A,
                                                          int jj, const int* __restrict__ info) {
   __shared__ T M[PBE];
   __shared__ T X[PBE];
-  __shared__ T Wi[PIE];
+  __shared__ T nrec[PB];
   int lo = 0, hi = count - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -489,9 +489,9 @@ __global__ __launch_bounds__(256) void bpotrf_row_kernel(T* __restrict__ A,
   pb_put<T, true>(M, v);
   pb_put<T, true>(X, x);
   __syncthreads();
-  pb_inv16<T>(M, Wi);
+  pb_recip<T>(M, nrec);
   __syncthreads();
-  pb_solve<T>(M, Wi, X, (threadIdx.x >> 6) * 16);
+  pb_solve<T>(M, nrec, X, (threadIdx.x >> 6) * 16);
   __syncthreads();
   pb_store<T, true>(As, s.ld, jj, c0, s.n - c0, X);
 }

@@ -90,9 +90,8 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
                                                          int global_base) {
   typedef typename PMfma<T>::v4 v4;
   __shared__ T M[PBE];
-  __shared__ T Xi_[PBE];
-  __shared__ T Xj[PBE];
-  __shared__ T Wi[PIE];
+  __shared__ T X[2 * PBE];  // column blocks j and i
+  __shared__ T nrec[PB];
   __shared__ int fail, stop;
   raise_wave_priority();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
@@ -131,12 +130,14 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
   pb_put<T, UPPER>(M, v);
   __syncthreads();
   if (stop) return;
-  pb_inv16<T>(M, Wi);
-  pb_put<T, UPPER>(Xj, xj);
-  if (two) pb_put<T, UPPER>(Xi_, xi);
+  pb_recip<T>(M, nrec);
+  const T* const Xj = X;
+  const T* const Xi = two ? X + PBE : X;
+  pb_put<T, UPPER>(X, xj);
+  if (two) pb_put<T, UPPER>(X + PBE, xi);
   __syncthreads();
-  pb_solve<T>(M, Wi, Xj, wave * 16);
-  if (two) pb_solve<T>(M, Wi, Xi_, wave * 16);
+  pb_solve<T>(M, nrec, X, wave * 16);
+  if (two) pb_solve<T>(M, nrec, X + PBE, wave * 16);
   __syncthreads();
   if (finish) {
     pb_store<T, UPPER>(A, lda, jp, cj, n - cj, Xj);
@@ -144,7 +145,6 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
   }
   if (ntile == 1) pb_store<T, UPPER>(A, lda, j0, cj, n - cj, Xj);  // the only reader of this row
   if (work) {
-    const T* Xi = two ? Xi_ : Xj;
     // the 64 products are summed by themselves and subtracted once: rounding
     // at the tile's own magnitude happens once, not at every k-step
     v4 acc[2][2];

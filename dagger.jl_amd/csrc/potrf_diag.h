@@ -3,7 +3,7 @@
 // level-synchronous factorization (batched.hip):
 //   pb_load / pb_store   a 64 x 64 block of the matrix <-> LDS
 //   pb_factor            Cholesky of a block in LDS
-//   pb_inv16             inverses of its four 16 x 16 diagonal blocks
+//   pb_recip             reciprocals of its diagonal, negated
 //   pb_solve             U^-T X for 16 columns of X per wave
 //
 // Blocks are kept as the matrix's upper view: element (r, c) is A[r, c] for
@@ -18,8 +18,6 @@ namespace dm {
 constexpr int PB = 64;        // panel width
 constexpr int PBS = PB + 1;   // LDS row stride of a block
 constexpr int PBE = PB * PBS; // LDS elements of a block
-constexpr int PIS = 17;       // LDS row stride of an inverted 16 x 16 block
-constexpr int PIE = 4 * 16 * PIS + 64;  // LDS elements of pb_inv16's result
 
 template <typename T> struct PMfma;
 // Output layouts (lane l, accumulator item r; 16x16 block D[i][j], j = l%16):
@@ -301,81 +299,151 @@ __device__ __forceinline__ int pb_factor(T* M, int kb, int* fail) {
   return bad;
 }
 
-// W_g = (U_gg)^-T (lower triangular, 16 x 16) of the four diagonal blocks of
-// the factored block in M: W_g(r, c) at Wi[g * 16 * PIS + r * PIS + c].  Wave
-// g inverts block g: its two 8 x 8 diagonal blocks by substitution (one
-// column per lane), then W21 = -V1 (L21 V0).  The caller's barrier follows.
-template <typename T>
-__device__ __forceinline__ void pb_inv16(const T* M, T* Wi) {
-  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const T* Mg = M + (g * 16) * PBS + g * 16;  // U_gg(p, r) = Mg[p * PBS + r] = L(r, p)
-  T* W = Wi + g * 16 * PIS;
-  T* dinv = Wi + 4 * 16 * PIS + g * 16;
-  if (lane < 16) dinv[lane] = T(1) / Mg[lane * PBS + lane];
-  for (int e = lane; e < 256; e += 64) W[(e >> 4) * PIS + (e & 15)] = T(0);
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  const int o = (lane >> 3) * 8, c = lane & 7;
-  if (lane < 16) {
-    T x[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) x[r] = r == c ? T(1) : T(0);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      x[r] *= dinv[o + r];
-#pragma unroll
-      for (int i = r + 1; i < 8; ++i) x[i] -= Mg[(o + r) * PBS + o + i] * x[r];
-    }
-#pragma unroll
-    for (int r = 0; r < 8; ++r) W[(o + r) * PIS + o + c] = x[r];
-  }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  // Z = L21 V0 in W's (otherwise zero) upper right block
-  const int r8 = lane >> 3;
-  T z = T(0);
-#pragma unroll
-  for (int p = 0; p < 8; ++p) z += Mg[p * PBS + 8 + r8] * W[p * PIS + c];
-  W[r8 * PIS + 8 + c] = z;
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  T y = T(0);
-#pragma unroll
-  for (int p = 0; p < 8; ++p) y -= W[(8 + r8) * PIS + 8 + p] * W[p * PIS + 8 + c];
-  __builtin_amdgcn_wave_barrier();  // every lane has read the block
-  W[(8 + r8) * PIS + c] = y;
-  W[r8 * PIS + 8 + c] = T(0);
+// Swaps of 16-lane groups between two registers (emulated lane by lane on the
+// host): the odd groups of a with the even ones of b; groups 2 and 3 of a with
+// groups 0 and 1 of b.
+__device__ __forceinline__ void swap_odd_groups(float& a, float& b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned ra = r[0], rb = r[1];
+  a = __builtin_bit_cast(float, ra);
+  b = __builtin_bit_cast(float, rb);
+#else
+  const int l = threadIdx.x & 63;
+  const bool odd = l & 16;
+  const float x = __shfl(a, l ^ 16, 64), y = __shfl(b, l ^ 16, 64);
+  if (odd) a = y;
+  else b = x;
+#endif
+}
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a),
+                                                  __builtin_bit_cast(unsigned, b), false, false);
+  const unsigned ra = r[0], rb = r[1];
+  a = __builtin_bit_cast(float, ra);
+  b = __builtin_bit_cast(float, rb);
+#else
+  const int l = threadIdx.x & 63;
+  const bool upper = l & 32;
+  const float x = __shfl(a, l ^ 32, 64), y = __shfl(b, l ^ 32, 64);
+  if (upper) a = y;
+  else b = x;
+#endif
+}
+template <void (*SWAP)(float&, float&)>
+__device__ __forceinline__ void swap_words(double& a, double& b) {
+  float x[2], y[2];
+  __builtin_memcpy(x, &a, 8);
+  __builtin_memcpy(y, &b, 8);
+  SWAP(x[0], y[0]);
+  SWAP(x[1], y[1]);
+  __builtin_memcpy(&a, x, 8);
+  __builtin_memcpy(&b, y, 8);
 }
 
-// Columns c0 .. c0+15 of X := U^-T X for the factored block M (with pb_inv16's
-// Wi), by one wave on matrix cores: block row b needs sum_{i<b} U_ib^T X_i and
-// then a product with W_b.  An accumulator of the matrix core holds rows
-// row(lk, r) of a column in item r, and the next product's operand of k-step
-// s is rows row(lk, s): the same lane and item, so the chain of 40 products
-// stays in registers.
+// Four consecutive rows of a block in the accumulator layout, block row s of
+// four: into v, row by row, where a lane can compute with them, and from v to
+// the layout of a product's operand, row k in lane group k.  FP64: the rows are
+// item s of the four groups, so every lane gets all of them and keeps one.
+// FP32: they are the four items of group s; the other groups compute with rows of
+// their own to no end, and a transposition hands out group s's.
+__device__ __forceinline__ void four_rows(const PMfma<double>::v4& x, int s, double (&v)[4]) {
+  v[0] = v[2] = x[s];
+  swap_words<swap_halves>(v[0], v[2]);
+  v[1] = v[0];
+  v[3] = v[2];
+  swap_words<swap_odd_groups>(v[0], v[1]);
+  swap_words<swap_odd_groups>(v[2], v[3]);
+}
+__device__ __forceinline__ void four_rows(const PMfma<float>::v4& x, int, float (&v)[4]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) v[q] = x[q];
+}
+__device__ __forceinline__ double row_by_group(const double (&v)[4], int) {
+  const int k = (threadIdx.x >> 4) & 3;
+  const double a = k & 1 ? v[1] : v[0], b = k & 1 ? v[3] : v[2];
+  return k & 2 ? b : a;
+}
+__device__ __forceinline__ float row_by_group(const float (&v)[4], int s) {
+  float a = v[0], b = v[1], c = v[2], d = v[3];
+  swap_odd_groups(a, b);
+  swap_odd_groups(c, d);
+  if (s & 1) {
+    swap_halves(b, d);
+    return s & 2 ? d : b;
+  }
+  swap_halves(a, c);
+  return s & 2 ? c : a;
+}
+
+// The negative reciprocals of the diagonal of the factored block in M, for
+// pb_solve (a barrier follows).
 template <typename T>
-__device__ __forceinline__ void pb_solve(const T* M, const T* Wi, T* X, int c0) {
+__device__ __forceinline__ void pb_recip(const T* M, T* nrec) {
+  if (threadIdx.x < PB) nrec[threadIdx.x] = T(-1) / M[threadIdx.x * PBS + threadIdx.x];
+}
+
+// Columns c0 .. c0+15 of X := U^-T X for the factored block M (with pb_recip's
+// nrec), by one wave: substitution by four rows at a time on the vector unit and
+// products of depth 4 on the matrix cores for the rows below, in sums of the
+// opposite sign (U^T X - B).
+//
+// Substitution rather than products with inverted diagonal blocks, whose error
+// grows with those blocks' condition: neighbouring rows of a covariance matrix
+// made the factor's error 1e-14 |A| at a condition of 1e12 and a pivot negative
+// at 1e15, where substitution keeps to 3e-16 and succeeds.
+//
+// Bound by the chain of the 16 steps (one product, seven operations, the trips
+// between the layouts).  The order below is the one that the wave issues in:
+// operands a step ahead, and the products that the next step does not need in
+// the gaps of the chain, where they would otherwise hold it up.
+template <typename T>
+__device__ __forceinline__ void pb_solve(const T* M, const T* nrec, T* X, int c0) {
   typedef typename PMfma<T>::v4 v4;
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   v4 x[4];
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) x[b][r] = X[(16 * b + PMfma<T>::row(lk, r)) * PBS + c0 + lr];
+    for (int r = 0; r < 4; ++r) x[b][r] = -X[(16 * b + PMfma<T>::row(lk, r)) * PBS + c0 + lr];
+  // of step t: U_oo of its four rows, their reciprocals, the products' other
+  // operand
+  T u[2][4][4], d[2][4], a[3][4], y = T(0);
+  auto read = [&](int t) {
+    const int o = 4 * t;
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
+    for (int p = 0; p < 4; ++p) {
 #pragma unroll
-    for (int i = 0; i < b; ++i)
+      for (int q = p + 1; q < 4; ++q) u[t & 1][p][q] = M[(o + p) * PBS + o + q];
+      d[t & 1][p] = nrec[o + p];
+      if (16 * p + 15 >= o) a[t % 3][p] = M[(o + lk) * PBS + 16 * p + lr];
+    }
+  };
+  read(0);
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
-        x[b] = PMfma<T>::mac(-M[(16 * i + PMfma<T>::row(lk, s)) * PBS + 16 * b + lr], x[i][s], x[b]);
-    v4 y = v4{0, 0, 0, 0};
+  for (int t = 0; t < 16; ++t) {
+    const int b = t / 4, s = t % 4, o = 4 * t, e = t & 1;
+    // the previous rows' product with block i
+    auto product = [&](int i) {
+      if (t > 0 && i < 4) x[i] = PMfma<T>::mac(a[(t + 2) % 3][i], y, x[i]);
+    };
+    product(b);
+    T v[4];
+    four_rows(x[b], s, v);
 #pragma unroll
-    for (int s = 0; s < 4; ++s)
-      y = PMfma<T>::mac(Wi[b * 16 * PIS + lr * PIS + PMfma<T>::row(lk, s)], x[b][s], y);
-    x[b] = y;
+    for (int q = 0; q < 4; ++q) {
+      __builtin_amdgcn_sched_barrier(0);
+      product(b + 1 + q);
+      if (q == 0 && t < 15) read(t + 1);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) X[(16 * b + PMfma<T>::row(lk, r)) * PBS + c0 + lr] = y[r];
+      for (int p = 0; p < q; ++p) v[q] += u[e][p][q] * v[p];
+      v[q] *= d[e][q];
+    }
+    y = row_by_group(v, s);
+    X[(o + lk) * PBS + c0 + lr] = y;
   }
 }
 

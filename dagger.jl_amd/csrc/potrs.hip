@@ -28,15 +28,14 @@
 namespace dm {
 
 // Inverse of one n x n (n <= 64) triangular block, one workgroup: the block's
-// upper view V (L^T for 'L') in LDS, the inverses of its 16 x 16 diagonal
-// blocks, and V^-T as the solve of the identity's columns, 16 a wave, on the
-// matrix cores.  V^-T is L^-1, and U^-1 its transpose.  Bound by latency
+// upper view V (L^T for 'L') in LDS and V^-T as the solve of the identity's
+// columns, 16 a wave.  V^-T is L^-1, and U^-1 its transpose.  Bound by latency
 // (load, two short chains, store): 7 us, against 60 us with one thread per
 // column substituting against the block in LDS.
 template <typename T, bool UPPER>
 __global__ __launch_bounds__(256) void trtri_leaf_kernel(const TrtriLeaf* __restrict__ leaves,
                                                          const int* __restrict__ abort) {
-  __shared__ T M[PBE], X[PBE], Wi[PIE];
+  __shared__ T M[PBE], X[PBE], nrec[PB];
   if (abort && *abort) return;
   const TrtriLeaf L = leaves[blockIdx.x];
   T v[16];
@@ -49,9 +48,9 @@ __global__ __launch_bounds__(256) void trtri_leaf_kernel(const TrtriLeaf* __rest
     X[r * PBS + c] = r == c ? T(1) : T(0);
   }
   __syncthreads();
-  pb_inv16<T>(M, Wi);
+  pb_recip<T>(M, nrec);
   __syncthreads();
-  pb_solve<T>(M, Wi, X, 16 * wave_id());
+  pb_solve<T>(M, nrec, X, 16 * wave_id());
   __syncthreads();
   const auto dst = gptr((T*)L.dst);
 #pragma unroll

@@ -121,6 +121,30 @@ def test_potrf_failed_pivot_leading_factor(dm, uplo, n, bad):
     assert np.abs(F - U).max() <= TOL[np.float64] * np.abs(U).max()
 
 
+def _smooth(n, nugget):
+    """A covariance matrix of close points: exp(-(x - y)^2 / 0.02) and a nugget
+    on the diagonal.  Its condition is about n / nugget, and most of that lies
+    within any few neighbouring rows."""
+    x = np.linspace(0.0, 1.0, n)
+    return np.exp(-(x[:, None] - x) ** 2 / 0.02) + nugget * np.eye(n)
+
+
+@pytest.mark.parametrize("dtype,nugget", [(np.float64, 1e-6), (np.float64, 1e-13),
+                                          (np.float32, 1e-4)])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n", [65, 256, 300])
+def test_potrf_backward_error(dm, dtype, nugget, uplo, n):
+    """The error of U^T U - A does not grow with A's condition.  An element is
+    a sum of at most n products with partial sums of at most 1, each rounded to
+    u = eps / 2: a random walk of sqrt(n) u."""
+    A = _smooth(n, nugget).astype(dtype)
+    got, info = _potrf(dm, A, uplo, dtype)
+    assert info == 0
+    U = (np.triu(got) if uplo == "U" else np.tril(got).T).astype(np.longdouble)
+    rms = np.sqrt(np.mean((U.T @ U - A) ** 2))
+    assert rms <= np.sqrt(n) * np.finfo(dtype).eps / 2
+
+
 def _trsm(dm, dtype, side, uplo, trans, diag, L, nv, alpha, pad):
     """One tile solve against its residual.  Substitution through inverted
     16 x 16 blocks is backward stable up to those blocks' condition (below 4
