@@ -17,7 +17,8 @@
 //    64 x 64 leaves factored in the registers of one workgroup.
 //  * TRSM: the same recursion on the triangle (solve, GEMM update, solve)
 //    down to 256 x 256 leaves, where a workgroup solves 16 right-hand-side
-//    vectors by block rows of 16 on the matrix cores.
+//    vectors by block rows of 16: substitution within a block row, products on
+//    the matrix cores between them.
 // Every kernel returns at once when the abort word is set (a failed pivot),
 // so the rest of a failed factorization becomes a no-op.
 #include "dm_internal.h"
@@ -257,20 +258,34 @@ __global__ __launch_bounds__(256) void zpotrf_leaf_kernel(R* __restrict__ A, int
     }
 }
 
+// -1 / d, scaled by the larger part: no square over- or underflows.
+template <typename V> __device__ __forceinline__ V neg_recip(V d) {
+  if (fabs(d.x) >= fabs(d.y)) {
+    const auto r = d.y / d.x, n = -1 / (d.x + d.y * r);
+    return V{n, -r * n};
+  }
+  const auto r = d.x / d.y, n = -1 / (d.x * r + d.y);
+  return V{r * n, -n};
+}
+
 // Solves op(T) x = alpha b for the vectors of B, T an L x L (L <= 256)
 // triangle.  Vector v's element i is B[v * vstride + i * estride].  op: 0 T,
 // 1 T^T, 2 T^H, 3 conj(T).  A workgroup owns 16 vectors and the whole triangle,
 // its wave p block row p of 16; an upper op(T) is solved as the lower triangle
 // that reversing both axes gives.  As in the real kernel, right-hand sides stay
-// in registers, sums in accumulators, the diagonal blocks' inverses W_p in LDS:
-//   X_p = W_p (alpha V_p - sum_{k<p} T_pk X_k),
-// each complex product four real ones, T straight from global memory.
+// in registers and sums in accumulators:
+//   T_pp X_p = alpha V_p - sum_{k<p} T_pk X_k,
+// each complex product four real ones, T straight from global memory, the
+// diagonal block from LDS by substitution (see pb_solve: the product with its
+// inverse loses accuracy where it is badly conditioned).
 //
 // Bound by the matrix cores (256 rows are 13 us of products on one CU) and the
 // chain from block to block (two block products and a barrier, about 1 us
-// each).  256 rows, up to 4096 vectors: 40-45 us FP64, against about 700 us for the
-// launches this replaces (four leaves of 64 rows at 145 us, one thread a vector
-// walking the triangle in LDS, and the products between them).
+// each).  256 rows FP64: 16 vectors 45-46 us, 2048 48-49 us, 20000 225-232 us,
+// against 670-700, 680-700 and 1350 us for the launches this replaces (four leaves
+// of 64 rows at 145 us, one thread a vector walking the triangle in LDS, and the
+// products between them).  One step of T in flight in FP64: with two the
+// registers of 16 waves do not hold the substitution's operands (16 vectors 51 us).
 template <typename R>
 __global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ T, int L, int ldt,
                                                           bool lower, int op, bool unit,
@@ -280,8 +295,9 @@ __global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ 
                                                           const int* __restrict__ abort) {
   typedef typename Mf<R>::v4 v4;
   typedef R v2 __attribute__((ext_vector_type(2)));
-  constexpr int S = ZTB + 1, D = 2;             // LDS row stride; steps of T in flight
-  __shared__ v2 Wd[ZTRSM_LEAF / ZTB][ZTB * S];  // diagonal blocks, then their inverses
+  constexpr int S = ZTB + 1, D = sizeof(R) == 4 ? 2 : 1;  // LDS row stride; steps of T in flight
+  __shared__ v2 Td[ZTRSM_LEAF / ZTB][ZTB * S];  // diagonal blocks
+  __shared__ v2 Rd[ZTRSM_LEAF / ZTB][ZTB];      // their diagonals' negative reciprocals
   __shared__ v2 Xs[2][ZTB * ZTB];               // X_J: [row][vector]
   if (abort && *abort) return;
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
@@ -308,74 +324,24 @@ __global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ 
 #pragma unroll
     for (int s = 0; s < 4; ++s) t[s] = *gptr(trow + (ZTB * J + tk(s)) * cs);
   };
-  // ---- the inverse of the diagonal block: its two 8 x 8 triangles by
-  // substitution, a column per lane, then the coupling block -V1 (L21 V0)
-  v2* const W = Wd[p];
-  {
+  // ---- the diagonal block, the identity's past the end, and -1 / T_rr
+  v2* const W = Td[p];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int x = lr, y = 4 * e + lk;  // x along the contiguous axis
-      const int r = tt ? y : x, c = tt ? x : y;
-      const bool in = ZTB * p + r < L && ZTB * p + c < L && r >= c;
-      v2 d = v2{r == c ? R(1) : R(0), R(0)};
-      if (in && !(unit && r == c)) {
-        d = *gptr(t0 + (ZTB * p + r) * rs + (ZTB * p + c) * cs);
-        d.y *= sg;
-      }
-      W[r * S + c] = d;
+  for (int e = 0; e < 4; ++e) {
+    const int x = lr, y = 4 * e + lk;  // x along the contiguous axis
+    const int r = tt ? y : x, c = tt ? x : y;
+    const bool in = ZTB * p + r < L && ZTB * p + c < L && r >= c;
+    v2 d = v2{r == c ? R(1) : R(0), R(0)};
+    if (in && !(unit && r == c)) {
+      d = *gptr(t0 + (ZTB * p + r) * rs + (ZTB * p + c) * cs);
+      d.y *= sg;
     }
-    auto sync = [] {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    // a - b c
-    auto sub = [](v2 a, v2 b, v2 c) {
-      a.x -= b.x * c.x;
-      a.x += b.y * c.y;
-      a.y -= b.x * c.y;
-      a.y -= b.y * c.x;
-      return a;
-    };
-    sync();
-    const int o = lr & 8, c = lr & 7, y = (o >> 1) + lk;
-    v2 x[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) x[r] = v2{r == c ? R(1) : R(0), R(0)};
-    // each lane group of 16 forms all columns (the four hold the same)
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const v2 d = W[(o + r) * S + o + r];
-      const R den = R(1) / (d.x * d.x + d.y * d.y);
-      const v2 q = v2{d.x * den, -d.y * den}, b = x[r];
-      x[r] = v2{b.x * q.x - b.y * q.y, b.x * q.y + b.y * q.x};
-#pragma unroll
-      for (int i = r + 1; i < 8; ++i) x[i] = sub(x[i], W[(o + i) * S + o + r], x[r]);
-    }
-    sync();
-    if (lk == 0)
-#pragma unroll
-      for (int r = 0; r < 8; ++r) W[(o + r) * S + o + c] = x[r];
-    sync();
-    v2 z = v2{0, 0};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) z = sub(z, W[(8 + y) * S + k], W[k * S + c]);
-    sync();
-    W[y * S + 8 + c] = z;  // -L21 V0, through the upper block
-    sync();
-    z = v2{0, 0};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const v2 a = W[(8 + y) * S + 8 + k];
-      z = sub(z, v2{-a.x, -a.y}, W[k * S + 8 + c]);
-    }
-    sync();
-    W[(8 + y) * S + c] = z;
-    W[y * S + 8 + c] = v2{0, 0};
-    sync();
+    W[r * S + c] = d;
+    if (r == c) Rd[p][r] = neg_recip(d);
   }
-  // (no load is moved above this point: the registers are needed above)
-  asm volatile("" ::: "memory");
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   v2 t[D][4];
 #pragma unroll
   for (int u = 0; u < D; ++u) load_t(u, t[u]);
@@ -391,34 +357,74 @@ __global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ 
   }
   // ---- forward substitution
   v4 ar = v4{0, 0, 0, 0}, ai = v4{0, 0, 0, 0};
+  // X_p from the sums: four rows at a time by substitution, a product of depth 4
+  // for the rows below, in sums of the opposite sign (as pb_solve).  The operands
+  // of a step are read while the matrix cores are at the one before.
+  v2 u[4][4], q[4];
+  auto read = [&](int s) {
+    const int o = 4 * s;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int k = 0; k < i; ++k) u[i][k] = W[(o + i) * S + o + k];
+      q[i] = Rd[p][o + i];
+    }
+  };
   auto solve = [&] {
-    v4 xr = v4{0, 0, 0, 0}, xi = v4{0, 0, 0, 0};
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      // the accumulator's item s is the operand of k-step s (same lane)
-      const int k = Mf<R>::row(lk, s);
-      const v2 w = W[lr * S + k];
-      const bool in = ZTB * p + k < L;
-      const R br = in ? alpha_re * v[s].x - alpha_im * v[s].y - ar[s] : R(0);
-      const R bi = in ? alpha_re * v[s].y + alpha_im * v[s].x - ai[s] : R(0);
-      xr = Mf<R>::mac(w.x, br, xr);
-      xi = Mf<R>::mac(w.x, bi, xi);
-      xr = Mf<R>::mac(-w.y, bi, xr);
-      xi = Mf<R>::mac(w.y, br, xi);
+      const bool in = ZTB * p + Mf<R>::row(lk, s) < L;
+      ar[s] = in ? ar[s] - (alpha_re * v[s].x - alpha_im * v[s].y) : R(0);
+      ai[s] = in ? ai[s] - (alpha_re * v[s].y + alpha_im * v[s].x) : R(0);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = Mf<R>::row(lk, r), i = ZTB * p + k;
-      const v2 x = v2{xr[r], xi[r]};
-      Xs[p & 1][k * ZTB + lr] = x;
+    for (int s = 0; s < 4; ++s) {
+      const int o = 4 * s;
+      R xr[4], xi[4];
+      four_rows(ar, s, xr);
+      four_rows(ai, s, xi);
+      const v2 a = W[lr * S + o + lk];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int k = 0; k < i; ++k) {
+          const v2 d = u[i][k];
+          xr[i] += d.x * xr[k];
+          xi[i] += d.x * xi[k];
+          xr[i] -= d.y * xi[k];
+          xi[i] += d.y * xr[k];
+        }
+        const v2 d = q[i];
+        const R w = xr[i];
+        xr[i] = w * d.x - xi[i] * d.y;
+        xi[i] = w * d.y + xi[i] * d.x;
+      }
+      const v2 x = v2{row_by_group(xr, s), row_by_group(xi, s)};
+      if (s < 3) {
+        ar = Mf<R>::mac(a.x, x.x, ar);
+        ai = Mf<R>::mac(a.x, x.y, ai);
+        ar = Mf<R>::mac(-a.y, x.y, ar);
+        __builtin_amdgcn_sched_barrier(0);
+        read(s + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        ai = Mf<R>::mac(a.y, x.x, ai);
+      }
+      const int i = ZTB * p + o + lk;
+      Xs[p & 1][(o + lk) * ZTB + lr] = x;
       if (mine && i < L) *gptr(bvec + i * es) = x;
     }
   };
-  if (p == 0) solve();
+  if (p == 0) {
+    read(0);
+    solve();
+  }
   __syncthreads();
   auto step = [&](int J, v2 (&tj)[4]) {
     if (J < p && J + 1 < nblk) {
-      if (p == J + 1) __builtin_amdgcn_s_setprio(3);
+      if (p == J + 1) {
+        __builtin_amdgcn_s_setprio(3);
+        read(0);
+      }
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const v2 x = Xs[J & 1][(2 * lk + tk(s)) * ZTB + lr];

@@ -311,6 +311,27 @@ def test_complex_potrf_leaf(dm, dtype, uplo, n, scale):
     assert np.array_equal(other(got), other(A))
 
 
+@pytest.mark.parametrize("dtype,nugget", [(np.complex128, 1e-6), (np.complex128, 1e-13),
+                                          (np.complex64, 1e-4)])
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("n", [129, 256, 300])
+def test_complex_potrf_backward_error(dm, dtype, nugget, uplo, n):
+    """As the real test, with the rows turned in the complex plane: each part
+    of an element is a sum of at most 2 n products, both parts sqrt(2) of that."""
+    w = np.exp(2j * np.pi * np.random.default_rng(n).random(n))
+    A = (w[:, None] * _smooth(n, nugget) * w.conj()).astype(dtype)
+    A[np.arange(n), np.arange(n)] = A[np.arange(n), np.arange(n)].real
+    d, info = Dev(dm, A), dm.DeviceInt(1)
+    p = "z" if dtype == np.complex128 else "c"
+    dm._lib.call(f"dm_{p}potrf", uplo.encode(), n, d.p, n, C.c_void_p(info.ptr), None)
+    assert int(info.get()[0]) == 0
+    got = d.get()
+    U = (np.triu(got) if uplo == "U" else np.tril(got).conj().T).astype(np.clongdouble)
+    E = np.triu(U.conj().T @ U - (A if uplo == "U" else A.conj().T))
+    rms = np.sqrt(2 * np.mean(np.abs(E) ** 2))
+    assert rms <= 2 * np.sqrt(n) * np.finfo(dtype).eps / 2
+
+
 @pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
 @pytest.mark.parametrize("trans", ["N", "T", "C"])
 @pytest.mark.parametrize("uplo", ["U", "L"])
