@@ -97,13 +97,13 @@ __device__ __forceinline__ void trsm_wave_sync() {
 template <typename T, bool LOWER, bool TTRANS, bool SIDE_L, int NB>
 __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restrict__ jobs,
                                                        int njobs, TrsmJob<T> single, int unit,
-                                                       const int* __restrict__ abort) {
+                                                       int prio, const int* __restrict__ abort) {
   typedef typename MfmaT<T>::v4 v4;
   constexpr int TD = trsm_depth<T, NB>();
   __shared__ T Wd[TRSM_LEAF / TB][TB * TIS];   // diagonal blocks, then their inverses
   __shared__ T Xs[2][TB * TB * NB];            // X_J: [k][vector]
   if (abort && *abort) return;
-  if (single.prio) raise_wave_priority();
+  if (prio) raise_wave_priority();
   TrsmJob<T> job;
   int local = blockIdx.x;
   if (njobs == 0) {
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restr
         __builtin_amdgcn_s_setprio(3);
         update(q);
         solve(J + 1, vals[q], acc[q]);
-        __builtin_amdgcn_s_setprio(0);
+        if (!prio) __builtin_amdgcn_s_setprio(0);  // back to the launch's own
       }
 #pragma unroll
     for (int q = 0; q < TQ; ++q) {
@@ -359,7 +359,7 @@ int trsm_launch(const TrsmShape& sh, const TrsmJob<T>* jobs_dev, int njobs,
   if (total_wg > 0x7fffffffL) return arg_fail(0, "trsm: too many workgroups");
 #define DM_TRSM_NB(LO, TT, SL, N)                                                            \
   hipLaunchKernelGGL((trsm_kernel<T, LO, TT, SL, N>), dim3((unsigned)total_wg), dim3(64 * TW), \
-                     0, s, jobs_dev, njobs, single, sh.unit ? 1 : 0, abort)
+                     0, s, jobs_dev, njobs, single, sh.unit ? 1 : 0, single.prio, abort)
 #define DM_TRSM_GO(LO, TT, SL)              \
   do {                                      \
     if (nb == 2) DM_TRSM_NB(LO, TT, SL, 2); \

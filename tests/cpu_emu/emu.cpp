@@ -34,6 +34,8 @@ struct Fiber {
   int linear = 0;
   State st = RUNNABLE;
   char* stack = nullptr;
+  bool synced = false;          // has passed a barrier or wave op
+  int given = -1, prio = 0;     // wave priority set before that, and now
 };
 
 constexpr size_t kStack = 256 * 1024;
@@ -88,6 +90,7 @@ void trampoline() {
 #endif
   (*r->body)();
   Fiber& me = r->f[r->cur];
+  if (me.given >= 0 && me.prio != me.given) die("a wave ends below the priority it was given");
   me.st = DONE;
   --r->live;
   // a barrier may now be complete for the remaining work-items
@@ -109,6 +112,9 @@ void run_block(Run& r) {
     f.linear = i;
     f.tid = dim3(i % r.bdim.x, (i / r.bdim.x) % r.bdim.y, i / (r.bdim.x * r.bdim.y));
     f.st = RUNNABLE;
+    f.synced = false;
+    f.given = -1;
+    f.prio = 0;
     f.stack = r.stacks[i];
     getcontext(&f.uc);
     f.uc.uc_stack.ss_sp = f.stack;
@@ -163,9 +169,16 @@ unsigned char* dynamic_shared() {
   return g_run->dyn;
 }
 
+void setprio(int p) {
+  Fiber& me = self();
+  if (!me.synced) me.given = p;
+  me.prio = p;
+}
+
 void syncthreads() {
   Run* r = g_run;
   Fiber& me = self();
+  me.synced = true;
   me.st = AT_BARRIER;
   if (++r->at_barrier == r->live) {
     for (Fiber& o : r->f)
@@ -180,6 +193,7 @@ void syncthreads() {
 void wave_exchange(const void* in, size_t bytes, void* all) {
   Run* r = g_run;
   Fiber& me = self();
+  me.synced = true;
   if (bytes > 64) die("wave op operand too large");
   const int wv = me.linear / 64, lane = me.linear % 64;
   if ((wv + 1) * 64 > r->n) die("wave op in a partial wavefront");

@@ -109,6 +109,7 @@ const dim3& block_idx();
 const dim3& block_dim();
 const dim3& grid_dim();
 void syncthreads();
+void setprio(int p);
 // Wave-wide exchange: every lane of the current wavefront contributes
 // `bytes` from `in`; on return `all` holds the 64 contributions (lane order).
 void wave_exchange(const void* in, size_t bytes, void* all);
@@ -170,7 +171,9 @@ inline int readlane(int v, int l) {
 #define __builtin_amdgcn_wave_barrier() ::emu::wave_exchange(nullptr, 0, nullptr)
 #define __builtin_amdgcn_fence(order, scope) ((void)0)
 #define __builtin_amdgcn_sched_barrier(mask) ((void)0)
-#define __builtin_amdgcn_s_setprio(p) ((void)0)
+// A priority that a kernel sets at its start, before any barrier or wave op, is
+// the launch's own: a wave that ends with another aborts.
+#define __builtin_amdgcn_s_setprio(p) ::emu::setprio(p)
 #define DM_GLOBAL_AS  /* host memory: no device address spaces */
 #define __builtin_amdgcn_readlane(v, l) ::emu::readlane((v), (l))
 #define hipLaunchKernelGGL(K, G, B, SH, ST, ...) \
