@@ -205,7 +205,8 @@ __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restr
     for (int r = 0; r < 8; ++r) x[r] = r == c ? T(1) : T(0);
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      x[r] *= __shfl(dinv, (lane & 56) + r, 64);
+      const T d = __shfl(dinv, (lane & 56) + r, 64);
+      x[r] = r < c ? T(0) : x[r] * d;  // zero above the diagonal, also for d infinite
 #pragma unroll
       for (int i = r + 1; i < 8; ++i) x[i] -= W[(o + i) * TIS + o + r] * x[r];
     }

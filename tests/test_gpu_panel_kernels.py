@@ -188,6 +188,23 @@ def test_trsm_leaf(dm, dtype, side, uplo, trans, diag):
         _trsm(dm, dtype, side, uplo, trans, diag, L, nv, 0.75, pad)
 
 
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("trans", ["N", "T"])
+@pytest.mark.parametrize("L", [1, 8, 40])
+def test_trsm_zero_diagonal(dm, uplo, trans, L):
+    """A zero in the first row that is solved makes that row infinite, with the
+    right-hand side's sign, not NaN."""
+    T = np.eye(L) * 2.0
+    first = 0 if (uplo == "L") == (trans == "N") else L - 1
+    T[first, first] = 0.0
+    B = np.ones((L, 3))
+    B[:, 1] = -1.0
+    dA, dB = Dev(dm, T), Dev(dm, B)
+    dm._lib.call("dm_dtrsm", b"L", uplo.encode(), trans.encode(), b"N", L, 3, 1.0, dA.p, L, dB.p, L,
+                 None)
+    assert np.array_equal(dB.get()[first], np.array([np.inf, -np.inf, np.inf]))
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("trans", ["N", "T"])
 @pytest.mark.parametrize("side", ["L", "R"])
