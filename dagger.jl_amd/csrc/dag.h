@@ -40,7 +40,7 @@ struct Group {
   TrsmShape shape{};
   struct Step {
     bool leaf = true;
-    int njobs = 0, nb = 1;  // leaf solves: 16-vector blocks per workgroup
+    int njobs = 0, L = 0, nb = 1;  // leaf solves: rows, 16-vector blocks per workgroup
     long total_wg = 0;
     bool ta = false, tb = false, vec = false;  // GEMM updates
     GemmCfgId cfg{0, 128, 128};

@@ -441,6 +441,7 @@ int Dag::build_device_tables() {
           rec.table_off = blob.size();
           if (st.leaf) {
             rec.njobs = (int)st.tjobs.size();
+            rec.L = st.L;
             rec.nb = st.nb;
             for (const TrsmJob<T>& j : st.tjobs) rec.flops += (double)j.L * j.L * j.NV;
             rec.total_wg = st.total_wg;
@@ -580,8 +581,8 @@ int Dag::launch_group_t(const Group& G, hipStream_t s) {
       if (st.leaf) {
         TrsmJob<T> dummy{};
         dummy.prio = prio;
-        rc = trsm_launch<T>(G.shape, (const TrsmJob<T>*)st.table_dev, st.njobs, dummy, st.total_wg,
-                            ab, s, st.nb);
+        rc = trsm_launch<T>(G.shape, (const TrsmJob<T>*)st.table_dev, st.njobs, dummy, st.L,
+                            st.total_wg, ab, s, st.nb);
       } else {
         GemmJob<T> dummy{};
         dummy.prio = prio;

@@ -190,19 +190,27 @@ struct TrsmShape {
 TrsmShape trsm_shape(char side, char uplo, char transa, char diag);
 
 constexpr int TRSM_LEAF = 512;  // longest solve of one launch (longer ones recurse)
-// 16-vector blocks per workgroup of the leaf kernel: two when that still gives
-// every CU a workgroup (the triangle is read once per workgroup and its steps'
-// fixed costs are shared; 512 rows, 16384 vectors from the right: FP64 139 us
-// with two and about 200 with one, FP32 95 and 131), else one: a CU left without a
-// workgroup would cost more (512 rows, 4096 vectors take 46 us with one)
-inline int trsm_vec_blocks(long vectors) { return vectors >= 32 * 256 ? 2 : 1; }
-inline int trsm_wgs(int NV, int nb) { return (NV + 16 * nb - 1) / (16 * nb); }
-// Batched / single leaf solve (L <= TRSM_LEAF) over total_wg workgroups of nb
-// 16-vector blocks each.
+// 16-vector blocks per workgroup of the leaf kernel.  Above 256 rows, where a
+// workgroup fills a CU: two when that still gives every CU a workgroup (the
+// triangle is read once per workgroup and its steps' fixed costs are shared; 512
+// rows, 16384 vectors from the right: FP64 139 us with two and about 200 with one,
+// FP32 95 and 131), else one: a CU left without a workgroup would cost more (512
+// rows, 4096 vectors take 46 us with one).  Up to 256 rows a CU holds 16 waves of
+// workgroups with a wave per block row; from two rounds of these on, one round of
+// them takes all vectors, two blocks at a time.
+inline int trsm_vec_blocks(int L, long vectors) {
+  const long nblk = (L + 15) / 16, blocks = (vectors + 15) / 16;
+  if (nblk > 16) return vectors >= 32 * 256 ? 2 : 1;
+  const long round = 256 * 16 / nblk;
+  return blocks < 2 * round ? 1 : (int)(2 * ((blocks + 2 * round - 1) / (2 * round)));
+}
+inline long trsm_wgs(int NV, int nb) { return ((long)NV + 16L * nb - 1) / (16L * nb); }
+// Batched / single leaf solve (L <= TRSM_LEAF rows in every job) over total_wg
+// workgroups of nb 16-vector blocks each.
 template <typename T>
 int trsm_launch(const TrsmShape& sh, const TrsmJob<T>* jobs_dev, int njobs,
-                const TrsmJob<T>& single, long total_wg, const int* abort,
-                hipStream_t s, long nb);
+                const TrsmJob<T>& single, int L, long total_wg, const int* abort,
+                hipStream_t s, int nb);
 
 // Recursive batched solve: the launches (leaf solves and GEMM updates, in
 // issue order) that solve every job of `jobs` (any lengths).
@@ -212,7 +220,7 @@ struct TrsmStep {
   std::vector<TrsmJob<T>> tjobs;  // leaf solves (wg_begin filled)
   std::vector<GemmJob<T>> gjobs;  // update C = alpha_j V2 - Tm21 X1
   bool ta = false, tb = false;    // update operand transposes
-  int nb = 1;  // leaf solves: 16-vector blocks per workgroup
+  int L = 0, nb = 1;  // leaf solves: rows, 16-vector blocks per workgroup
   long total_wg = 0;
 };
 template <typename T>

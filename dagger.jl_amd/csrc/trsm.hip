@@ -12,6 +12,7 @@
 // update the second part with one (batched) GEMM on the MFMA GEMM kernel,
 // solve the second part -- so most of the flops of a long solve run at GEMM
 // speed.  A leaf is one launch of trsm_kernel; it needs no workspace.
+#include <algorithm>
 #include "dm_internal.h"
 #include "trsm_plan.h"
 
@@ -43,7 +44,7 @@ template <> struct Pair<float> { typedef float t __attribute__((ext_vector_type(
 
 constexpr int TB = 16;                 // block row
 constexpr int TW = 16;                 // waves of a workgroup
-constexpr int TQ = TRSM_LEAF / (TB * TW);  // block rows per wave
+constexpr int trsm_rows_per_wave(bool is_short) { return is_short ? 1 : TRSM_LEAF / (TB * TW); }
 // Steps of the triangle in flight, as many as the registers of 16 waves hold.
 template <typename T, int NB> constexpr int trsm_depth() {
   return sizeof(T) == 4 ? 4 : NB == 1 ? 2 : 1;
@@ -94,13 +95,30 @@ __device__ __forceinline__ void trsm_wave_sync() {
 // rows at 31 us that kept a whole 32-row chain in one wave, the products
 // between them and the inversion of the diagonal blocks).  Loads made
 // unconditional or a deeper prefetch measured slower or the same.
-template <typename T, bool LOWER, bool TTRANS, bool SIDE_L, int NB>
+//
+// SHORT: triangles of up to 256 rows, with a wave per block row and no more, their
+// diagonal blocks in as much LDS, and many vectors by a loop in each workgroup:
+// 16 waves and the whole LDS for a few block rows left most of a CU idle, and
+// every 32 vectors paid for the inverses again.  FP64, from the left: 8 rows,
+// 2000000 vectors 63 us, 1126 without; 64 rows, 100000 vectors 43 and 120; 256
+// rows, 100000 vectors 351 and 411; 64 rows, 64 vectors 8.5 and 10.2.
+template <typename T, bool LOWER, bool TTRANS, bool SIDE_L, int NB, bool SHORT>
 __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restrict__ jobs,
                                                        int njobs, TrsmJob<T> single, int unit,
-                                                       int prio, const int* __restrict__ abort) {
+                                                       int prio, int nb,
+                                                       const int* __restrict__ abort) {
   typedef typename MfmaT<T>::v4 v4;
-  constexpr int TD = trsm_depth<T, NB>();
-  __shared__ T Wd[TRSM_LEAF / TB][TB * TIS];   // diagonal blocks, then their inverses
+  constexpr int TD = trsm_depth<T, NB>(), TQ = trsm_rows_per_wave(SHORT);
+  __shared__ T Wd[SHORT ? 1 : TRSM_LEAF / TB][TB * TIS];
+  // diagonal blocks, then their inverses
+  auto Wb = [&](int p) -> T* {
+    if constexpr (SHORT) {
+      DM_DYNAMIC_LDS(trsm_lds);
+      return (T*)trsm_lds + p * TB * TIS;
+    } else {
+      return Wd[p];
+    }
+  };
   __shared__ T Xs[2][TB * TB * NB];            // X_J: [k][vector]
   if (abort && *abort) return;
   if (prio) raise_wave_priority();
@@ -120,7 +138,6 @@ __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restr
   const int L = job.L, NV = job.NV, nblk = (L + TB - 1) / TB;
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const int wave = __builtin_amdgcn_readlane((int)threadIdx.x >> 6, 0);
-  const int j0 = local * TB * NB;
   const auto A = gptr(job.A);
   const auto B = gptr(job.B);
   const size_t lda = job.lda, ldb = job.ldb;
@@ -135,8 +152,9 @@ __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restr
   // this lane's element of block row 0 and the steps along rows and vectors
   const ptrdiff_t bstep = (LOWER ? 1 : -1) * (SIDE_L ? 1 : (ptrdiff_t)ldb);
   const ptrdiff_t vstep = SIDE_L ? (ptrdiff_t)ldb : 1;
-  const auto brow = B + (LOWER ? 0 : (L - 1) * (SIDE_L ? 1 : (ptrdiff_t)ldb)) +
-                    MfmaT<T>::row(lk, 0) * bstep + (j0 + lr) * vstep;
+  unsigned j0 = (unsigned)local * TB * (SHORT ? nb : NB);
+  auto brow = B + (LOWER ? 0 : (L - 1) * (SIDE_L ? 1 : (ptrdiff_t)ldb)) +
+              MfmaT<T>::row(lk, 0) * bstep + (ptrdiff_t)(j0 + lr) * vstep;
   constexpr int RS = sizeof(T) == 8 ? 4 : 1;  // row(lk, r) = row(lk, 0) + RS r
   auto b_at = [&](int p, int r, int n) {
     return brow + uniform_offset((TB * p + RS * r) * bstep + TB * n * vstep);
@@ -188,7 +206,7 @@ __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restr
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int x = lr, y = 4 * e + lk;
-      Wd[p][(TTRANS ? y : x) * TIS + (TTRANS ? x : y)] = d[e];
+      Wb(p)[(TTRANS ? y : x) * TIS + (TTRANS ? x : y)] = d[e];
     }
   }
   trsm_wave_sync();
@@ -196,7 +214,7 @@ __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restr
   {
     const int p = wave + TW * lk;
     const bool on = lk < TQ && p < nblk;
-    T* W = Wd[on ? p : wave % nblk];
+    T* W = Wb(on ? p : wave % nblk);
     const int o = lr & 8, c = lr & 7;
     T x[8], z[4];
     const T dinv = T(1) / W[lr * TIS + lr];
@@ -247,124 +265,140 @@ __global__ __launch_bounds__(64 * TW) void trsm_kernel(const TrsmJob<T>* __restr
 
   // (no load is moved above this point: the registers are needed above)
   asm volatile("" ::: "memory");
-  // ---- this wave's right-hand sides (accumulator layout)
-  T vals[TQ][NB][4];
-#pragma unroll
-  for (int q = 0; q < TQ; ++q) {
-    const int p = wave + TW * q;
-#pragma unroll
-    for (int n = 0; n < NB; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = TB * p + MfmaT<T>::row(lk, r), j = j0 + TB * n + lr;
-        const bool in = i < L && j < NV;
-        vals[q][n][r] = *(in ? b_at(p, r, n) : B);
-        if (!in) vals[q][n][r] = T(0);
-      }
-  }
-  // the triangle's first TD steps
-  T t[TD][TQ][4];
-#pragma unroll
-  for (int u = 0; u < TD; ++u)
-#pragma unroll
-    for (int q = 0; q < TQ; ++q) {
-      if (nblk > 1) load_t(q, u, t[u][q]);
-    }
-  // ---- forward substitution
-  v4 acc[TQ][NB];
-#pragma unroll
-  for (int q = 0; q < TQ; ++q)
-#pragma unroll
-    for (int n = 0; n < NB; ++n) acc[q][n] = v4{0, 0, 0, 0};
-  const T alpha = job.alpha;
-  // X_p of block row p = wave + 16 q: to B, and to LDS for the later rows
-  auto finish = [&](int p, const v4 (&x)[NB]) {
-#pragma unroll
-    for (int n = 0; n < NB; ++n) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        Xs[p & 1][(MfmaT<T>::row(lk, r) * NB + n) * TB + lr] = x[n][r];
-    }
-#pragma unroll
-    for (int n = 0; n < NB; ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i = TB * p + MfmaT<T>::row(lk, r), j = j0 + TB * n + lr;
-        if (i < L && j < NV) *b_at(p, r, n) = x[n][r];
-      }
-  };
-  // X_p = W_p (alpha V_p - sum)
-  auto solve = [&](int p, const T (&v)[NB][4], const v4 (&sum)[NB]) {
-    T w[4];
-    v4 x[NB];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) w[s] = Wd[p][lr * TIS + MfmaT<T>::row(lk, s)];
-#pragma unroll
-    for (int n = 0; n < NB; ++n) {
-      x[n] = v4{0, 0, 0, 0};
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        // the accumulator's item s is the operand of k-step s (same lane)
-        const T rhs =
-            TB * p + MfmaT<T>::row(lk, s) < L ? alpha * v[n][s] - sum[n][s] : T(0);
-        x[n] = MfmaT<T>::mac(w[s], rhs, x[n]);
-      }
-    }
-    finish(p, x);
-  };
-  if (wave == 0) solve(0, vals[0], acc[0]);
-  __syncthreads();
-  auto step = [&](int J, T (&tj)[TQ][4]) {
-    T x[NB][4];
-#pragma unroll
-    for (int n = 0; n < NB; ++n)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) x[n][s] = Xs[J & 1][(tk(lk, s) * NB + n) * TB + lr];
-    auto update = [&](int q) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int n = 0; n < NB; ++n) acc[q][n] = MfmaT<T>::mac(tj[q][s], x[n][s], acc[q][n]);
-    };
-    // the next block row first, ahead of the other waves
-#pragma unroll
-    for (int q = 0; q < TQ; ++q)
-      if (wave + TW * q == J + 1 && J + 1 < nblk) {
-        __builtin_amdgcn_s_setprio(3);
-        update(q);
-        solve(J + 1, vals[q], acc[q]);
-        if (!prio) __builtin_amdgcn_s_setprio(0);  // back to the launch's own
-      }
+  // ---- NB vector blocks
+  int left = std::min(nb, (int)(NV - j0 - 1) / TB + 1);
+  for (;;) {
+    // this wave's right-hand sides (accumulator layout)
+    T vals[TQ][NB][4];
 #pragma unroll
     for (int q = 0; q < TQ; ++q) {
       const int p = wave + TW * q;
-      if (p > J + 1 && p < nblk) update(q);
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = TB * p + MfmaT<T>::row(lk, r);
+          const bool in = i < L && j0 + TB * n + lr < (unsigned)NV;
+          vals[q][n][r] = *(in ? b_at(p, r, n) : B);
+          if (!in) vals[q][n][r] = T(0);
+        }
     }
+    // the triangle's first TD steps
+    T t[TD][TQ][4];
 #pragma unroll
-    for (int q = 0; q < TQ; ++q) load_t(q, J + TD, tj[q]);
+    for (int u = 0; u < TD; ++u)
+#pragma unroll
+      for (int q = 0; q < TQ; ++q) {
+        if (nblk > 1) load_t(q, u, t[u][q]);
+      }
+    // ---- forward substitution
+    v4 acc[TQ][NB];
+#pragma unroll
+    for (int q = 0; q < TQ; ++q)
+#pragma unroll
+      for (int n = 0; n < NB; ++n) acc[q][n] = v4{0, 0, 0, 0};
+    const T alpha = job.alpha;
+    // X_p of block row p = wave + 16 q: to B, and to LDS for the later rows
+    auto finish = [&](int p, const v4 (&x)[NB]) {
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          Xs[p & 1][(MfmaT<T>::row(lk, r) * NB + n) * TB + lr] = x[n][r];
+      }
+#pragma unroll
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = TB * p + MfmaT<T>::row(lk, r);
+          if (i < L && j0 + TB * n + lr < (unsigned)NV) *b_at(p, r, n) = x[n][r];
+        }
+    };
+    // X_p = W_p (alpha V_p - sum)
+    auto solve = [&](int p, const T (&v)[NB][4], const v4 (&sum)[NB]) {
+      T w[4];
+      v4 x[NB];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) w[s] = Wb(p)[lr * TIS + MfmaT<T>::row(lk, s)];
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        x[n] = v4{0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          // the accumulator's item s is the operand of k-step s (same lane)
+          const T rhs =
+              TB * p + MfmaT<T>::row(lk, s) < L ? alpha * v[n][s] - sum[n][s] : T(0);
+          x[n] = MfmaT<T>::mac(w[s], rhs, x[n]);
+        }
+      }
+      finish(p, x);
+    };
+    if (wave == 0) solve(0, vals[0], acc[0]);
     __syncthreads();
-  };
-  // steps past the last block row only load (again) and pass the barrier
-#pragma unroll 1
-  for (int J = 0; J + 1 < nblk; J += TD) {
+    auto step = [&](int J, T (&tj)[TQ][4]) {
+      T x[NB][4];
 #pragma unroll
-    for (int u = 0; u < TD; ++u) step(J + u, t[u]);
+      for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x[n][s] = Xs[J & 1][(tk(lk, s) * NB + n) * TB + lr];
+      auto update = [&](int q) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int n = 0; n < NB; ++n) acc[q][n] = MfmaT<T>::mac(tj[q][s], x[n][s], acc[q][n]);
+      };
+      // the next block row first, ahead of the other waves
+#pragma unroll
+      for (int q = 0; q < TQ; ++q)
+        if (wave + TW * q == J + 1 && J + 1 < nblk) {
+          __builtin_amdgcn_s_setprio(3);
+          update(q);
+          solve(J + 1, vals[q], acc[q]);
+          if (!prio) __builtin_amdgcn_s_setprio(0);  // back to the launch's own
+        }
+#pragma unroll
+      for (int q = 0; q < TQ; ++q) {
+        const int p = wave + TW * q;
+        if (p > J + 1 && p < nblk) update(q);
+      }
+#pragma unroll
+      for (int q = 0; q < TQ; ++q) load_t(q, J + TD, tj[q]);
+      __syncthreads();
+    };
+    // steps past the last block row only load (again) and pass the barrier
+#pragma unroll 1
+    for (int J = 0; J + 1 < nblk; J += TD) {
+#pragma unroll
+      for (int u = 0; u < TD; ++u) step(J + u, t[u]);
+    }
+    if (!SHORT || (left -= NB) <= 0) break;
+    j0 += TB * NB;
+    brow += TB * NB * vstep;
   }
 }
 
 // ------------------------------------------------------------ host side
 template <typename T>
 int trsm_launch(const TrsmShape& sh, const TrsmJob<T>* jobs_dev, int njobs,
-                const TrsmJob<T>& single, long total_wg, const int* abort, hipStream_t s, long nb) {
+                const TrsmJob<T>& single, int L, long total_wg, const int* abort, hipStream_t s,
+                int nb) {
   if (total_wg <= 0) return 0;
   if (total_wg > 0x7fffffffL) return arg_fail(0, "trsm: too many workgroups");
-#define DM_TRSM_NB(LO, TT, SL, N)                                                            \
-  hipLaunchKernelGGL((trsm_kernel<T, LO, TT, SL, N>), dim3((unsigned)total_wg), dim3(64 * TW), \
-                     0, s, jobs_dev, njobs, single, sh.unit ? 1 : 0, single.prio, abort)
-#define DM_TRSM_GO(LO, TT, SL)              \
-  do {                                      \
-    if (nb == 2) DM_TRSM_NB(LO, TT, SL, 2); \
-    else DM_TRSM_NB(LO, TT, SL, 1);         \
+  const int nblk = (L + TB - 1) / TB, waves = std::min(nblk, TW);
+  const size_t lds = nblk <= TW ? sizeof(T) * nblk * TB * TIS : 0;
+#define DM_TRSM_NB(LO, TT, SL, N, SH)                                                              \
+  hipLaunchKernelGGL((trsm_kernel<T, LO, TT, SL, N, SH>), dim3((unsigned)total_wg),                \
+                     dim3(64 * waves), lds, s, jobs_dev, njobs, single, sh.unit ? 1 : 0,           \
+                     single.prio, nb, abort)
+#define DM_TRSM_GO(LO, TT, SL)                                                \
+  do {                                                                        \
+    if (nblk <= TW) {                                                         \
+      if (nb > 1) DM_TRSM_NB(LO, TT, SL, 2, true);                            \
+      else DM_TRSM_NB(LO, TT, SL, 1, true);                                   \
+    } else {                                                                  \
+      if (nb > 1) DM_TRSM_NB(LO, TT, SL, 2, false);                           \
+      else DM_TRSM_NB(LO, TT, SL, 1, false);                                  \
+    }                                                                         \
   } while (0)
   if (sh.lower) {
     if (sh.ttrans) { if (sh.side_l) DM_TRSM_GO(true, true, true); else DM_TRSM_GO(true, true, false); }
@@ -387,8 +421,8 @@ static int trsm_eff(const TrsmShape& sh, int L, int NV, T alpha, const T* A, int
   if (L <= TRSM_LEAF) {
     TrsmJob<T> j{};
     j.A = A; j.B = B; j.L = L; j.NV = NV; j.lda = lda; j.ldb = ldb; j.alpha = alpha;
-    const int nb = trsm_vec_blocks(NV);
-    return trsm_launch<T>(sh, nullptr, 0, j, trsm_wgs(NV, nb), abort, s, nb);
+    const int nb = trsm_vec_blocks(L, NV);
+    return trsm_launch<T>(sh, nullptr, 0, j, L, trsm_wgs(NV, nb), abort, s, nb);
   }
   const TrsmSplit sp = trsm_split(sh, L);
   int rc = trsm_eff<T>(sh, sp.first_n, NV, alpha, tm_sub(sh, A, lda, sp.first_r, sp.first_r), lda,
@@ -418,9 +452,9 @@ int trsm_full(char side, char uplo, char transa, char diag, int m, int n, T alph
 }
 
 template int trsm_launch<double>(const TrsmShape&, const TrsmJob<double>*, int,
-                                 const TrsmJob<double>&, long, const int*, hipStream_t, long);
+                                 const TrsmJob<double>&, int, long, const int*, hipStream_t, int);
 template int trsm_launch<float>(const TrsmShape&, const TrsmJob<float>*, int,
-                                const TrsmJob<float>&, long, const int*, hipStream_t, long);
+                                const TrsmJob<float>&, int, long, const int*, hipStream_t, int);
 template int trsm_full<double>(char, char, char, char, int, int, double, const double*, int,
                                double*, int, const int*, hipStream_t);
 template int trsm_full<float>(char, char, char, char, int, int, float, const float*, int, float*,

@@ -33,7 +33,8 @@ static void plan_rec(const TrsmShape& sh, int L, const std::vector<TrsmJob<T>>& 
     st.leaf = true;
     long vectors = 0;
     for (const TrsmJob<T>& j : jobs) vectors += j.NV;
-    st.nb = trsm_vec_blocks(vectors);
+    st.L = L;
+    st.nb = trsm_vec_blocks(L, vectors);
     long wg = 0;
     for (TrsmJob<T> j : jobs) {
       j.L = L;

@@ -90,7 +90,16 @@ template <typename T> int gemm_launch(bool, bool, bool, GemmCfgId, const GemmJob
 int gemm_wgs_per_cu(GemmCfgId c) { return c.id == 0 ? 1 : 2; }
 template <typename T> int gemm_single(bool, bool, int, int, int, T, const T*, int, const T*, int, T, T*, int, int, const int*, hipStream_t s) { trace_launch(s); ++g_launch; return 0; }
 template <typename T> int trinv_blocks_launch(const TrsmShape&, const T*, int, int, T* inv, const int*, hipStream_t s, int) { if (!inv) abort(); trace_launch(s); ++g_launch; return 0; }
-template <typename T> int trsm_launch(const TrsmShape&, const TrsmJob<T>*, int, const TrsmJob<T>&, long, const int*, hipStream_t s, long max_wg) { if (max_wg < 0) abort(); trace_launch(s); ++g_launch; return 0; }
+template <typename T> int trsm_launch(const TrsmShape&, const TrsmJob<T>* jobs, int njobs, const TrsmJob<T>&, int L, long total_wg, const int*, hipStream_t s, int nb) {
+  // the job table (device memory is host memory here) against the launch
+  if (L < 1 || L > TRSM_LEAF || nb < 1 || (nb > 1 && nb % 2) || (nb > 2 && L > 256)) abort();
+  long wg = 0;
+  for (int i = 0; i < njobs; ++i) {
+    if (jobs[i].L != L || jobs[i].NV < 1 || jobs[i].wg_begin != wg) abort();
+    wg += trsm_wgs(jobs[i].NV, nb);
+  }
+  if (wg != total_wg) abort();
+  trace_launch(s); ++g_launch; return 0; }
 template <typename T> int trsm_full(char, char, char, char, int, int, T, const T*, int, T*, int, T* ws, const int*, hipStream_t s) { if (!ws) abort(); trace_launch(s); ++g_launch; return 0; }
 template <typename T> int potrf_full(bool, int, T*, int, int*, int*, int, T*, hipStream_t s) { trace_launch(s); ++g_launch; return 0; }
 int potrf_f64_of_f32(bool, int, float*, int, double* W, int*, int*, int, hipStream_t s) { if (!W) abort(); trace_launch(s); ++g_launch; return 0; }
@@ -170,7 +179,7 @@ template <typename R> int zpotrf_rec(bool, int, R*, int, int*, int, int*, int, h
   template int gemm_launch<T>(bool, bool, bool, GemmCfgId, const GemmJob<T>*, int, const GemmJob<T>&, long, const int*, hipStream_t, long); \
   template int gemm_single<T>(bool, bool, int, int, int, T, const T*, int, const T*, int, T, T*, int, int, const int*, hipStream_t); \
   template int trinv_blocks_launch<T>(const TrsmShape&, const T*, int, int, T*, const int*, hipStream_t, int); \
-  template int trsm_launch<T>(const TrsmShape&, const TrsmJob<T>*, int, const TrsmJob<T>&, long, const int*, hipStream_t, long); \
+  template int trsm_launch<T>(const TrsmShape&, const TrsmJob<T>*, int, const TrsmJob<T>&, int, long, const int*, hipStream_t, int); \
   template int trsm_full<T>(char, char, char, char, int, int, T, const T*, int, T*, int, T*, const int*, hipStream_t); \
   template int potrf_full<T>(bool, int, T*, int, int*, int*, int, T*, hipStream_t); \
   template int gemv_launch<T>(bool, int, int, T, const T*, int, const T*, int, T, T*, int, const int*, hipStream_t); \

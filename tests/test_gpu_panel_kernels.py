@@ -188,6 +188,17 @@ def test_trsm_leaf(dm, dtype, side, uplo, trans, diag):
         _trsm(dm, dtype, side, uplo, trans, diag, L, nv, 0.75, pad)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("side,uplo,trans", [("L", "U", "T"), ("L", "L", "T"), ("R", "U", "T"),
+                                             ("R", "L", "N")])
+@pytest.mark.parametrize("L,nv", [(1, 131073), (16, 131103), (17, 65600), (130, 16389),
+                                  (256, 16400)])
+def test_trsm_many_vectors(dm, dtype, side, uplo, trans, L, nv):
+    """Short triangles whose vectors take more than a round of the chip: a
+    workgroup loops over several blocks of them, the last one over fewer."""
+    _trsm(dm, dtype, side, uplo, trans, "N", L, nv, 0.5, 1)
+
+
 @pytest.mark.parametrize("uplo", ["U", "L"])
 @pytest.mark.parametrize("trans", ["N", "T"])
 @pytest.mark.parametrize("L", [1, 8, 40])
