@@ -79,7 +79,6 @@ int exec_streams(hipStream_t, int count, hipStream_t* out) {
   return 0;
 }
 void release_exec_streams(hipStream_t) {}
-int trsm_init_attributes() { return 0; }
 int run_big_stack(std::function<int()> fn) { return fn(); }
 template <typename T> GemmCfgId gemm_pick_cfg(int, int, int, int, bool) { return GemmCfgId{0, 128, 128}; }
 template <typename T> long gemm_prepare_jobs(GemmJob<T>* jobs, int nj, GemmCfgId c) {
@@ -89,7 +88,6 @@ static long g_launch = 0;
 template <typename T> int gemm_launch(bool, bool, bool, GemmCfgId, const GemmJob<T>*, int, const GemmJob<T>&, long, const int*, hipStream_t s, long max_wg) { if (max_wg < 0) abort(); trace_launch(s); ++g_launch; return 0; }
 int gemm_wgs_per_cu(GemmCfgId c) { return c.id == 0 ? 1 : 2; }
 template <typename T> int gemm_single(bool, bool, int, int, int, T, const T*, int, const T*, int, T, T*, int, int, const int*, hipStream_t s) { trace_launch(s); ++g_launch; return 0; }
-template <typename T> int trinv_blocks_launch(const TrsmShape&, const T*, int, int, T* inv, const int*, hipStream_t s, int) { if (!inv) abort(); trace_launch(s); ++g_launch; return 0; }
 template <typename T> int trsm_launch(const TrsmShape&, const TrsmJob<T>* jobs, int njobs, const TrsmJob<T>&, int L, long total_wg, const int*, hipStream_t s, int nb) {
   // the job table (device memory is host memory here) against the launch
   if (L < 1 || L > TRSM_LEAF || nb < 1 || (nb > 1 && nb % 2) || (nb > 2 && L > 256)) abort();
@@ -100,7 +98,6 @@ template <typename T> int trsm_launch(const TrsmShape&, const TrsmJob<T>* jobs, 
   }
   if (wg != total_wg) abort();
   trace_launch(s); ++g_launch; return 0; }
-template <typename T> int trsm_full(char, char, char, char, int, int, T, const T*, int, T*, int, T* ws, const int*, hipStream_t s) { if (!ws) abort(); trace_launch(s); ++g_launch; return 0; }
 template <typename T> int potrf_full(bool, int, T*, int, int*, int*, int, T*, hipStream_t s) { trace_launch(s); ++g_launch; return 0; }
 int potrf_f64_of_f32(bool, int, float*, int, double* W, int*, int*, int, hipStream_t s) { if (!W) abort(); trace_launch(s); ++g_launch; return 0; }
 bool gemm_split_ok(bool ta, bool tb, const GemmJob<float>& j) {
@@ -178,9 +175,7 @@ template <typename R> int zpotrf_rec(bool, int, R*, int, int*, int, int*, int, h
   template bool gemm_job_vec_ok<T>(bool, bool, const GemmJob<T>&); \
   template int gemm_launch<T>(bool, bool, bool, GemmCfgId, const GemmJob<T>*, int, const GemmJob<T>&, long, const int*, hipStream_t, long); \
   template int gemm_single<T>(bool, bool, int, int, int, T, const T*, int, const T*, int, T, T*, int, int, const int*, hipStream_t); \
-  template int trinv_blocks_launch<T>(const TrsmShape&, const T*, int, int, T*, const int*, hipStream_t, int); \
   template int trsm_launch<T>(const TrsmShape&, const TrsmJob<T>*, int, const TrsmJob<T>&, int, long, const int*, hipStream_t, int); \
-  template int trsm_full<T>(char, char, char, char, int, int, T, const T*, int, T*, int, T*, const int*, hipStream_t); \
   template int potrf_full<T>(bool, int, T*, int, int*, int*, int, T*, hipStream_t); \
   template int gemv_launch<T>(bool, int, int, T, const T*, int, const T*, int, T, T*, int, const int*, hipStream_t); \
   template size_t getrf_panel_ws_bytes<T>(int64_t, int); \
