@@ -214,16 +214,18 @@ template int potrf_full<double>(bool, int, double*, int, int*, int*, int, double
 template int potrf_full<float>(bool, int, float*, int, int*, int*, int, float*, hipStream_t);
 
 // ------------------------------------------------------------ gemv
-// y := alpha op(A) x + beta y.  'N': a workgroup owns 32 rows, its 32 groups
-// of 32 lanes split the columns (coalesced along rows, eight columns a group in
-// flight) and reduce through LDS.  Bound by the latency of its few loads per
-// thread and, one workgroup per 32 rows, by how many CUs a tile reaches: 512 x
-// 512 FP64 6 us, against 39 us for 64 rows on four waves, one load at a time.
+// y := alpha op(A) x + beta y.  'N': a workgroup owns GN_ROWS rows, its groups of
+// as many lanes split the columns (coalesced along rows, eight columns a group in
+// flight) and reduce through LDS.  Bound by the latency of its few loads per thread
+// and by how many CUs a tile reaches: 512 x 512 FP64 as 32 groups on 32 rows 6 us,
+// against 39 us for 64 rows on four waves, one load at a time.  Other shapes where
+// 32 groups would have no column each or the rows alone fill the chip
+// (gemv_launch): 1000000 rows of 1, 4, 16 and 64 columns took 57, 81, 92 and 193 us
+// as 32 groups on 32 rows.
 // 'T': one wave per output element (column dot product, coalesced).
 // An empty inner dimension (n = 0 for 'N', m = 0 for 'T') leaves
 // y := beta y, as BLAS does (beta == 0 writes zeros without reading y).
-constexpr int GN_ROWS = 32, GN_GROUPS = 32;
-template <typename T>
+template <typename T, int GN_ROWS, int GN_GROUPS>
 __global__ __launch_bounds__(GN_ROWS * GN_GROUPS) void gemv_n_kernel(
     int m, int n, T alpha, const T* __restrict__ A, int lda, const T* __restrict__ x, int incx,
     T beta, T* __restrict__ y, int incy, const int* __restrict__ abort) {
@@ -287,9 +289,22 @@ int gemv_launch(bool trans, int m, int n, T alpha, const T* A, int lda, const T*
   // products: the 'N' kernel's column loop and the 'T' kernel's row loop
   // run zero times)
   if (!trans) {
-    hipLaunchKernelGGL(gemv_n_kernel<T>, dim3((m + GN_ROWS - 1) / GN_ROWS),
-                       dim3(GN_ROWS * GN_GROUPS), 0, s, m, n, alpha, A, lda, x, incx, beta, y, incy,
-                       abort);
+    // about eight columns a group; from 65536 rows on (1024 workgroups of 64) few
+    // groups on more rows, whose columns are longer contiguous pieces
+#define DM_GEMV_N(R, G)                                                                           \
+  hipLaunchKernelGGL((gemv_n_kernel<T, R, G>), dim3((unsigned)(((long)m + R - 1) / R)), dim3(R * G), \
+                     0, s, m, n, alpha, A, lda, x, incx, beta, y, incy, abort)
+    if (m >= 65536) {
+      if (n <= 8) DM_GEMV_N(256, 1);
+      else DM_GEMV_N(64, 4);
+    } else if (n <= 16) {
+      DM_GEMV_N(32, 2);
+    } else if (n <= 128) {
+      DM_GEMV_N(32, 8);
+    } else {
+      DM_GEMV_N(32, 32);
+    }
+#undef DM_GEMV_N
   } else {
     hipLaunchKernelGGL(gemv_t_kernel<T>, dim3((n + 3) / 4), dim3(256), 0, s, m, n, alpha, A, lda,
                        x, incx, beta, y, incy, abort);

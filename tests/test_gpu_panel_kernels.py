@@ -438,6 +438,21 @@ def test_gemv_n(dm, inc):
         assert np.array_equal(got[rest], y[rest])
 
 
+@pytest.mark.parametrize("m", [33, 65535, 65536, 65537])
+@pytest.mark.parametrize("n", [0, 1, 8, 9, 16, 17, 128, 129, 300])
+def test_gemv_n_groups(dm, m, n):
+    """Around the columns and rows at which a workgroup's shape changes, by the
+    product's bound 4 (n + 4) eps (|A| |x| + |y|)."""
+    rng = np.random.default_rng(m + n)
+    A = rng.standard_normal((m, max(n, 1)))
+    x, y = rng.standard_normal(max(n, 1)), rng.standard_normal(m)
+    dA, dx, dy = Dev(dm, A), Dev(dm, x), Dev(dm, y)
+    dm._lib.call("dm_dgemv", b"N", m, n, 0.5, dA.p, m, dx.p, 1, -2.0, dy.p, 1, None)
+    a, v = A[:, :n], x[:n]
+    bound = 4 * (n + 4) * np.finfo(float).eps * (np.abs(a) @ np.abs(v) + 2 * np.abs(y))
+    assert (np.abs(dy.get() - (0.5 * (a @ v) - 2.0 * y)) <= bound).all()
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("uplo", ["U", "L"])
 @pytest.mark.parametrize("n,nb", [(1, 1), (15, 15), (16, 16), (17, 17), (63, 63), (64, 64), (65, 65),
