@@ -18,6 +18,9 @@
 // launch's tiles, which only touch later rows.  The last launch has a single
 // tile and finishes its own row.
 //
+// Tiles of several thousand columns take separate launches for their first
+// panels (potrf_fused_blocks).
+//
 // Bound by the chain of launches and pivots, not by flops.  Measured per 64
 // columns of a 512 tile (FP64): one launch of 20 us, 8 of them the diagonal
 // block; the panel row and the update as two launches, with the block factored
@@ -60,16 +63,16 @@ __device__ __forceinline__ bool potrf_stop(const int* info, const int* abort, in
 }
 
 template <typename T, bool UPPER>
-__global__ __launch_bounds__(256) void potrf_diag_kernel(T* __restrict__ A, int n, int lda,
+__global__ __launch_bounds__(256) void potrf_diag_kernel(T* __restrict__ A, int n, int lda, int j0,
                                                          int* __restrict__ info,
                                                          int* __restrict__ abort,
                                                          int global_base) {
   __shared__ T M[PBE];
   __shared__ int fail, stop;
   raise_wave_priority();  // always on the critical path of a factorization
-  const int kb = min(PB, n);
+  const int kb = min(PB, n - j0);
   T v[16];
-  pb_load_diag<T, UPPER>(A, lda, 0, kb, v);
+  pb_load_diag<T, UPPER>(A, lda, j0, kb, v);
   if (threadIdx.x == 0) {
     stop = (abort && *abort) || (info && *info);
     // an info word that was set before this call stops its other launches too
@@ -78,7 +81,7 @@ __global__ __launch_bounds__(256) void potrf_diag_kernel(T* __restrict__ A, int 
   pb_put<T, UPPER>(M, v);
   __syncthreads();
   if (stop) return;
-  potrf_block<T, UPPER>(M, &fail, A, lda, 0, kb, info, abort, global_base);
+  potrf_block<T, UPPER>(M, &fail, A, lda, j0, kb, info, abort, global_base);
 }
 
 // The launch of panel j0 (see above): workgroups [0, ntile) own the tiles of
@@ -182,23 +185,52 @@ __global__ __launch_bounds__(256) void potrf_step_kernel(T* __restrict__ A, int 
 }
 
 namespace {
+// Column blocks right of a panel up to which its row, the trailing update and
+// the next diagonal block are one launch.  Beyond them the launch has several
+// rounds of workgroups (in FP64 a CU holds one), each solving its two row blocks
+// again, and a launch each for the row, the update (a product with K = 64 on the
+// GEMM's tiles) and the diagonal block is faster.  U, FP64, lines at 23, 31 and 47
+// blocks and none: n = 2048 774, 755, 753 and 755 us, 3072 1497, 1478, 1632 and
+// 1634, 4096 2765, 2755, 2914 and 3133, 8192 13.8, 13.8, 14.0 and 20.2 ms; FP32
+// 2048 577, 504, 504 and 504 us, 3072 1055, 980, 949 and 949, 4096 1630, 1558, 1541
+// and 1658, 8192 5.9, 5.8, 5.7 and 8.5 ms.
+template <typename T> constexpr int potrf_fused_blocks = sizeof(T) == 8 ? 31 : 47;
+
 template <typename T, bool UPPER>
 int potrf_panels(int n, T* A, int lda, int* info, int* abort, int global_offset, hipStream_t s) {
   // Launches after a failed pivot are no-ops: they watch the plan-level
   // abort flag when there is one, else info.
   if (n <= 0) return 0;
-  hipLaunchKernelGGL((potrf_diag_kernel<T, UPPER>), dim3(1), dim3(256), 0, s, A, n, lda, info, abort,
-                     global_offset);
-  DM_LAUNCH_CHECK("potrf_diag_kernel");
-  for (int j0 = 0; n - j0 > PB; j0 += PB) {
-    const int nt = (n - j0 - 1) / PB;  // 64-column blocks right of the panel
-    const int ntile = nt * (nt + 1) / 2;
-    const int nfin = j0 > 0 ? nt + 1 : 0;
+  auto diag = [&](int j0) {
+    hipLaunchKernelGGL((potrf_diag_kernel<T, UPPER>), dim3(1), dim3(256), 0, s, A, n, lda, j0, info,
+                       abort, global_offset);
+    DM_LAUNCH_CHECK("potrf_diag_kernel");
+    return 0;
+  };
+  auto step = [&](int j0, int ntile, int nfin) {
     hipLaunchKernelGGL((potrf_step_kernel<T, UPPER>), dim3((unsigned)(ntile + nfin)), dim3(256), 0, s,
                        A, n, lda, j0, ntile, info, abort, global_offset);
     DM_LAUNCH_CHECK("potrf_step_kernel");
+    return 0;
+  };
+  int rc = diag(0);
+  bool finish = false;  // the row of the panel before is not yet solved
+  for (int j0 = 0; !rc && n - j0 > PB; j0 += PB) {
+    const int nt = (n - j0 - 1) / PB;  // 64-column blocks right of the panel
+    if (nt <= potrf_fused_blocks<T>) {
+      rc = step(j0, nt * (nt + 1) / 2, finish ? nt + 1 : 0);
+      finish = true;
+      continue;
+    }
+    const int j1 = j0 + PB, rest = n - j1;
+    const T* const row = A + (UPPER ? (size_t)j1 * lda + j0 : (size_t)j0 * lda + j1);
+    rc = step(j1, 0, nt);
+    if (!rc)
+      rc = gemm_single<T>(UPPER, !UPPER, rest, rest, PB, T(-1), row, lda, row, lda, T(1),
+                          A + (size_t)j1 * lda + j1, lda, UPPER ? 1 : 2, abort ? abort : info, s);
+    if (!rc) rc = diag(j1);
   }
-  return 0;
+  return rc;
 }
 }  // namespace
 

@@ -121,6 +121,33 @@ def test_potrf_failed_pivot_leading_factor(dm, uplo, n, bad):
     assert np.abs(F - U).max() <= TOL[np.float64] * np.abs(U).max()
 
 
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("dtype,n", [(np.float64, 2048), (np.float64, 2113), (np.float64, 2300),
+                                     (np.float32, 3073), (np.float32, 3200)])
+def test_potrf_large_tile(dm, dtype, n, uplo):
+    """Around the size from which a panel's row, update and next diagonal block
+    are launches of their own: the factor by its backward error (sqrt(n) u, see
+    test_potrf_backward_error), the other triangle untouched."""
+    A = _smooth(n, 1.0).astype(dtype)
+    got, info = _potrf(dm, A, uplo, dtype)
+    assert info == 0
+    U = (np.triu(got) if uplo == "U" else np.tril(got).T).astype(np.float64)
+    # FP64: the product that checks has an error of its own of as much
+    rms = np.sqrt(np.mean((U.T @ U - A) ** 2))
+    assert rms <= (2 if dtype == np.float64 else 1) * 2 * np.sqrt(n) * np.finfo(dtype).eps / 2
+    other = np.tril(got, -1) if uplo == "U" else np.triu(got, 1)
+    assert np.array_equal(other, np.tril(A, -1) if uplo == "U" else np.triu(A, 1))
+
+
+@pytest.mark.parametrize("uplo", ["U", "L"])
+@pytest.mark.parametrize("bad", [63, 64, 200, 320, 1000, 2299])
+def test_potrf_failed_pivot_large_tile(dm, uplo, bad):
+    """The leading factor before a failed pivot where panels have launches of
+    their own, at the change to one launch (column 256) and after it."""
+    F, U = _leading_factor(dm, uplo, 2300, bad)
+    assert np.abs(F - U).max() <= 10 * TOL[np.float64] * np.abs(U).max()
+
+
 def _smooth(n, nugget):
     """A covariance matrix of close points: exp(-(x - y)^2 / 0.02) and a nugget
     on the diagonal.  Its condition is about n / nugget, and most of that lies
