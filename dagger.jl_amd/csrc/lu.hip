@@ -480,19 +480,21 @@ __global__ void lu_ipiv_kernel(const int* __restrict__ piv, int npiv, int64_t ro
 // four columns a workgroup spread the elements over the chip.  512 steps on
 // 512 columns of 4096 rows, FP64: 33 us, against 215 us with one thread a
 // column that made the swaps one after the other; the swaps within a panel
-// 6 against 23 us.
+// 6 against 23 us.  Fewer steps than threads (2^lg or fewer) take as many times
+// the columns: 8 steps on 1000000 columns 30 us, 726 with four a workgroup.
 constexpr int LS_THREADS = 512, LS_COLS = 4;
 template <typename T>
 __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base, int64_t Mr, int W,
                                                            int mb, int c0, int c1, int p0, int p1,
-                                                           const int* __restrict__ piv,
+                                                           int lg, const int* __restrict__ piv,
                                                            int64_t off,
                                                            const int* __restrict__ abort) {
   __shared__ int q[LS_THREADS], home[LS_THREADS];
   __shared__ int backward;
   if (abort && *abort) return;
-  const int t = threadIdx.x;
-  c0 += blockIdx.x * LS_COLS;
+  // thread t of a set of 2^lg: step t of columns c0, c0 + sets, ...
+  const int t = threadIdx.x & ((1 << lg) - 1), set = threadIdx.x >> lg, sets = LS_THREADS >> lg;
+  c0 += blockIdx.x * (sets * LS_COLS);
   for (int b0 = p0; b0 < p1; b0 += LS_THREADS) {
     const int n = std::min(LS_THREADS, p1 - b0), p = b0 + t;
     int mine = -1;
@@ -500,8 +502,8 @@ __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base,
       const int64_t to = (int64_t)piv[p - p0] - off;
       mine = to >= 0 && to < Mr ? (int)to : p;
     }
-    if (t == 0) backward = 0;
-    q[t] = mine;
+    if (threadIdx.x == 0) backward = 0;
+    if (set == 0) q[t] = mine;
     __syncthreads();
     if (t < n && mine < p) backward = 1;
     // the last earlier step that names this step's row, the last earlier one
@@ -515,14 +517,14 @@ __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base,
       if (i < t && x == mine) same = i;
       if (i > t && x == mine) later = true;
     }
-    home[t] = own;
+    if (set == 0) home[t] = own;
     __syncthreads();
     if (backward) {
-      if (t < LS_COLS && c0 + t < c1)
+      for (int c = c0 + threadIdx.x; c < std::min(c0 + sets * LS_COLS, c1); c += LS_THREADS)
         for (int i = 0; i < n; ++i)
           if (q[i] != b0 + i) {
-            T* a = tiled_at(base, Mr, mb, W, b0 + i, c0 + t);
-            T* b = tiled_at(base, Mr, mb, W, q[i], c0 + t);
+            T* a = tiled_at(base, Mr, mb, W, b0 + i, c);
+            T* b = tiled_at(base, Mr, mb, W, q[i], c);
             const T v = *a;
             *a = *b;
             *b = v;
@@ -548,8 +550,10 @@ __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base,
         const int64_t k = from[e] / mb, l = std::min<int64_t>(mb, Mr - k * mb);
         const T* a = base + k * (int64_t)mb * W + (from[e] - k * mb);
 #pragma unroll
-        for (int c = 0; c < LS_COLS; ++c)
-          if (c0 + c < c1) v[e][c] = a[(c0 + c) * l];
+        for (int c = 0; c < LS_COLS; ++c) {
+          const int col = c0 + set + sets * c;
+          if (col < c1) v[e][c] = a[col * l];
+        }
       }
     __syncthreads();
 #pragma unroll
@@ -558,8 +562,10 @@ __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base,
         const int64_t k = to[e] / mb, l = std::min<int64_t>(mb, Mr - k * mb);
         T* a = base + k * (int64_t)mb * W + (to[e] - k * mb);
 #pragma unroll
-        for (int c = 0; c < LS_COLS; ++c)
-          if (c0 + c < c1) a[(c0 + c) * l] = v[e][c];
+        for (int c = 0; c < LS_COLS; ++c) {
+          const int col = c0 + set + sets * c;
+          if (col < c1) a[col * l] = v[e][c];
+        }
       }
     __syncthreads();
   }
@@ -572,8 +578,13 @@ unsigned blocks_of(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 template <typename T>
 int laswp_launch(T* base, int64_t Mr, int W, int mb, int c0, int c1, int p0, int p1,
                  const int* piv, int64_t off, const int* abort, hipStream_t s) {
-  hipLaunchKernelGGL((laswp_kernel<T>), dim3(blocks_of(c1 - c0, LS_COLS)), dim3(LS_THREADS), 0, s,
-                     base, Mr, W, mb, c0, c1, p0, p1, piv, off, abort);
+  // sets of threads no larger than the steps need, as long as every CU has columns
+  int lg = 0;
+  while ((1 << lg) < std::min(p1 - p0, LS_THREADS) ||
+         ((1 << lg) < LS_THREADS && blocks_of(c1 - c0, (LS_THREADS >> lg) * LS_COLS) < 256))
+    ++lg;
+  hipLaunchKernelGGL((laswp_kernel<T>), dim3(blocks_of(c1 - c0, (LS_THREADS >> lg) * LS_COLS)),
+                     dim3(LS_THREADS), 0, s, base, Mr, W, mb, c0, c1, p0, p1, lg, piv, off, abort);
   DM_LAUNCH_CHECK("laswp_kernel");
   return 0;
 }

@@ -336,6 +336,24 @@ def test_row_swaps(dm, m, n, nb, steps, kind):
     assert np.array_equal(D.collect(), B)
 
 
+@pytest.mark.parametrize("m,n,steps", [(3, 524288, 1), (9, 260000, 3), (40, 16385, 17), (300, 1030, 257)])
+@pytest.mark.parametrize("kind", ["pivots", "any"])
+def test_row_swaps_many_columns(dm, m, n, steps, kind):
+    """Fewer steps than threads: sets of them on columns of their own."""
+    rng = np.random.default_rng(n)
+    B = rng.standard_normal((m, n))
+    piv = np.array([rng.integers(p, m) for p in range(steps)]) + 1
+    if kind == "any":
+        piv = rng.integers(-3, m + 5, steps)
+    D, ip = dm.DArray.from_array(B, dm.Blocks(n, n)), Dev(dm, piv.astype(np.int32))
+    t = D.tiled()
+    dm._lib.call("dm_tiled_laswp", C.byref(t), ip.p, steps, None)
+    for p, q in enumerate(piv - 1):
+        if 0 <= q < m:
+            B[[p, q]] = B[[q, p]]
+    assert np.array_equal(D.collect(), B)
+
+
 def _crand(rng, *shape):
     return rng.standard_normal(shape) + 1j * rng.standard_normal(shape)
 
