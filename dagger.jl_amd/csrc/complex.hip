@@ -21,6 +21,7 @@
 //    the matrix cores between them.
 // Every kernel returns at once when the abort word is set (a failed pivot),
 // so the rest of a failed factorization becomes a no-op.
+#include <algorithm>
 #include "dm_internal.h"
 #include "complex_ops.h"
 #include "potrf_diag.h"
@@ -286,23 +287,27 @@ template <typename V> __device__ __forceinline__ V neg_recip(V d) {
 // of 64 rows at 145 us, one thread a vector walking the triangle in LDS, and the
 // products between them).  One step of T in flight in FP64: with two the
 // registers of 16 waves do not hold the substitution's operands (16 vectors 51 us).
-template <typename R>
-__global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ T, int L, int ldt,
+//
+// SHORT: up to 32 rows, with a loop over the vectors in each workgroup and the
+// diagonal blocks in as much LDS as they need (the LDS of 256 rows lets a CU hold
+// one workgroup of one or two waves): 1 row, 2000000 vectors FP64 72 us, 671
+// without, 16 rows, 1000000 vectors 100 and 435; from 64 rows on the loop's
+// registers cost more than it gives (100000 vectors 184 and 142 us).
+template <typename R, bool SHORT>
+__global__ __launch_bounds__(SHORT ? 512 : 1024) void ztrsm_leaf_kernel(const R* __restrict__ T, int L, int ldt,
                                                           bool lower, int op, bool unit,
                                                           R alpha_re, R alpha_im,
                                                           R* __restrict__ B, int64_t estride,
-                                                          int64_t vstride, int nvec,
+                                                          int64_t vstride, int nvec, int nb,
                                                           const int* __restrict__ abort) {
   typedef typename Mf<R>::v4 v4;
   typedef R v2 __attribute__((ext_vector_type(2)));
   constexpr int S = ZTB + 1, D = sizeof(R) == 4 ? 2 : 1;  // LDS row stride; steps of T in flight
-  __shared__ v2 Td[ZTRSM_LEAF / ZTB][ZTB * S];  // diagonal blocks
-  __shared__ v2 Rd[ZTRSM_LEAF / ZTB][ZTB];      // their diagonals' negative reciprocals
-  __shared__ v2 Xs[2][ZTB * ZTB];               // X_J: [row][vector]
+  __shared__ v2 Xs[2][ZTB * ZTB];  // X_J: [row][vector]
   if (abort && *abort) return;
   const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
   const int p = __builtin_amdgcn_readlane((int)threadIdx.x >> 6, 0);
-  const int nblk = (L + ZTB - 1) / ZTB, j0 = blockIdx.x * ZTB;
+  const int nblk = (L + ZTB - 1) / ZTB;
   const bool tt = op == 1 || op == 2, lo = tt ? !lower : lower;
   const R sg = op >= 2 ? R(-1) : R(1);  // conjugation
   // element (i, k) of the lower triangle: t0[i * rs + k * cs]
@@ -325,7 +330,16 @@ __global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ 
     for (int s = 0; s < 4; ++s) t[s] = *gptr(trow + (ZTB * J + tk(s)) * cs);
   };
   // ---- the diagonal block, the identity's past the end, and -1 / T_rr
-  v2* const W = Td[p];
+  constexpr int TE = ZTB * S + ZTB;  // LDS elements of both
+  v2* W;
+  if constexpr (SHORT) {
+    DM_DYNAMIC_LDS(ztrsm_lds);
+    W = (v2*)ztrsm_lds + p * TE;
+  } else {
+    __shared__ v2 Td[ZTRSM_LEAF / ZTB][TE];
+    W = Td[p];
+  }
+  v2* const Rd = W + ZTB * S;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int x = lr, y = 4 * e + lk;  // x along the contiguous axis
@@ -337,115 +351,123 @@ __global__ __launch_bounds__(1024) void ztrsm_leaf_kernel(const R* __restrict__ 
       d.y *= sg;
     }
     W[r * S + c] = d;
-    if (r == c) Rd[p][r] = neg_recip(d);
+    if (r == c) Rd[r] = neg_recip(d);
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  v2 t[D][4];
+  unsigned j0 = blockIdx.x * (unsigned)(ZTB * (SHORT ? nb : 1));
+  int left = std::min(nb, (int)(nvec - j0 - 1) / ZTB + 1);
+  for (;;) {
+    asm volatile("" ::: "memory");  // (no operand is kept from one pass to the next)
+    v2 t[D][4];
 #pragma unroll
-  for (int u = 0; u < D; ++u) load_t(u, t[u]);
-  // the right-hand side in the accumulator layout
-  v2 v[4];
-  v2* const bvec = b0 + (j0 + lr) * vstride;
-  const bool mine = j0 + lr < nvec;
+    for (int u = 0; u < D; ++u) load_t(u, t[u]);
+    // the right-hand side in the accumulator layout
+    v2 v[4];
+    v2* const bvec = b0 + (int64_t)(j0 + lr) * vstride;
+    const bool mine = j0 + lr < (unsigned)nvec;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int i = ZTB * p + Mf<R>::row(lk, r);
-    v[r] = v2{0, 0};
-    if (mine && i < L) v[r] = *gptr((const v2*)bvec + i * es);
-  }
-  // ---- forward substitution
-  v4 ar = v4{0, 0, 0, 0}, ai = v4{0, 0, 0, 0};
-  // X_p from the sums: four rows at a time by substitution, a product of depth 4
-  // for the rows below, in sums of the opposite sign (as pb_solve).  The operands
-  // of a step are read while the matrix cores are at the one before.
-  v2 u[4][4], q[4];
-  auto read = [&](int s) {
-    const int o = 4 * s;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-      for (int k = 0; k < i; ++k) u[i][k] = W[(o + i) * S + o + k];
-      q[i] = Rd[p][o + i];
+    for (int r = 0; r < 4; ++r) {
+      const int i = ZTB * p + Mf<R>::row(lk, r);
+      v[r] = v2{0, 0};
+      if (mine && i < L) v[r] = *gptr((const v2*)bvec + i * es);
     }
-  };
-  auto solve = [&] {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const bool in = ZTB * p + Mf<R>::row(lk, s) < L;
-      ar[s] = in ? ar[s] - (alpha_re * v[s].x - alpha_im * v[s].y) : R(0);
-      ai[s] = in ? ai[s] - (alpha_re * v[s].y + alpha_im * v[s].x) : R(0);
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    // ---- forward substitution
+    v4 ar = v4{0, 0, 0, 0}, ai = v4{0, 0, 0, 0};
+    // X_p from the sums: four rows at a time by substitution, a product of depth 4
+    // for the rows below, in sums of the opposite sign (as pb_solve).  The operands
+    // of a step are read while the matrix cores are at the one before.
+    v2 u[4][4], q[4];
+    auto read = [&](int s) {
       const int o = 4 * s;
-      R xr[4], xi[4];
-      four_rows(ar, s, xr);
-      four_rows(ai, s, xi);
-      const v2 a = W[lr * S + o + lk];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int k = 0; k < i; ++k) {
-          const v2 d = u[i][k];
-          xr[i] += d.x * xr[k];
-          xi[i] += d.x * xi[k];
-          xr[i] -= d.y * xi[k];
-          xi[i] += d.y * xr[k];
-        }
-        const v2 d = q[i];
-        const R w = xr[i];
-        xr[i] = w * d.x - xi[i] * d.y;
-        xi[i] = w * d.y + xi[i] * d.x;
+        for (int k = 0; k < i; ++k) u[i][k] = W[(o + i) * S + o + k];
+        q[i] = Rd[o + i];
       }
-      const v2 x = v2{row_by_group(xr, s), row_by_group(xi, s)};
-      if (s < 3) {
-        ar = Mf<R>::mac(a.x, x.x, ar);
-        ai = Mf<R>::mac(a.x, x.y, ai);
-        ar = Mf<R>::mac(-a.y, x.y, ar);
-        __builtin_amdgcn_sched_barrier(0);
-        read(s + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        ai = Mf<R>::mac(a.y, x.x, ai);
-      }
-      const int i = ZTB * p + o + lk;
-      Xs[p & 1][(o + lk) * ZTB + lr] = x;
-      if (mine && i < L) *gptr(bvec + i * es) = x;
-    }
-  };
-  if (p == 0) {
-    read(0);
-    solve();
-  }
-  __syncthreads();
-  auto step = [&](int J, v2 (&tj)[4]) {
-    if (J < p && J + 1 < nblk) {
-      if (p == J + 1) {
-        __builtin_amdgcn_s_setprio(3);
-        read(0);
+    };
+    auto solve = [&] {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bool in = ZTB * p + Mf<R>::row(lk, s) < L;
+        ar[s] = in ? ar[s] - (alpha_re * v[s].x - alpha_im * v[s].y) : R(0);
+        ai[s] = in ? ai[s] - (alpha_re * v[s].y + alpha_im * v[s].x) : R(0);
       }
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        const v2 x = Xs[J & 1][(2 * lk + tk(s)) * ZTB + lr];
-        const R tr = tj[s].x, ti = sg * tj[s].y;
-        ar = Mf<R>::mac(tr, x.x, ar);
-        ai = Mf<R>::mac(tr, x.y, ai);
-        ar = Mf<R>::mac(-ti, x.y, ar);
-        ai = Mf<R>::mac(ti, x.x, ai);
+        const int o = 4 * s;
+        if (SHORT && ZTB * p + o >= L) break;
+        R xr[4], xi[4];
+        four_rows(ar, s, xr);
+        four_rows(ai, s, xi);
+        const v2 a = W[lr * S + o + lk];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+          for (int k = 0; k < i; ++k) {
+            const v2 d = u[i][k];
+            xr[i] += d.x * xr[k];
+            xi[i] += d.x * xi[k];
+            xr[i] -= d.y * xi[k];
+            xi[i] += d.y * xr[k];
+          }
+          const v2 d = q[i];
+          const R w = xr[i];
+          xr[i] = w * d.x - xi[i] * d.y;
+          xi[i] = w * d.y + xi[i] * d.x;
+        }
+        const v2 x = v2{row_by_group(xr, s), row_by_group(xi, s)};
+        if (s < 3) {
+          ar = Mf<R>::mac(a.x, x.x, ar);
+          ai = Mf<R>::mac(a.x, x.y, ai);
+          ar = Mf<R>::mac(-a.y, x.y, ar);
+          __builtin_amdgcn_sched_barrier(0);
+          read(s + 1);
+          __builtin_amdgcn_sched_barrier(0);
+          ai = Mf<R>::mac(a.y, x.x, ai);
+        }
+        const int i = ZTB * p + o + lk;
+        Xs[p & 1][(o + lk) * ZTB + lr] = x;
+        if (mine && i < L) *gptr(bvec + i * es) = x;
       }
-      if (p == J + 1) {
-        solve();
-        __builtin_amdgcn_s_setprio(0);
-      }
-      load_t(J + D, tj);
+    };
+    if (p == 0) {
+      read(0);
+      solve();
     }
     __syncthreads();
-  };
-#pragma unroll 1
-  for (int J = 0; J + 1 < nblk; J += D) {
+    auto step = [&](int J, v2 (&tj)[4]) {
+      if (J < p && J + 1 < nblk) {
+        if (p == J + 1) {
+          __builtin_amdgcn_s_setprio(3);
+          read(0);
+        }
 #pragma unroll
-    for (int u = 0; u < D; ++u) step(J + u, t[u]);
+        for (int s = 0; s < 4; ++s) {
+          const v2 x = Xs[J & 1][(2 * lk + tk(s)) * ZTB + lr];
+          const R tr = tj[s].x, ti = sg * tj[s].y;
+          ar = Mf<R>::mac(tr, x.x, ar);
+          ai = Mf<R>::mac(tr, x.y, ai);
+          ar = Mf<R>::mac(-ti, x.y, ar);
+          ai = Mf<R>::mac(ti, x.x, ai);
+        }
+        if (p == J + 1) {
+          solve();
+          __builtin_amdgcn_s_setprio(0);
+        }
+        load_t(J + D, tj);
+      }
+      __syncthreads();
+    };
+#pragma unroll 1
+    for (int J = 0; J + 1 < nblk; J += D) {
+#pragma unroll
+      for (int u = 0; u < D; ++u) step(J + u, t[u]);
+    }
+    if (!SHORT || --left <= 0) break;
+    j0 += ZTB;
   }
 }
 
@@ -495,9 +517,20 @@ int ztrsm_rec(bool left, bool lower, int op, bool unit, int L, R ar, R ai, const
     // on B's rows (op N<->T, H<->conj)
     const int lop = left ? op : (op == 0 ? 1 : op == 1 ? 0 : op == 2 ? 3 : 2);
     const int64_t es = left ? 1 : ldb, vs = left ? ldb : 1;
-    hipLaunchKernelGGL((ztrsm_leaf_kernel<R>), dim3((nv + ZTB - 1) / ZTB),
-                       dim3(64 * ((L + ZTB - 1) / ZTB)), 0, s, T, L, ldt, lower, lop, unit, ar, ai,
-                       B, es, vs, nv, abort);
+    const int nblk = (L + ZTB - 1) / ZTB;
+    const long blocks = ((long)nv + ZTB - 1) / ZTB;
+    if (nblk <= 2) {
+      // from two rounds of 12 waves a CU on, one round takes all vectors
+      const long round = 256 * 12 / nblk;
+      const int nb = blocks < 2 * round ? 1 : (int)((blocks + round - 1) / round);
+      const size_t lds = 2 * sizeof(R) * nblk * (ZTB * (ZTB + 1) + ZTB);
+      hipLaunchKernelGGL((ztrsm_leaf_kernel<R, true>), dim3((unsigned)((blocks + nb - 1) / nb)),
+                         dim3(64 * nblk), lds, s, T, L, ldt, lower, lop, unit, ar, ai, B, es, vs, nv,
+                         nb, abort);
+    } else {
+      hipLaunchKernelGGL((ztrsm_leaf_kernel<R, false>), dim3((unsigned)blocks), dim3(64 * nblk), 0, s,
+                         T, L, ldt, lower, lop, unit, ar, ai, B, es, vs, nv, 1, abort);
+    }
     DM_LAUNCH_CHECK("ztrsm_leaf_kernel");
     return 0;
   }

@@ -442,6 +442,35 @@ def test_complex_trsm_leaf(dm, dtype, side, uplo, trans):
 
 
 @pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("side,uplo,trans", [("L", "U", "C"), ("L", "L", "T"), ("R", "U", "C"),
+                                             ("R", "L", "N")])
+@pytest.mark.parametrize("L,nv", [(1, 98305), (4, 98320), (6, 131), (16, 98303), (17, 49200),
+                                  (32, 49153)])
+def test_complex_trsm_many_vectors(dm, dtype, side, uplo, trans, L, nv):
+    """Short triangles: a workgroup loops over its vectors once they take more
+    than two rounds of the chip; the bound of test_complex_trsm_leaf."""
+    rng = np.random.default_rng(L)
+    A = (0.5 * _crand(rng, L, L) / np.sqrt(2 * L)).astype(dtype)
+    A[np.arange(L), np.arange(L)] = 1.5 + rng.random(L) + 0.5j * rng.random(L)
+    m, n = (L, nv) if side == "L" else (nv, L)
+    B = _crand(rng, m + 1, n).astype(dtype)
+    dA, dB = Dev(dm, A), Dev(dm, B)
+    p, R = ("z", np.float64) if dtype == np.complex128 else ("c", np.float32)
+    alpha = np.array([1.0, 0.5], R)
+    dm._lib.call(f"dm_{p}trsm", side.encode(), uplo.encode(), trans.encode(), b"N", m, n,
+                 alpha.ctypes.data_as(C.c_void_p), dA.p, L, dB.p, m + 1, None)
+    got = dB.get()
+    assert np.array_equal(got[m:], B[m:])
+    T = (np.triu(A) if uplo == "U" else np.tril(A)).astype(complex)
+    op = {"N": T, "T": T.T, "C": T.conj().T}[trans]
+    X, rhs = got[:m].astype(complex), (1.0 + 0.5j) * B[:m].astype(complex)
+    if side == "R":
+        op, X, rhs = op.T, X.T, rhs.T
+    bound = 8 * (L + 16) * np.finfo(dtype).eps * (np.abs(op) @ np.abs(X))
+    assert (np.abs(op @ X - rhs) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
 @pytest.mark.parametrize("ta", ["N", "T", "C"])
 @pytest.mark.parametrize("tb", ["N", "T", "C"])
 def test_complex_gemm_tiles(dm, dtype, ta, tb):
