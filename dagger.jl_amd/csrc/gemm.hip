@@ -449,7 +449,11 @@ struct GemmKernel {
     }
     // Ragged and diagonal tiles: the old values are loaded without branches
     // (past an edge, the last row or column again), for the same reason (FP32
-    // 2000 x 2000 x 512: 71 us with a branch around each load, 65 without).
+    // 2000 x 2000 x 512: 71 us with a branch around each load, 65 without).  Not on
+    // FP32 tiles of 64: 18 more registers, a wave less on each SIMD (A B, 130 x
+    // 130 x 8000 320 us with the branches, 352 without; 1000 x 1000 x 1000 50 and
+    // 54), nor on FP32 A^T B^T (4096 x 4096 x 4096 1269 us and 1465).
+    constexpr bool free_loads = sizeof(T) == 8 || (BM * BN > 64 * 64 && !(TA && TB));
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       const int m = m0 + wm0 + i * 16 + lr;
@@ -459,8 +463,11 @@ struct GemmKernel {
 #pragma unroll
         for (int j = 0; j < FN; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            old[j][r] = crow[(size_t)min(n0 + wn0 + j * 16 + Mfma<T>::row(lk, r), N - 1) * job.ldc];
+          for (int r = 0; r < 4; ++r) {
+            const int n = n0 + wn0 + j * 16 + Mfma<T>::row(lk, r);
+            if (free_loads) old[j][r] = crow[(size_t)min(n, N - 1) * job.ldc];
+            else old[j][r] = in_c(m, n, M, N, tri) ? crow[(size_t)n * job.ldc] : T(0);
+          }
       }
 #pragma unroll
       for (int j = 0; j < FN; ++j)
@@ -719,12 +726,14 @@ int launch_cfg(int id, const GemmJob<T>* jobs, int njobs, const GemmJob<T>& sing
       return launch_one<T, 128, 128, 32, 4, 4, TA, TB, VEC>(jobs, njobs, single, total, grid, abort,
                                                             s);
   } else {
-    // eight waves rather than four: with four a CU holds too few of them to
-    // cover a short K (2000 x 2000 x 512: 65 us against 58, 4000 x 4000 x 256:
-    // 107 against 103; 4096 x 4096 x 4096 1208 against 1212)
+    // eight waves rather than four where one operand is transposed: with four a CU
+    // holds too few of them to cover a short K (A^T B, 2000 x 2000 x 512: 65 us
+    // against 58, 4000 x 4000 x 256: 107 against 103; 4096 x 4096 x 4096 1278 against
+    // 1260, A B^T 1278 against 1236).  A B and A^T B^T lose by them (4096 x 4096 x 64 43 and
+    // 52 us, 4096 x 4096 x 4096 1273 and 1345).
     if (id == 0)
-      return launch_one<T, 128, 128, 16, 4, 2, TA, TB, VEC>(jobs, njobs, single, total, grid, abort,
-                                                            s);
+      return launch_one<T, 128, 128, 16, TA != TB ? 4 : 2, 2, TA, TB, VEC>(jobs, njobs, single, total,
+                                                                           grid, abort, s);
   }
   if (id == 1)
     return launch_one<T, 64, 64, 16, 2, 2, TA, TB, VEC>(jobs, njobs, single, total, grid, abort, s);
