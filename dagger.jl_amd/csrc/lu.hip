@@ -609,7 +609,10 @@ int getf2_leaf(T* P, int64_t Mp, int c0, int nc, int* piv, int* linfo, int* abor
   if (r <= 4) return getf2_reg_launch<T, 4, 8>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
   if (r <= 8) return getf2_reg_launch<T, 8, 8>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
   if (r <= 16) return getf2_reg_launch<T, 16, 4>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
-  if (r <= 32) return getf2_reg_launch<T, 32, 2>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
+  // (1 to 3 FP64 columns of 12000 rows: 80, 89 and 112 us from registers, which
+  // spill here, 64, 81 and 97 in memory)
+  if (r <= 32 && (sizeof(T) == 4 || nc > 3))
+    return getf2_reg_launch<T, 32, 2>(P, Mp, c0, nc, piv, linfo, abort, pivot, s);
   hipLaunchKernelGGL((getf2_leaf_kernel<T>), dim3(1), dim3(LU_THREADS), 0, s, P, Mp, c0, nc, piv,
                      linfo, abort, pivot ? 1 : 0);
   DM_LAUNCH_CHECK("getf2_leaf_kernel");

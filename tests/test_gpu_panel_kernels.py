@@ -291,6 +291,20 @@ def test_lu_panel(dm, dtype, pivot, m, n):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("m", [8192, 8193, 16384])
+@pytest.mark.parametrize("n", [1, 2, 3, 4])
+def test_lu_panel_narrow(dm, dtype, m, n):
+    """Around the columns and rows at which a leaf goes from registers to
+    memory: test_lu_panel's pivots and bound."""
+    A = np.random.default_rng(m + n).standard_normal((m, n)).astype(dtype)
+    DA = dm.DArray.from_array(A, dm.Blocks(m, m))
+    F = dm.lu_(DA, dm.RowMaximum(), check=False)
+    want, piv = _getf2(A, True)
+    assert np.array_equal(F.ipiv, piv)
+    assert np.abs(DA.collect() - want).max() <= 32 * n * np.finfo(dtype).eps * np.abs(want).max()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_lu_panel_values(dm, dtype):
     """Columns of zeros, NaN and infinities, pivots too small to invert."""
     rng = np.random.default_rng(3)
