@@ -45,7 +45,8 @@ template <> struct Pair<float> { typedef float t __attribute__((ext_vector_type(
 constexpr int TB = 16;                 // block row
 constexpr int TW = 16;                 // waves of a workgroup
 constexpr int trsm_rows_per_wave(bool is_short) { return is_short ? 1 : TRSM_LEAF / (TB * TW); }
-// Steps of the triangle in flight, as many as the registers of 16 waves hold.
+// Steps of the triangle in flight, as many as the 128 registers of 16 waves hold
+// (FP64 with two vector blocks, above 256 rows, spills two).
 template <typename T, int NB> constexpr int trsm_depth() {
   return sizeof(T) == 4 ? 4 : NB == 1 ? 2 : 1;
 }
