@@ -22,9 +22,10 @@
 // panels (potrf_fused_blocks).
 //
 // Bound by the chain of launches and pivots, not by flops.  Measured per 64
-// columns of a 512 tile (FP64): one launch of 20 us, 8 of them the diagonal
-// block; the panel row and the update as two launches, with the block factored
-// by one lane per column from LDS rows, took 23 + 40 us.
+// columns of a 512 tile (FP64): one launch of 20 us, 8 of them pb_factor; the
+// panel row and the update as two launches, with the block factored by one lane
+// per column from LDS rows, took 23 + 40 us.
+//
 // After a failed pivot the remaining launches do nothing but finish the rows
 // before it (the factor of the leading minor is whole, as LAPACK leaves it).  A
 // workgroup decides that once, for all its waves (potrf_stop), by the order of

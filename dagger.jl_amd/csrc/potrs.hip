@@ -30,8 +30,8 @@ namespace dm {
 // Inverse of one n x n (n <= 64) triangular block, one workgroup: the block's
 // upper view V (L^T for 'L') in LDS and V^-T as the solve of the identity's
 // columns, 16 a wave.  V^-T is L^-1, and U^-1 its transpose.  Bound by latency
-// (load, two short chains, store): 7 us, against 60 us with one thread per
-// column substituting against the block in LDS.
+// (load, the chain, store): 8 us, against 60 us with one thread per column
+// substituting against the block in LDS.
 template <typename T, bool UPPER>
 __global__ __launch_bounds__(256) void trtri_leaf_kernel(const TrtriLeaf* __restrict__ leaves,
                                                          const int* __restrict__ abort) {
