@@ -520,7 +520,8 @@ __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base,
     if (set == 0) home[t] = own;
     __syncthreads();
     if (backward) {
-      for (int c = c0 + threadIdx.x; c < std::min(c0 + sets * LS_COLS, c1); c += LS_THREADS)
+      const int64_t end = std::min<int64_t>((int64_t)c0 + sets * LS_COLS, c1);
+      for (int64_t c = (int64_t)c0 + threadIdx.x; c < end; c += LS_THREADS)
         for (int i = 0; i < n; ++i)
           if (q[i] != b0 + i) {
             T* a = tiled_at(base, Mr, mb, W, b0 + i, c);
@@ -551,7 +552,7 @@ __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base,
         const T* a = base + k * (int64_t)mb * W + (from[e] - k * mb);
 #pragma unroll
         for (int c = 0; c < LS_COLS; ++c) {
-          const int col = c0 + set + sets * c;
+          const int64_t col = (int64_t)c0 + set + sets * c;
           if (col < c1) v[e][c] = a[col * l];
         }
       }
@@ -563,7 +564,7 @@ __global__ __launch_bounds__(LS_THREADS) void laswp_kernel(T* __restrict__ base,
         T* a = base + k * (int64_t)mb * W + (to[e] - k * mb);
 #pragma unroll
         for (int c = 0; c < LS_COLS; ++c) {
-          const int col = c0 + set + sets * c;
+          const int64_t col = (int64_t)c0 + set + sets * c;
           if (col < c1) a[col * l] = v[e][c];
         }
       }
